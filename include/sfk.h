@@ -191,7 +191,7 @@ typedef struct sfk_schedule {
                           grid, no scatter; the automatic choice then) */
   int tile_shape;      /* cont_scatter 2: tile of cells in x/y per workgroup,
                           an index < the count sfk_op_tile_shape returns
-                          (0 = default) */
+                          (0 = default: chosen for the mesh by a cost model) */
   int z_cells;         /* cont_scatter 2: cells in z per workgroup (0 =
                           automatic) */
 } sfk_schedule;
@@ -207,23 +207,25 @@ sfk_status sfk_op_get_smoother_schedule(const sfk_op *op, sfk_schedule *s);
 /* Sets the schedule (of the matvec and of the Chebyshev launches);
  * SFK_ERR_INVALID_ARG if cells_per_block exceeds
  * sfk_op_max_cells_per_block; SFK_ERR_UNSUPPORTED if the tile shape needs
- * more LDS than a workgroup has in the operator's precision (the widest Q6
- * tile fits FP32 only; sfk_tune skips such shapes). */
+ * more LDS in the operator's precision than leaves room for two workgroups
+ * per CU (the widest Q6 tile fits FP32 only; sfk_tune skips such shapes). */
 sfk_status sfk_op_set_schedule(sfk_op *op, const sfk_schedule *s);
 /* Largest cells_per_block of the operator (workgroup of at most 256 threads,
  * LDS within the device's per-workgroup limit). */
 sfk_status sfk_op_max_cells_per_block(const sfk_op *op, int *max_cells);
 /* Number of tile shapes of the continuous tensor-product kernel and the
- * shape's cells in x and y (bx, by may be NULL). */
+ * shape's cells in x and y (bx, by may be NULL; shape 0: those of the shape
+ * chosen for this operator's mesh). */
 sfk_status sfk_op_tile_shape(const sfk_op *op, int shape, int *count, int *bx, int *by);
 /* Times sfk_apply for every candidate schedule (`repeats` applies each,
  * after a warm-up apply, on internal scratch vectors; stream-ordered on
  * `stream`), sets the fastest on the handle and returns it in *best with its
  * time per apply in *best_seconds (either may be NULL).  Candidates: every
  * cells_per_block in [1, max] x both block orders x, for the continuous
- * Laplacian, both scatters, and with a constant coefficient every tile shape
- * x z_cells (powers of two up to the cells in z) of the tensor-product
- * kernel; for that kernel the fused Chebyshev launch (three-term form, four
+ * Laplacian, both scatters, and with a constant coefficient the tile shapes
+ * x z_cells (the mesh in 1, 2, 3, ... ranges) of the tensor-product kernel
+ * that its cost model puts within 1.6 of the cheapest; for that kernel the
+ * fused Chebyshev launch (three-term form, four
  * vector streams) is timed over the same tile shapes, z_cells and orders and
  * its fastest kept separately (sfk_op_get_smoother_schedule), and for the
  * per-q-metric SIPG kernel the fused Chebyshev step over cells_per_block and

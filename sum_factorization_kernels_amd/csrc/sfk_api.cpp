@@ -133,21 +133,6 @@ bool uses_tp(const sfk_op *op)
   return has_tp(op) && (op->cont_scatter == 2 || op->cont_scatter == -1);
 }
 
-// default cells in z per workgroup of the tensor-product kernel: about 1024
-// workgroups (4 per CU) unless the mesh has fewer tile columns x cells in z
-int tp_default_zc(const sfk_op *op, int shape)
-{
-  int bx = 0, by = 0;
-  tp_shape(op->d.degree + 1, shape, &bx, &by);
-  if (bx <= 0 || by <= 0) return 0;
-  const long long tiles = (long long)((op->d.n_cells[0] + bx - 1) / bx) * ((op->d.n_cells[1] + by - 1) / by);
-  const int nz = op->d.n_cells[2];
-  long long zc = tiles * nz / 1024;
-  if (zc < 1) zc = 1;
-  if (zc > nz) zc = nz;
-  return (int)zc;
-}
-
 void fill_tp_launch(const sfk_op *op, TpLaunch &L, bool cheby)
 {
   L.n = op->d.degree + 1;
@@ -158,8 +143,8 @@ void fill_tp_launch(const sfk_op *op, TpLaunch &L, bool cheby)
   L.vstride = op->nvec;
   const bool own = cheby && op->cheby_shape >= 0;
   L.shape = own ? op->cheby_shape : op->tp_shape;
-  const int zc = own ? op->cheby_zc : op->tp_zc;
-  L.zc = zc > 0 ? zc : tp_default_zc(op, L.shape);
+  L.zc = own ? op->cheby_zc : op->tp_zc;
+  tp_plan(L.n, L.fp32, L.nc, &L.shape, &L.zc);
   L.order = own ? op->cheby_order : op->sched_order;
 }
 

@@ -24,32 +24,52 @@
 // oracle at 1e-12).  Dirichlet nodes are 0 on input and output.
 //
 // A workgroup owns a tile of TX x TY nodes (BX x BY cells) in x/y and marches
-// through a range of cells in z:
-//   phase Y  (per z layer, the p new node planes): y lines of the input read
-//            from HBM (lanes on consecutive x: coalesced), for the tile's rows
-//            and a halo of p+1 columns (the x sweep needs the cell before the
-//            tile and the tile's last node) -> a, b in LDS;
-//   phase X  x lines of a, b from LDS -> c, d in LDS;
+// through a range of cells in z, one layer (p node planes) at a time:
+//   phase Y  y lines of the input from HBM (lanes on consecutive x:
+//            coalesced), for the tile's rows and a halo of p+1 columns (the x
+//            sweep needs the cell before the tile and the tile's last node)
+//            -> a, b in LDS;
+//   phase X  x lines of a, b from LDS -> registers -> c, d over a, b;
 //   phase Z  one thread per node column: z line of c, d (the layer's first
 //            plane kept in registers from the layer before), z sweep, stores
 //            of the p finished planes (coalesced); the sum for the shared
 //            plane is carried in a register to the next layer.
-// Two barriers per layer.  A z range that starts above z = 0 first rebuilds
-// the carried state from the cell below (one plane, then one layer without
-// stores).  Optionally the Chebyshev update of do_cheby_iter<true>
-// (evaluation_dg_laplacian.h:485-502) is fused into phase Z: the assembled
-// value of a node is final there, and all its streams are coalesced.
+// A z range that starts above z = 0 first rebuilds the carried state from the
+// cell below (one plane, then one layer without stores).  Optionally the
+// Chebyshev update of do_cheby_iter<true> (evaluation_dg_laplacian.h:485-502)
+// is fused into phase Z: the assembled value of a node is final there, and all
+// its streams are coalesced.
+//
+// What bounds it, and why it is built this way (Q6 64^3 FP64 unless stated;
+// 913 MB of vectors, 160-190 us at the rate of a plain copy):
+// * c, d overwrite a, b (four barriers per layer instead of two): half the
+//   LDS, so two or more workgroups share a CU and one computes while another
+//   waits.  With four arrays one workgroup of 13 waves ran per CU.
+// * Every load and store of the layer loop is an unconditional buffer access;
+//   lanes without work carry an offset beyond the buffer, which reads 0 and
+//   stores nothing.  Loads and stores share one completion counter, and from
+//   divergent branches the compiler could only wait for all of them: every
+//   layer then waited for its own stores to reach memory.  Now the wait for
+//   the y lines counts past the stores issued after them.  It also makes
+//   Dirichlet rows, tile edges and the y boundary one code path.
+// * Idle threads repeat the last work item instead of being masked, and row
+//   and plane strides are re-derived at each use: 536 instead of about 900
+//   instructions per layer and thread, 20 instead of 60 of them scalar spills.
+// * The row pitch is 1 modulo the banks and items run over the rows of one
+//   cell, then its x neighbours, so the lanes of an LDS pass of phase X fall
+//   on consecutive banks (conflicts 0.21 -> 0.05 of the LDS cycles).
+// * The fused forms keep the input values of phase Y in a third LDS array for
+//   phase Z instead of reading them again: with 10 MB of streams per layer in
+//   flight on an XCD the second read missed its 4 MB L2 (29 % more HBM reads).
+// Measured before -> after: matvec FP64 282 -> 264 us (3.5 TB/s; 3.9 TB/s with
+// the halo), FP32 172 -> 127 us; three-term Chebyshev step FP64 675 -> 457 us
+// (4.0 TB/s), FP32 358 -> 247 us; Q3 101x107x100 FP32 96 -> 58 us.
+#include <cmath>
 #include <type_traits>
 
 #include "sfk_device.h"
 #include "sfk_kernels.h"
 
-#ifndef SFK_TP_SCHED
-#define SFK_TP_SCHED 1
-#endif
-#ifndef SFK_TP_WAVES
-#define SFK_TP_WAVES 1
-#endif
 
 namespace sfk {
 
@@ -74,72 +94,62 @@ __device__ __forceinline__ const SFK_CONST_AS TpTab<N, T> &tptab(const void *p)
   return *(const SFK_CONST_AS TpTab<N, T> *)opaque_ptr(p);
 }
 
-constexpr int odd_up(int v) { return v | 1; }
 constexpr int round64(int v) { return (v + 63) / 64 * 64; }
-constexpr int imax(int a, int b) { return a > b ? a : b; }
 
 template <int N, typename T, int BX, int BY>
 struct TpCfg {
   static constexpr int p = N - 1;
   static constexpr int TX = BX * p, TY = BY * p;
   static constexpr int HX = TX + p + 1;   // columns of phase Y (halo of p before, 1 after)
-  static constexpr int RPA = odd_up(HX);  // row pitches: odd, so that 16 lanes on
-  static constexpr int RPC = odd_up(TX);  // consecutive rows hit distinct banks
-  static constexpr int NYI = p * BY * HX; // work items of phase Y (p planes)
+  static constexpr int NYI = p * BY * HX; // work items of phase Y (p planes): the most of all phases
   static constexpr int NXI = p * TY * BX; // phase X
   static constexpr int NZI = TX * TY;     // phase Z (node columns)
-  static constexpr int THREADS_RAW = round64(imax(NYI, imax(NXI, NZI)));
-  static constexpr int THREADS = THREADS_RAW > 1024 ? 1024 : THREADS_RAW;
-  static constexpr int LA = p * TY * RPA; // one of a, b
-  static constexpr int LC = p * TY * RPC; // one of c, d
-  static constexpr int LDS_VALUES = 2 * LA + 2 * LC;
+  static constexpr int THREADS = round64(NYI);
+  static_assert(THREADS <= 1024, "one phase-Y item per thread");
+  // LDS banks in units of T (32 banks of 4 bytes): a row pitch of 1 modulo
+  // the banks puts the p rows of a cell, and with them the rows of its x
+  // neighbours (p further), on consecutive banks; the plane pitch continues
+  // that sequence from one plane to the next when BY = 1
+  static constexpr int LW = 128 / (int)sizeof(T);
+  static constexpr int RPA = (HX - 2) / LW * LW + LW + 1;
+  static constexpr int PSA = TY * RPA + ((p * BX - TY * RPA) % LW + LW) % LW;
+  static constexpr int LA = p * PSA;      // one of a, b (c, d)
+  // input values at the nodes (fused forms), one spare column per row
+  static constexpr int RPU = (TX + 1) | 1;
+  static constexpr int PSU = TY * RPU;
+  static constexpr int LU = p * PSU;
+  static constexpr int lds_values(bool fused) { return 2 * LA + (fused ? LU : 0); }
 };
 
-// waves per SIMD that the LDS of one tile shape allows (160 KiB per CU in
-// 1280-byte granules, at most 32 waves per CU): the kernel asks the
-// compiler for registers that let this many waves be resident, since an
-// allocation above 512/W VGPRs would drop a whole workgroup per CU
-template <int N, typename T, int BX, int BY>
+// The next layer's y lines are loaded before phase X of the current one where
+// the registers allow it; without that prefetch the matvec needs 28 registers
+// less (FP64), which from degree 7 on decides whether two workgroups fit a CU.
+// The fused forms hold their streams instead (Q6 64^3 FP64 Chebyshev step: 457
+// us without, 502 us with it).
+template <int N, typename T, int CHEBY>
+constexpr bool tp_prefetch()
+{
+  return CHEBY == 0 && (sizeof(T) == 4 || N <= 7);
+}
+// The fused forms' streams (rhs, previous iterate, ...) are loaded before
+// phase X (hidden behind it) or, where that would spill, at the start of
+// phase Z (FP64 from degree 7; the six-stream form in FP64).
+template <int N, typename T, int CHEBY>
+constexpr bool tp_streams_early()
+{
+  return sizeof(T) == 4 || (N <= 7 && CHEBY != 1);
+}
+// Waves per SIMD asked of the compiler.  FP64 up to degree 6: 4 (128
+// registers), i.e. two workgroups of 8 waves or four of 4 waves per CU; asking
+// for 5 or 6 spilled (Q6 matvec 264 -> 312 us).  Degrees 7 and 8 hold 4 only
+// in the matvec's 8-wave tiles (Chebyshev step of Q7 46x44x45: 301 us at 3,
+// 310 us at 4 with spills).  FP32 needs at most 95 registers by itself.
+template <int N, typename T, int CHEBY, int THREADS>
 constexpr int tp_waves()
 {
-  using C = TpCfg<N, T, BX, BY>;
-  constexpr int bytes = C::LDS_VALUES * (int)sizeof(T);
-  constexpr int alloc = (bytes + 1279) / 1280 * 1280;
-  constexpr int wpg = C::THREADS / 64;
-  int wgs = 163840 / alloc;
-  if (wgs * wpg > 32) wgs = 32 / wpg;
-  const int w = (wgs * wpg + 3) / 4;
-  return w < 1 ? 1 : (w > 8 ? 8 : w);
-}
-
-// waves per SIMD the kernel is compiled for: the matvec (CHEBY 0) asks for
-// what the LDS allows; the Chebyshev forms hold more streams in registers
-// (prefetched rhs, diagonal, tm / previous iterate) and would spill at that
-// occupancy, so unless SFK_TP_CHEBY_WAVES is set they ask for one wave only
-// (the register count then sets the occupancy)
-#ifndef SFK_TP_CHEBY_WAVES
-#define SFK_TP_CHEBY_WAVES 0
-#endif
-template <int N, typename T, int BX, int BY, int CHEBY>
-constexpr int tp_waves_of()
-{
-  return CHEBY == 0 || CHEBY == 5 ? tp_waves<N, T, BX, BY>()
-                    : (SFK_TP_CHEBY_WAVES > 0 ? SFK_TP_CHEBY_WAVES
-                                              : (SFK_TP_CHEBY_WAVES < 0 ? tp_waves<N, T, BX, BY>() : 1));
-}
-
-// element at a 32-bit byte offset (per lane) from a uniform base pointer:
-// the load or store takes the scalar base and the vector offset directly
-// (no per-lane 64-bit address arithmetic)
-template <typename T>
-__device__ __forceinline__ const T &at(const T *base, unsigned off)
-{
-  return *reinterpret_cast<const T *>(reinterpret_cast<const char *>(base) + off);
-}
-template <typename T>
-__device__ __forceinline__ T &at(T *base, unsigned off)
-{
-  return *reinterpret_cast<T *>(reinterpret_cast<char *>(base) + off);
+  if (sizeof(T) == 4) return 1;
+  if (N <= 7) return 4;
+  return (CHEBY == 0 || CHEBY == 5) && THREADS > 256 ? 4 : 3;
 }
 
 template <typename T>
@@ -187,9 +197,44 @@ __device__ __forceinline__ void line_one(const void *tab, const T (&in)[2 * N - 
   o[0] = r[0] + v;
 #pragma unroll
   for (int i = 1; i < p; ++i) o[i] = r[i];
-#if SFK_TP_SCHED
   __builtin_amdgcn_sched_barrier(0);
-#endif
+}
+
+
+// Buffer accesses: a uniform base, a 32-bit offset per lane and a uniform
+// offset.  A lane offset of kOob lies beyond every buffer described here
+// (fewer than 2^31 bytes): such lanes read 0 and store nothing.
+constexpr unsigned kOob = 0x80000000u, kAll = 0x7fffffffu;
+typedef unsigned sfk_u2 __attribute__((ext_vector_type(2)));
+using Rsrc = __amdgpu_buffer_rsrc_t;
+template <typename T>
+__device__ __forceinline__ Rsrc make_rsrc(const T *p, unsigned bytes = kAll)
+{
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<T *>(p), 0, (int)bytes, 0x00027000);
+}
+template <typename T>
+__device__ __forceinline__ T buf_load(Rsrc r, unsigned voff, unsigned soff)
+{
+  if constexpr (sizeof(T) == 8)
+    return __builtin_bit_cast(T, __builtin_amdgcn_raw_buffer_load_b64(r, (int)voff, (int)soff, 0));
+  else
+    return __builtin_bit_cast(T, __builtin_amdgcn_raw_buffer_load_b32(r, (int)voff, (int)soff, 0));
+}
+template <int NT, typename T>
+__device__ __forceinline__ void buf_store(Rsrc r, unsigned voff, unsigned soff, T v)
+{
+  constexpr int aux = NT ? 2 : 0; // non-temporal
+  if constexpr (sizeof(T) == 8)
+    __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(sfk_u2, v), r, (int)voff, (int)soff, aux);
+  else
+    __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, v), r, (int)voff, (int)soff, aux);
+}
+// the same value, unknown to the compiler: keeps multiples of a stride from
+// being hoisted out of the layer loop into scalar registers it then spills
+__device__ __forceinline__ unsigned opaque_s(unsigned v)
+{
+  __asm__ volatile("" : "+s"(v));
+  return v;
 }
 
 // CHEBY: 0 matvec; 1 the Chebyshev step of do_cheby_iter<true>
@@ -199,27 +244,22 @@ __device__ __forceinline__ void line_one(const void *tab, const T (&in)[2 * N - 
 // dst = u - c_tm (prev - u) - c_np D^{-1} (A u - rhs), four streams instead
 // of six, and dst may be prev (each node is read, then written, by one
 // thread); 3 and 4 the three-term step whose input (3) or previous iterate
-// (4) is the first iterate s_rhs D^{-1} rhs, formed from rhs in the kernel
+// (4) is the first iterate s_rhs D^{-1} rhs, formed from rhs in the kernel;
+// 5 the matvec with the workgroup's partial sum of src . dst
 template <int N, typename T, int BX, int BY, int CHEBY>
 __global__ void __launch_bounds__((TpCfg<N, T, BX, BY>::THREADS))
-#if SFK_TP_WAVES
-__attribute__((amdgpu_waves_per_eu(tp_waves_of<N, T, BX, BY, CHEBY>(), 8)))
-#endif
+__attribute__((amdgpu_waves_per_eu(tp_waves<N, T, CHEBY, TpCfg<N, T, BX, BY>::THREADS>(), 8)))
 cont_tp_kernel(const TpArgs<T> a)
 {
   using C = TpCfg<N, T, BX, BY>;
-  constexpr int p = N - 1, TX = C::TX, TY = C::TY, HX = C::HX, RPA = C::RPA, RPC = C::RPC;
+  constexpr int p = N - 1, TX = C::TX, TY = C::TY, HX = C::HX, RPA = C::RPA, PSA = C::PSA, ES = (int)sizeof(T);
   // three-term form (2, 3, 4); 3: the input, 4: the previous iterate is
   // s_rhs D^{-1} rhs (the first iterate, never stored)
   constexpr bool TT = CHEBY >= 2 && CHEBY <= 4, RSRC = CHEBY == 3, RPREV = CHEBY == 4, DOT = CHEBY == 5;
-  // CHEBY 5: a layer's outputs held in registers and stored, with the
-  // prefetch of the next layer's input at the node, after the next layer's
-  // wait for its y lines (see flush below)
-  constexpr bool DELAY = DOT;
-  T *sA = dyn_lds<T>();
-  T *sB = sA + C::LA;
-  T *sC = sB + C::LA;
-  T *sD = sC + C::LC;
+  constexpr bool FUSED = CHEBY != 0; // phase Z needs the input at its nodes
+  constexpr bool PF = tp_prefetch<N, T, CHEBY>(), EARLY = tp_streams_early<N, T, CHEBY>();
+  T *sA = dyn_lds<T>(); // a, then c; b, then d follow at C::LA
+  T *sU = sA + 2 * C::LA;
 
   const unsigned L = logical_block(blockIdx.x, gridDim.x, a.order);
   const int tx = (int)(L % (unsigned)a.ntx);
@@ -231,183 +271,165 @@ cont_tp_kernel(const TpArgs<T> a)
   const int ez_begin = chunk * a.zc;
   const int ez_end = ez_begin + a.zc < a.nz ? ez_begin + a.zc : a.nz;
   const int gx = a.gx, gy = a.gy, gz = a.gz;
-  const long long plane = (long long)gx * gy;
-  const long long rr = blockIdx.y;
-  const T *src = a.src + rr * a.vstride;
-  T *dst = a.dst + rr * a.vstride;
+  // (the host checks that the p+1 planes of a layer hold less than 2^31 bytes)
+  const int plane = gx * gy;
+  const unsigned plane_bytes = (unsigned)plane * ES, row_bytes = (unsigned)gx * ES;
+  const long long layer_size = (long long)p * plane;
+  const T *src = a.src + (long long)blockIdx.y * a.vstride;
+  T *dst = a.dst + (long long)blockIdx.y * a.vstride;
+  const int it = threadIdx.x;
 
-  // phase Y, split in two so that the loads of the next layer are in flight
-  // during phases X and Z of the current one: load_y fetches this thread's
-  // y line (planes Z = ez p + k0 + s, s < NK, one work item per thread:
-  // NK BY HX <= THREADS) into registers, store_y contracts it into slot s.
-  static_assert(p * BY * HX <= C::THREADS, "one phase-Y item per thread");
-  // the y lines of the tile's cells ey0 .. ey0+BY-1 span the rows
-  // (ey0-1) p .. (ey0+BY) p: all interior node rows unless the tile is
-  // within one cell of the y boundary
-  const bool ybnd = !(ey0 >= 2 && ey0 + BY < a.ny);
-  T u[2 * N - 1];
-  bool yact = false;
-  auto load_y_to = [&](T(&uu)[2 * N - 1], bool &act, int ez, int k0, auto nkc) {
-    constexpr int NK = decltype(nkc)::value;
-    const int it = threadIdx.x;
-    const int xh = it % HX, rest = it / HX, eyl = rest % BY, s = rest / BY;
-    const int ey = ey0 + eyl;
-    // rows beyond the mesh are never read
-    act = it < NK * BY * HX && ey < a.ny;
-    const int X = x0 - p + xh, Z = ez * p + k0 + s;
-    if (act && X > 0 && X < gx - 1 && Z > 0 && Z < gz - 1) {
-      if (!ybnd) {
-        // interior tile row range: every row of the line is an interior
-        // node row; row j of all lanes is one uniform base + the lane's
-        // 32-bit offset within the layer (the host checks that the layer's
-        // planes span less than 2 GiB)
-        const T *lb = src + (long long)(ez * p) * plane;
-        const unsigned off = (unsigned)(((k0 + s) * (int)plane + (ey * p - p) * gx + X) * (int)sizeof(T));
-#pragma unroll
-        for (int j = 0; j < 2 * N - 1; ++j) uu[j] = at(lb + j * gx, off);
-      } else {
-        const T *col = src + (long long)Z * plane + X;
-#pragma unroll
-        for (int j = 0; j < 2 * N - 1; ++j) {
-          const int Y = ey * p - p + j;
-          uu[j] = (Y > 0 && Y < gy - 1) ? col[(long long)Y * gx] : T(0);
-        }
-      }
-    } else {
-#pragma unroll
-      for (int j = 0; j < 2 * N - 1; ++j) uu[j] = T(0);
+  // ---- phase Y: this thread's y line is column X, plane ez p + 1 + ys, rows
+  // (ey-1) p .. (ey+1) p.  Offsets are relative to row -p of the layer's
+  // first plane, so they are never negative.  Row 0 of the line is a node
+  // with a value if ey >= 2, rows 1..p if ey >= 1, the last row if the cell
+  // is not the last in y; the grid's last plane (ys = p-1 of the last layer)
+  // has none.
+  unsigned o_first, o_low, o_mid, o_last, top_plane;
+  int ys;
+  T *ya, *yu = nullptr;
+  T dxz = T(0), exz = T(0), dxz0 = T(0), exz0 = T(0);
+  {
+    const int i = it < C::NYI ? it : C::NYI - 1; // idle threads repeat the last item
+    const int xh = i % HX, rest = i / HX, eyl = rest % BY;
+    ys = rest / BY;
+    const int ey = ey0 + eyl, X = x0 - p + xh;
+    const bool ok = ey < a.ny && X > 0 && X < gx - 1;
+    const unsigned o = (unsigned)(((1 + ys) * plane + ey * p * gx + X) * ES);
+    o_first = ok && ey >= 2 ? o : kOob;
+    o_low = ok && ey >= 1 ? o : kOob;
+    o_mid = ok ? o : kOob;
+    o_last = ok && ey + 1 < a.ny ? o : kOob;
+    top_plane = ys == p - 1 ? kOob : 0u;
+    ya = sA + ys * PSA + eyl * p * RPA + xh;
+    if constexpr (FUSED) {
+      // halo columns share the spare slot after the tile's last column
+      const int xu = xh >= p && xh < p + TX ? xh - p : TX;
+      yu = sU + ys * C::PSU + eyl * p * C::RPU + xu;
     }
     if constexpr (RSRC) {
-      {
-        // the line holds rhs: scale node j by s_rhs / D, D = a_xz dm[j % p] +
-        // b_xz dk_y[j % p] with the x/z factors of this line (row j of a
-        // line is node j % p of its cell; index 0 is the shared vertex);
-        // the Dirichlet nodes were loaded as 0
-        const auto &tb = tptab<N, T>(a.tab);
-        const int ix = xh % p, iz = (k0 + s) % p;
-        const T axz = tb.dk[0][ix] * tb.dm[iz] + tb.dm[ix] * tb.dk[2][iz];
-        const T bxz = tb.dm[ix] * tb.dm[iz];
-#pragma unroll
-        for (int j = 0; j < 2 * N - 1; ++j) uu[j] *= a.s_rhs / (axz * tb.dm[j % p] + bxz * tb.dk[1][j % p]);
-      }
+      // x/z factors of the line's diagonal: D = dxz dm[j % p] + exz dk_y[j % p]
+      // at its row j (row j of a line is node j % p of its cell; index 0 is
+      // the shared vertex)
+      const auto &tb = tptab<N, T>(a.tab);
+      const int jx = xh % p, jz = (ys + 1) % p;
+      dxz = tb.dk[0][jx] * tb.dm[jz] + tb.dm[jx] * tb.dk[2][jz];
+      exz = tb.dm[jx] * tb.dm[jz];
+      dxz0 = tb.dk[0][jx] * tb.dm[0] + tb.dm[jx] * tb.dk[2][0]; // in a layer's plane 0
+      exz0 = tb.dm[jx] * tb.dm[0];
     }
+  }
+  T u[2 * N - 1];
+  auto load_lines = [&](const T *layer, unsigned bytes, unsigned v0, unsigned v1, unsigned vm, unsigned vl) {
+    const Rsrc r = make_rsrc(layer - (long long)p * gx, bytes);
+    const unsigned rb = opaque_s(row_bytes);
+#pragma unroll
+    for (int j = 0; j < 2 * N - 1; ++j)
+      u[j] = buf_load<T>(r, j == 0 ? v0 : (j <= p ? v1 : (j < 2 * p ? vm : vl)), (unsigned)j * rb);
   };
-  auto load_y = [&](int ez, int k0, auto nkc) { load_y_to(u, yact, ez, k0, nkc); };
-  auto store_y_from = [&](const T(&uu)[2 * N - 1], bool act) {
-    if (!act) return;
-    const int it = threadIdx.x;
-    const int xh = it % HX, rest = it / HX, eyl = rest % BY, s = rest / BY;
+  // (live false: nothing is read, the loads only keep the loop uniform)
+  auto load_y = [&](int ez, bool live) {
+    const unsigned m = ez == a.nz - 1 ? top_plane : 0u;
+    load_lines(src + (long long)ez * layer_size, live ? kAll : 0u, o_first | m, o_low | m, o_mid | m, o_last | m);
+  };
+  auto phase_y = [&](bool plane0) {
+    T un[FUSED ? p : 1]; // the input (RSRC: the right-hand side) at the line's own nodes
+    if constexpr (FUSED)
+#pragma unroll
+      for (int i = 0; i < p; ++i) un[i] = u[p + i];
+    if constexpr (RSRC) {
+      const auto &tb = tptab<N, T>(a.tab);
+#pragma unroll
+      for (int j = 0; j < 2 * N - 1; ++j)
+        u[j] *= a.s_rhs / ((plane0 ? dxz0 : dxz) * tb.dm[j % p] + (plane0 ? exz0 : exz) * tb.dk[1][j % p]);
+    }
     T va[N - 1], vb[N - 1];
-    line_one<N, T, 0>(a.tab, uu, va); // a = M_y u
-    line_one<N, T, 2>(a.tab, uu, vb); // b = c_y K_y u
-    T *ra = sA + (s * TY + eyl * p) * RPA + xh;
-    T *rb = sB + (s * TY + eyl * p) * RPA + xh;
+    line_one<N, T, 0>(a.tab, u, va); // a = M_y u
+    line_one<N, T, 2>(a.tab, u, vb); // b = c_y K_y u
+    __syncthreads();                 // phase Z of the layer before has read c, d
 #pragma unroll
     for (int i = 0; i < p; ++i) {
-      ra[i * RPA] = va[i];
-      rb[i * RPA] = vb[i];
+      ya[i * RPA] = va[i];
+      ya[C::LA + i * RPA] = vb[i];
     }
-  };
-  auto store_y = [&]() { store_y_from(u, yact); };
-
-  // phase X: rows of slots s < NK
-  auto phase_x = [&](auto nkc) {
-    constexpr int NK = decltype(nkc)::value;
-    for (int it = threadIdx.x; it < NK * TY * BX; it += C::THREADS) {
-      const int yt = it % TY, rest = it / TY, s = rest % NK, exl = rest / NK;
-      if (ex0 + exl >= a.nx || y0 + yt >= gy - 1) continue; // no owned output
-      const T *ra = sA + (s * TY + yt) * RPA + exl * p;
-      const T *rb = sB + (s * TY + yt) * RPA + exl * p;
-      T *rc = sC + (s * TY + yt) * RPC + exl * p;
-      T *rd = sD + (s * TY + yt) * RPC + exl * p;
-      // c = M a;  d = M b + c_x K a, one input line at a time (registers)
-      T ua[2 * N - 1], cm[N - 1], ck[N - 1];
+    if constexpr (FUSED)
 #pragma unroll
-      for (int j = 0; j < 2 * N - 1; ++j) ua[j] = ra[j];
-      line_one<N, T, 0>(a.tab, ua, cm);
-#pragma unroll
-      for (int i = 0; i < p; ++i) rc[i] = cm[i];
-      line_one<N, T, 1>(a.tab, ua, ck);
-      T ub[2 * N - 1], dm[N - 1];
-#pragma unroll
-      for (int j = 0; j < 2 * N - 1; ++j) ub[j] = rb[j];
-      line_one<N, T, 0>(a.tab, ub, dm);
-#pragma unroll
-      for (int i = 0; i < p; ++i) rd[i] = dm[i] + ck[i];
-    }
+      for (int i = 0; i < p; ++i) yu[i * C::RPU] = un[i];
+    __syncthreads();
   };
 
-  // phase Z state of this thread's node column
-  const int zt = threadIdx.x;
+  // ---- phase X: rows of one cell run fastest over the threads, then its x
+  // neighbours, the rows of the next cells in y, the planes
+  T *xa;
+  {
+    const int i = it < C::NXI ? it : C::NXI - 1;
+    const int yi = i % p, r1 = i / p, exl = r1 % BX, r2 = r1 / BX, eyl = r2 % BY, xs = r2 / BY;
+    xa = sA + xs * PSA + (eyl * p + yi) * RPA + exl * p;
+  }
+  auto phase_x = [&]() {
+    // c = M a;  d = M b + c_x K a, one input line at a time (registers)
+    T cm[N - 1], dm[N - 1], ck[N - 1];
+    T ua[2 * N - 1];
+#pragma unroll
+    for (int j = 0; j < 2 * N - 1; ++j) ua[j] = xa[j];
+    line_one<N, T, 0>(a.tab, ua, cm);
+    line_one<N, T, 1>(a.tab, ua, ck);
+    T ub[2 * N - 1];
+#pragma unroll
+    for (int j = 0; j < 2 * N - 1; ++j) ub[j] = xa[C::LA + j];
+    line_one<N, T, 0>(a.tab, ub, dm);
+#pragma unroll
+    for (int i = 0; i < p; ++i) dm[i] += ck[i];
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < p; ++i) {
+      xa[i] = cm[i];
+      xa[C::LA + i] = dm[i];
+    }
+    __syncthreads();
+  };
+
+  // ---- phase Z: this thread's node column
+  const int zt = it < C::NZI ? it : C::NZI - 1;
   const int Xt = zt % TX, Yt = zt / TX;
   const int X = x0 + Xt, Y = y0 + Yt;
-  // 0: compute, 1: Dirichlet column of the grid's last x or y node (zeros),
-  // 2: outside the grid or no column
-  const int zone = zt >= C::NZI || X >= gx || Y >= gy ? 2 : (X == gx - 1 || Y == gy - 1 ? 1 : 0);
+  const bool has = it < C::NZI && X < gx && Y < gy; // the thread stores this column
+  const bool inner = has && X > 0 && X < gx - 1 && Y > 0 && Y < gy - 1;
   // the tile ends exactly at the last (Dirichlet) node: its zeros are
   // written by the threads of the nodes before it
-  const bool xtra_x = zone != 2 && Xt == TX - 1 && X + 1 == gx - 1;
-  const bool xtra_y = zone != 2 && Yt == TY - 1 && Y + 1 == gy - 1;
-  // byte offset of this thread's node column inside a plane (planes hold
-  // less than 2^31 bytes: checked on the host)
-  const unsigned coff = zone == 2 ? 0u : (unsigned)((Y * gx + X) * (int)sizeof(T));
-  T cp = T(0), dp = T(0), yp = T(0);
-
-  // output of node (column offset off) in plane Z (Dirichlet nodes only for
-  // the three-term form: the inverse diagonal is 0 there)
-  auto put = [&](int Z, unsigned off, T v) {
-    const long long zo = (long long)Z * plane; // uniform
-    if constexpr (TT) {
-      // (a first iterate formed from rhs is 0 on these nodes)
-      const long long g = zo + off / (unsigned)sizeof(T);
-      const T us = RSRC ? T(0) : src[g];
-      const T pv = !RSRC && !RPREV && a.prev ? a.prev[g] : T(0); // null: the zero vector
-      dst[g] = us - a.c_tm * (pv - us);
-    } else if constexpr (CHEBY == 1) {
-      // r = A u - rhs; tm = c_tm tm + c_np diag r; dst = u - tm (five
-      // streams: lane addresses, not five uniform bases per plane, which
-      // would not fit the scalar registers)
-      const long long g = zo + off / (unsigned)sizeof(T);
-      const T res = v - a.rhs[g];
-      const T t = (a.c_tm != T(0) ? a.c_tm * a.tm[g] : T(0)) + a.c_np * a.diag[g] * res;
-      a.tm[g] = t;
-      dst[g] = src[g] - t;
-    } else {
-      __builtin_nontemporal_store(v, &at(dst + zo, off));
-    }
-  };
-  // fused Chebyshev: rhs, diag, tmp (or the previous iterate) and the input
-  // at this thread's node column, plane k of a layer in q_*[k].  A rolling
-  // prefetch one layer ahead: the first layer's planes are loaded before the
-  // layer loop, and as soon as phase Z has written plane k of layer ez, the
-  // registers of plane k take the loads of layer ez + 1, in flight during the
-  // rest of phase Z and the next layer's phases Y and X (loaded at the start
-  // of their own layer, their latency was only partly hidden)
-  constexpr int NCH = CHEBY ? p : 1; // CHEBY 5: q_s only
-  T q_r[NCH], q_d[CHEBY == 1 ? NCH : 1], q_t[NCH], q_s[NCH];
-  double dot_acc = 0.; // CHEBY 5
-  auto load_plane = [&](int ez, int k) {
-    if constexpr (CHEBY == 1) {
-      const long long g = (long long)(ez * p + k) * plane + coff / (unsigned)sizeof(T);
-      q_r[k] = a.rhs[g];
-      q_d[k] = a.diag[g];
-      q_t[k] = a.c_tm != T(0) ? a.tm[g] : T(0);
-      q_s[k] = src[g];
-    } else if constexpr (DOT) {
-      q_s[k] = at(src + (long long)(ez * p + k) * plane, coff);
-    } else if constexpr (TT) {
-      // uniform plane bases + this lane's 32-bit column offset
-      const long long zo = (long long)(ez * p + k) * plane;
-      q_r[k] = at(a.rhs + zo, coff);
-      if constexpr (!RSRC && !RPREV) q_t[k] = a.prev ? at(a.prev + zo, coff) : T(0);
-      if constexpr (!RSRC) q_s[k] = at(src + zo, coff);
-    }
-  };
-  if constexpr (CHEBY != 0) {
-    if (zone != 2 && ez_begin < ez_end)
+  const bool xtra_x = has && Xt == TX - 1 && X + 1 == gx - 1;
+  const bool xtra_y = has && Yt == TY - 1 && Y + 1 == gy - 1;
+  const bool xtra = xtra_x || xtra_y;
+  const unsigned coff = has ? (unsigned)((Y * gx + X) * ES) : kOob;
+  const T *za = sA + Yt * RPA + Xt, *zu = sU + Yt * C::RPU + Xt;
+  T cp = T(0), dp = T(0), yp = T(0), up = T(0); // carried: c, d, the shared plane's sum, the input
+  double dot_acc = 0.;
+  // streams of the fused forms at this column, plane k of the layer
+  constexpr int NCH = CHEBY == 1 || TT ? p : 1;
+  T q_r[NCH], q_d[CHEBY == 1 ? NCH : 1], q_t[NCH];
+  auto load_streams = [&](int ez) {
+    const long long zb = (long long)ez * layer_size;
+    const unsigned pb = opaque_s(plane_bytes);
+    if constexpr (CHEBY == 1 || (TT && !RSRC)) {
+      const Rsrc r = make_rsrc(a.rhs + zb);
 #pragma unroll
-      for (int k = 0; k < p; ++k) load_plane(ez_begin, k);
-  }
+      for (int k = 0; k < p; ++k) q_r[k] = buf_load<T>(r, coff, k * pb);
+    }
+    if constexpr (CHEBY == 1) {
+      // c_tm == 0: tm is not read
+      const Rsrc rd = make_rsrc(a.diag + zb), rt = make_rsrc(a.tm + zb, a.c_tm != T(0) ? kAll : 0u);
+#pragma unroll
+      for (int k = 0; k < p; ++k) q_d[k] = buf_load<T>(rd, coff, k * pb);
+#pragma unroll
+      for (int k = 0; k < p; ++k) q_t[k] = buf_load<T>(rt, coff, k * pb);
+    }
+    if constexpr (TT && !RSRC && !RPREV) {
+      // no previous iterate: the zero vector
+      const Rsrc r = make_rsrc(a.prev ? a.prev + zb : src, a.prev ? kAll : 0u);
+#pragma unroll
+      for (int k = 0; k < p; ++k) q_t[k] = buf_load<T>(r, coff, k * pb);
+    }
+  };
   // three-term form: the inverse diagonal of this node column in plane k of a
   // cell, D = d1 dm[k] + d2 dk[2][k] with the x/y factors d1, d2 of the
   // column (0 off the interior columns); the same in every layer, so formed
@@ -415,156 +437,136 @@ cont_tp_kernel(const TpArgs<T> a)
   T dinvk[TT ? p : 1];
   if constexpr (TT) {
     const auto &tb = tptab<N, T>(a.tab);
-    const bool inner = zone == 0 && X > 0 && Y > 0;
     const int ix = inner ? X % p : 0, iy = inner ? Y % p : 0;
     const T d1 = tb.dk[0][ix] * tb.dm[iy] + tb.dm[ix] * tb.dk[1][iy];
     const T d2 = tb.dm[ix] * tb.dm[iy];
 #pragma unroll
     for (int k = 0; k < p; ++k) dinvk[k] = inner ? T(1) / (d1 * tb.dm[k] + d2 * tb.dk[2][k]) : T(0);
   }
-  // output v of this thread's node in plane ez p + k (prefetched streams)
-  auto put_own = [&](int ez, int k, T v) {
+  // Dirichlet node at element g outside the layer loop's columns and planes
+  // (A u = 0 there; three-term form: the inverse diagonal is 0 too, and a
+  // first iterate formed from rhs is 0)
+  auto put_zero = [&](int Z, unsigned off) {
+    const long long g = (long long)Z * plane + off / ES;
     if constexpr (TT) {
-      const long long zo = (long long)(ez * p + k) * plane; // uniform
-      const T dinv = ez * p + k > 0 ? dinvk[k] : T(0);
-      const T z1 = a.s_rhs * dinv * q_r[k]; // the first iterate, when formed here
-      const T us = RSRC ? z1 : q_s[k];
-      const T pv = RPREV ? z1 : (RSRC ? T(0) : q_t[k]);
-      const T t = a.c_tm * (pv - us) + a.c_np * dinv * (v - q_r[k]);
-      at(dst + zo, coff) = us - t;
-      if (ez + 1 < ez_end) load_plane(ez + 1, k);
+      const T us = RSRC ? T(0) : src[g];
+      const T pv = !RSRC && !RPREV && a.prev ? a.prev[g] : T(0);
+      dst[g] = us - a.c_tm * (pv - us);
     } else if constexpr (CHEBY == 1) {
-      const long long g = (long long)(ez * p + k) * plane + coff / (unsigned)sizeof(T);
-      const T res = v - q_r[k];
-      const T t = (a.c_tm != T(0) ? a.c_tm * q_t[k] : T(0)) + a.c_np * q_d[k] * res;
+      const T t = (a.c_tm != T(0) ? a.c_tm * a.tm[g] : T(0)) + a.c_np * a.diag[g] * (T(0) - a.rhs[g]);
       a.tm[g] = t;
-      dst[g] = q_s[k] - t;
-      if (ez + 1 < ez_end) load_plane(ez + 1, k);
+      dst[g] = src[g] - t;
     } else {
-      put(ez * p + k, coff, v);
-      if constexpr (DOT) {
-        dot_acc += double(q_s[k]) * double(v);
-        if (ez + 1 < ez_end) load_plane(ez + 1, k);
-      }
+      dst[g] = T(0);
     }
   };
-  // zero (Dirichlet) outputs of plane Z for this thread: its own node when
-  // zone 1 (plane ez p + k), the extra last-node columns
-  auto put_zeros = [&](int Z, int ez, int k) {
-    if (zone == 1) {
-      if (k >= 0) put_own(ez, k, T(0));
-      else put(Z, coff, T(0));
-    }
-    if (xtra_x) put(Z, coff + (unsigned)sizeof(T), T(0));
-    if (xtra_y) put(Z, coff + (unsigned)(gx * (int)sizeof(T)), T(0));
-    if (xtra_x && xtra_y) put(Z, coff + (unsigned)((gx + 1) * (int)sizeof(T)), T(0));
+  auto put_xtra = [&](int Z) {
+    if (xtra_x) put_zero(Z, coff + ES);
+    if (xtra_y) put_zero(Z, coff + row_bytes);
+    if (xtra_x && xtra_y) put_zero(Z, coff + row_bytes + ES);
   };
-
-  // delayed outputs: po[k] of plane ez p + k of the last layer phase Z stored
-  T po[DELAY ? N - 1 : 1];
   auto phase_z = [&](int ez, bool store) {
-    if (zone == 0) {
-      T c[N], d[N], o[N];
-      c[0] = cp;
-      d[0] = dp;
+    if (!EARLY && store) load_streams(ez);
+    T c[N], d[N], o[N], us[FUSED ? N : 1];
+    c[0] = cp;
+    d[0] = dp;
 #pragma unroll
-      for (int k = 1; k < N; ++k) {
-        c[k] = sC[((k - 1) * TY + Yt) * RPC + Xt];
-        d[k] = sD[((k - 1) * TY + Yt) * RPC + Xt];
+    for (int k = 1; k < N; ++k) {
+      c[k] = za[(k - 1) * PSA];
+      d[k] = za[C::LA + (k - 1) * PSA];
+    }
+    if constexpr (FUSED) {
+      us[0] = up;
+#pragma unroll
+      for (int k = 1; k < N; ++k) us[k] = zu[(k - 1) * C::PSU];
+      up = us[p];
+    }
+    T om[N], ok[N];
+    eo_apply<N, 1>(tptab<N, T>(a.tab).M, d, om);
+    __builtin_amdgcn_sched_barrier(0);
+    eo_apply<N, 1>(tptab<N, T>(a.tab).K[2], c, ok);
+#pragma unroll
+    for (int k = 0; k < N; ++k) o[k] = om[k] + ok[k];
+    o[0] += yp;
+    cp = c[p];
+    dp = d[p];
+    yp = o[p];
+    if (!store) return;
+    const long long zb = (long long)ez * layer_size;
+    if constexpr (FUSED && !DOT) {
+      // Dirichlet columns: phase Y took 0 for their values, the update takes
+      // what the vector holds
+      if (has && !inner) {
+#pragma unroll
+        for (int k = 0; k < p; ++k) us[k] = src[zb + (long long)k * plane + coff / ES];
       }
-      T om[N], ok[N];
-      eo_apply<N, 1>(tptab<N, T>(a.tab).M, d, om);
-#if SFK_TP_SCHED
-      __builtin_amdgcn_sched_barrier(0);
-#endif
-      eo_apply<N, 1>(tptab<N, T>(a.tab).K[2], c, ok);
+    }
+    const unsigned pb = opaque_s(plane_bytes);
+    const Rsrc rd = make_rsrc(dst + zb), rt = make_rsrc(CHEBY == 1 ? a.tm + zb : dst);
 #pragma unroll
-      for (int k = 0; k < N; ++k) o[k] = om[k] + ok[k];
-      o[0] += yp;
-      if (store) {
-        const bool bxy = X == 0 || Y == 0;
-#pragma unroll
-        for (int k = 0; k < p; ++k) {
-          const int Z = ez * p + k;
-          if constexpr (DELAY) po[k] = (bxy || Z == 0) ? T(0) : o[k];
-          else put_own(ez, k, (bxy || Z == 0) ? T(0) : o[k]);
-        }
+    for (int k = 0; k < p; ++k) {
+      const bool above = k > 0 || ez > 0; // not the grid's first plane
+      const T v = inner && above ? o[k] : T(0);
+      if constexpr (TT) {
+        const T dinv = above ? dinvk[k] : T(0);
+        const T rhs = RSRC ? us[k] : q_r[k];
+        const T z1 = a.s_rhs * dinv * rhs; // the first iterate, when formed here
+        const T ui = RSRC ? z1 : us[k];
+        const T pv = RPREV ? z1 : (RSRC ? T(0) : q_t[k]);
+        const T t = a.c_tm * (pv - ui) + a.c_np * dinv * (v - rhs);
+        buf_store<0>(rd, coff, k * pb, ui - t);
+      } else if constexpr (CHEBY == 1) {
+        const T res = v - q_r[k];
+        const T t = (a.c_tm != T(0) ? a.c_tm * q_t[k] : T(0)) + a.c_np * q_d[k] * res;
+        buf_store<0>(rt, coff, k * pb, t);
+        buf_store<0>(rd, coff, k * pb, us[k] - t);
+      } else {
+        buf_store<1>(rd, coff, k * pb, v);
+        if constexpr (DOT) dot_acc += double(us[k]) * double(v);
       }
-      cp = c[p];
-      dp = d[p];
-      yp = o[p];
     }
-    if (!DELAY && store && zone != 2) {
-#pragma unroll
-      for (int k = 0; k < p; ++k) put_zeros(ez * p + k, ez, k);
-    }
-  };
-  // the stores (and, CHEBY 5, the prefetch of the next layer's q_s) of the
-  // pending layer.  Vector-memory loads and stores share one completion
-  // counter, and these accesses sit in divergent branches, so the wait for
-  // the next layer's y lines (store_y) is a wait for everything issued
-  // before it: issued at the end of phase Z, the q_s prefetch of CHEBY 5 was
-  // waited for at the start of the next layer.  Issued right after that wait
-  // instead, it has a whole layer to arrive (Q6 64^3 FP64 CG-Chebyshev: the
-  // solve 2 % faster).  The plain matvec and the Chebyshev forms measured
-  // slower this way (the held outputs cost registers: Q6 FP64 matvec 337 ->
-  // 347 us, Chebyshev steps 583 -> 605 us).
-  // (ez: the layer whose outputs are pending, uniform)
-  auto flush = [&](int ez) {
-    if constexpr (DELAY) {
-      if (zone == 0)
-#pragma unroll
-        for (int k = 0; k < p; ++k) put_own(ez, k, po[k]);
-      if (zone != 2)
-#pragma unroll
-        for (int k = 0; k < p; ++k) put_zeros(ez * p + k, ez, k);
-    }
+    if (xtra)
+#pragma unroll 1
+      for (int k = 0; k < p; ++k) put_xtra(ez * p + k);
   };
 
-  using one = std::integral_constant<int, 1>;
-  using all = std::integral_constant<int, p>;
-  // one layer: phase Y from the prefetched registers, the next layer's
-  // loads, phases X and Z
-  auto layer = [&](int ez, bool store, int ez_next) {
-    store_y();
-    // the layer before this one stored its outputs (delayed form)
-    if (DELAY && store && ez > ez_begin) flush(ez - 1);
-    __syncthreads();
-    if (ez_next >= 0) load_y(ez_next, 1, all());
-    phase_x(all());
-    __syncthreads();
+  // one layer; next: the layer to prefetch (ez itself: none)
+  auto layer = [&](int ez, bool store, int next) {
+    if (!PF) load_y(ez, true);
+    phase_y(false);
+    if (PF) load_y(next, next > ez);
+    if (EARLY && store) load_streams(ez);
+    phase_x();
     phase_z(ez, store);
   };
   if (ez_begin > 0) {
     // carried state at plane ez_begin p: c, d of the plane below the cell
-    // below, then that cell's layer without stores.  The plane's and the
-    // layer's y lines are loaded together (two sets of registers): one
-    // memory round trip instead of two before the first sweep
-    {
-      T u0[2 * N - 1];
-      bool yact0 = false;
-      load_y_to(u0, yact0, ez_begin - 1, 0, one());
-      load_y(ez_begin - 1, 1, all());
-      store_y_from(u0, yact0);
-    }
-    __syncthreads();
-    phase_x(one());
-    __syncthreads();
-    if (zone == 0) {
-      cp = sC[Yt * RPC + Xt];
-      dp = sD[Yt * RPC + Xt];
-    }
-    layer(ez_begin - 1, false, ez_begin < ez_end ? ez_begin : -1);
-  } else if (ez_begin < ez_end) {
-    load_y(ez_begin, 1, all());
+    // below (slot 0; zero at the grid's first plane), then that cell's layer
+    // without stores
+    const int e0 = ez_begin - 1;
+    const bool on = ys == 0 && e0 > 0;
+    auto below = [&](unsigned o) { return on && o != kOob ? o - plane_bytes : kOob; };
+    load_lines(src + (long long)e0 * layer_size, kAll, below(o_first), below(o_low), below(o_mid), below(o_last));
+    phase_y(true);
+    if (PF) load_y(e0, true);
+    phase_x();
+    cp = za[0];
+    dp = za[C::LA];
+    if constexpr (FUSED) up = zu[0];
+    layer(e0, false, ez_begin);
+  } else {
+    if (PF) load_y(ez_begin, true);
+    if constexpr (FUSED && !DOT) up = has ? src[coff / ES] : T(0); // the first plane (Dirichlet)
   }
-  for (int ez = ez_begin; ez < ez_end; ++ez) layer(ez, true, ez + 1 < ez_end ? ez + 1 : -1);
-  if (DELAY && ez_end > ez_begin) flush(ez_end - 1);
+  // (vmcnt(0): entering the loop with no access pending, so that the wait
+  // for a layer's y lines inside it counts only what the loop issued)
+  __builtin_amdgcn_s_waitcnt(0x0f70);
+#pragma unroll 1
+  for (int ez = ez_begin; ez < ez_end; ++ez) layer(ez, true, ez + 1 < ez_end ? ez + 1 : ez);
   // the grid's last z plane (Dirichlet)
-  if (ez_end == a.nz && zone != 2) {
-    const int Z = gz - 1;
-    if (zone == 0) put(Z, coff, T(0));
-    put_zeros(Z, 0, -1);
+  if (ez_end == a.nz && has) {
+    put_zero(gz - 1, coff);
+    put_xtra(gz - 1);
   }
   if constexpr (DOT) {
     // workgroup sum of this thread's src . dst terms: within each wave by
@@ -574,7 +576,7 @@ cont_tp_kernel(const TpArgs<T> a)
     for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
     __syncthreads();
     double *red = reinterpret_cast<double *>(sA);
-    const int wave = threadIdx.x / 64, nw = (C::THREADS + 63) / 64;
+    const int wave = threadIdx.x / 64, nw = C::THREADS / 64;
     if (threadIdx.x % 64 == 0) red[wave] = v;
     __syncthreads();
     if (threadIdx.x == 0) {
@@ -707,7 +709,7 @@ static hipError_t launch_tp_shape(const TpLaunch &L, hipStream_t s)
   const long long nchunks = (a.nz + a.zc - 1) / a.zc;
   const long long blocks = (long long)a.ntx * a.nty * nchunks;
   if (blocks <= 0 || blocks > 0x7fffffffLL) return hipErrorInvalidConfiguration;
-  const size_t lds = size_t(C::LDS_VALUES) * sizeof(T);
+  const size_t lds = size_t(C::lds_values(L.cheby != 0 || L.dot_part)) * sizeof(T);
   // the matvec with src . dst (CHEBY 5) exists for FP64 only (the solver's
   // outer matvec)
   decltype(&cont_tp_kernel<N, T, BX, BY, 0>) kdot = nullptr;
@@ -724,20 +726,24 @@ static hipError_t launch_tp_shape(const TpLaunch &L, hipStream_t s)
   return hipGetLastError();
 }
 
-// tile shapes (BX, BY) per points per direction N; shape 0 is the default
-#define SFK_TP_SHAPES(X)                                                                       \
-  X(2, 0, 32, 16) X(2, 1, 64, 8) X(2, 2, 16, 32) X(2, 3, 32, 8) X(2, 4, 128, 4)                 \
-  X(3, 0, 16, 8) X(3, 1, 32, 4) X(3, 2, 8, 16) X(3, 3, 16, 4) X(3, 4, 64, 2)                    \
-  X(4, 0, 8, 8) X(4, 1, 16, 4) X(4, 2, 4, 16) X(4, 3, 8, 4) X(4, 4, 32, 2)                      \
-  X(5, 0, 8, 4) X(5, 1, 16, 2) X(5, 2, 8, 2) X(5, 3, 16, 1) X(5, 4, 32, 1) X(5, 5, 43, 1)                \
-  X(6, 0, 4, 4) X(6, 1, 8, 2) X(6, 2, 8, 4) X(6, 3, 4, 2) X(6, 4, 16, 1)                        \
-  X(7, 0, 4, 4) X(7, 1, 4, 2) X(7, 2, 8, 2) X(7, 3, 8, 1) X(7, 4, 16, 1) X(7, 5, 24, 1) X(7, 6, 22, 1) \
-  X(8, 0, 4, 2) X(8, 1, 2, 4) X(8, 2, 2, 2) X(8, 3, 4, 1) X(8, 4, 8, 1)                         \
-  X(9, 0, 4, 2) X(9, 1, 2, 2) X(9, 2, 4, 1) X(9, 3, 2, 1) X(9, 4, 8, 1)
+// Tile shapes (BX, BY) per points per direction N, from 1 (shape 0: tp_plan
+// chooses).  Wide in x (the x halo of p+1 columns costs (p+1)/(BX p)), with
+// BY p BX as large as fits and a phase Y that fills a multiple of four waves:
+// 4 or 8 of them spread evenly over the SIMDs (Q6 52x50x52 FP64: 13 x 1 cells
+// in 8 full waves 129 us, 7 x 1 in 5 waves 177 us, 16 x 1 in 10 waves 195 us).
+#define SFK_TP_SHAPES(X)                                                        \
+  X(2, 1, 30, 8) X(2, 2, 126, 4) X(2, 3, 62, 4) X(2, 4, 30, 16)                  \
+  X(3, 1, 30, 2) X(3, 2, 62, 2) X(3, 3, 30, 4) X(3, 4, 14, 4)                    \
+  X(4, 1, 27, 1) X(4, 2, 8, 3) X(4, 3, 27, 2) X(4, 4, 12, 2)                     \
+  X(5, 1, 14, 1) X(5, 2, 30, 1) X(5, 3, 9, 3) X(5, 4, 14, 2) X(5, 5, 6, 2)       \
+  X(6, 1, 9, 1) X(6, 2, 19, 1) X(6, 3, 16, 1) X(6, 4, 11, 1)                     \
+  X(7, 1, 13, 1) X(7, 2, 11, 1) X(7, 3, 5, 1) X(7, 4, 9, 1) X(7, 5, 24, 1) X(7, 6, 7, 1) \
+  X(8, 1, 4, 1) X(8, 2, 9, 1) X(8, 3, 7, 1) X(8, 4, 4, 2)                        \
+  X(9, 1, 6, 1) X(9, 2, 2, 1) X(9, 3, 4, 1) X(9, 4, 3, 1)
 
 int tp_shape_count(int n)
 {
-  int c = 0;
+  int c = 1;
 #define SFK_X(NN, SH, BXX, BYY) c += n == NN ? 1 : 0;
   SFK_TP_SHAPES(SFK_X)
 #undef SFK_X
@@ -756,20 +762,82 @@ void tp_shape(int n, int shape, int *bx, int *by)
 #undef SFK_X
 }
 
-size_t tp_lds_bytes(int n, int shape, bool fp32)
+// a CU (lds_max bytes) holds two workgroups of the matvec: below that the
+// kernel's phases have nothing to overlap with (Q6 52x50x52 FP64 on 24 x 1
+// cells, one workgroup of 94 KB per CU: 196 us instead of 129 us)
+bool tp_shape_fits(int n, int shape, bool fp32, size_t lds_max)
 {
   size_t v = 0;
 #define SFK_X(NN, SH, BXX, BYY) \
-  if (n == NN && shape == SH) v = (size_t)TpCfg<NN, double, BXX, BYY>::LDS_VALUES;
+  if (n == NN && shape == SH)   \
+    v = fp32 ? TpCfg<NN, float, BXX, BYY>::lds_values(false) * 4 : TpCfg<NN, double, BXX, BYY>::lds_values(false) * 8;
   SFK_TP_SHAPES(SFK_X)
 #undef SFK_X
-  return v * (fp32 ? 4 : 8);
+  return 2 * v <= lds_max;
+}
+
+// Modelled cost of a schedule, in work items x layers per CU.  A workgroup
+// costs its items, half of them rounded up to whole sets of four waves (the
+// wave that a SIMD has more than the others is waited for at every barrier),
+// and more where fewer than 16 waves of a CU are there to overlap;
+// its range of cells in z costs 1.2 layers more when it starts above the
+// bottom and 0.6 for its start; and a CU with few workgroups still needs the
+// latency of a layer, about what 500 items cost, per set of resident ones.
+double tp_cost(int n, const int nc[3], int shape, int zc)
+{
+  int bx = 0, by = 0;
+  tp_shape(n, shape, &bx, &by);
+  if (bx <= 0 || zc <= 0) return 1e300;
+  const int p = n - 1, items = p * by * (bx * p + p + 1), waves = (items + 63) / 64;
+  const long long tiles = (long long)((nc[0] + bx - 1) / bx) * ((nc[1] + by - 1) / by);
+  const long long chunks = (nc[2] + zc - 1) / zc, per_cu = (tiles * chunks + 255) / 256;
+  const long long slots = 16 / waves > 0 ? 16 / waves : 1;
+  const long long resident = (per_cu < slots ? per_cu : slots) * waves;
+  double work = double(per_cu) * (0.5 * items + 0.5 * 256 * ((waves + 3) / 4));
+  if (resident < 16) work *= std::sqrt(16. / double(resident));
+  const double latency = double((per_cu + slots - 1) / slots) * 500.;
+  return (zc + (chunks > 1 ? 1.8 : 0.6)) * (work > latency ? work : latency);
+}
+
+// cells in z per workgroup worth trying: the mesh in 1, 2, 3, ... parts
+std::vector<int> tp_zc_candidates(int nz)
+{
+  std::vector<int> v;
+  for (int k : {1, 2, 3, 4, 5, 6, 8, 10, 12, 16, 20, 24, 32, 48, 64, 96, 128})
+    if (k <= nz && (v.empty() || (nz + k - 1) / k != v.back())) v.push_back((nz + k - 1) / k);
+  if (v.back() != 1) v.push_back(1);
+  return v;
+}
+
+// the schedule of shape 0 and / or zc 0 (automatic): the cheapest by tp_cost.
+// Untuned Q6 64^3 FP64 380 -> 266 us (the tuner finds 264), Q4 16^3: see the
+// launch-bound meshes' 500-item latency above.
+void tp_plan(int n, bool fp32, const int nc[3], int *shape, int *zc)
+{
+  if (*shape > 0 && *zc > 0) return;
+  const std::vector<int> zcs = *zc > 0 ? std::vector<int>{*zc < nc[2] ? *zc : nc[2]} : tp_zc_candidates(nc[2]);
+  const int s0 = *shape > 0 ? *shape : 1, s1 = *shape > 0 ? *shape : tp_shape_count(n) - 1;
+  double best = -1.;
+  int bs = s0, bz = zcs[0];
+  for (int sh = s0; sh <= s1; ++sh) {
+    if (*shape == 0 && !tp_shape_fits(n, sh, fp32, 163840)) continue;
+    for (int z : zcs) {
+      const double c = tp_cost(n, nc, sh, z);
+      if (best < 0. || c < best) {
+        best = c;
+        bs = sh;
+        bz = z;
+      }
+    }
+  }
+  *shape = bs;
+  *zc = bz;
 }
 
 template <typename T>
 static hipError_t launch_tp_t(const TpLaunch &L, hipStream_t s)
 {
-  const int shape = L.shape >= 0 && L.shape < tp_shape_count(L.n) ? L.shape : 0;
+  const int shape = L.shape;
 #define SFK_X(NN, SH, BXX, BYY) \
   if (L.n == NN && shape == SH) return launch_tp_shape<NN, T, BXX, BYY>(L, s);
   SFK_TP_SHAPES(SFK_X)

@@ -69,7 +69,7 @@ struct TpLaunch {
   int nc[3] = {1, 1, 1};
   int nrhs = 1;
   long long vstride = 0;
-  int shape = 0;        // tile shape index (tp_shape)
+  int shape = 1;        // tile shape index (tp_shape)
   int zc = 0;           // cells in z per workgroup (0: all)
   int order = 1;        // block order
 };
@@ -78,7 +78,11 @@ long long tp_launch_blocks(const TpLaunch &L); // workgroups of one right-hand s
 hipError_t upload_tp_tables(const Tables1D &t, const double inv_jac[3], bool fp32, void **dev);
 int tp_shape_count(int n);
 void tp_shape(int n, int shape, int *bx, int *by);
-size_t tp_lds_bytes(int n, int shape, bool fp32);
+bool tp_shape_fits(int n, int shape, bool fp32, size_t lds_max);
+double tp_cost(int n, const int nc[3], int shape, int zc);
+std::vector<int> tp_zc_candidates(int nz);
+// resolves an automatic tile shape (0) and / or cells in z (0) for a mesh
+void tp_plan(int n, bool fp32, const int nc[3], int *shape, int *zc);
 hipError_t launch_cell_diagonal(const CellLaunch &L, hipStream_t stream);
 
 // DG-SIPG with per-quadrature-point metric (deformed mesh)

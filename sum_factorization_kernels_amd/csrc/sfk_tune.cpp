@@ -77,6 +77,18 @@ bool tp_ok(const sfk_op *op)
   return op->d.kind == SFK_CONT_LAPLACE && !(op->d.flags & SFK_FLAG_VARIABLE_COEF) && op->d.degree <= kMaxDegreeTp;
 }
 
+// modelled cost of the automatic schedule of the tensor-product kernel; the
+// tuner tries what is modelled within kTpTry of it (the fastest of a full
+// sweep over tiles and z ranges was modelled within 1.45 of the cheapest for
+// every degree, in both precisions, matvec and Chebyshev step)
+constexpr double kTpTry = 1.6;
+double tp_best_cost(const sfk_op *op)
+{
+  int shape = 0, zc = 0;
+  tp_plan(op->d.degree + 1, op->d.precision == SFK_FP32, op->d.n_cells, &shape, &zc);
+  return tp_cost(op->d.degree + 1, op->d.n_cells, shape, zc);
+}
+
 int max_cb(const sfk_op *op)
 {
   const int n = op->d.degree + 1;
@@ -189,7 +201,8 @@ sfk_status sfk_op_tile_shape(const sfk_op *op, int shape, int *count, int *bx, i
   const int n = op->d.degree + 1, c = tp_shape_count(n);
   if (count) *count = c;
   if (shape < 0 || shape >= c) TUNE_FAIL(SFK_ERR_INVALID_ARG, "tile shape must be in 0.." + std::to_string(c - 1));
-  int x = 0, y = 0;
+  int x = 0, y = 0, zc = 1;
+  if (shape == 0) tp_plan(n, op->d.precision == SFK_FP32, op->d.n_cells, &shape, &zc);
   tp_shape(n, shape, &x, &y);
   if (bx) *bx = x;
   if (by) *by = y;
@@ -218,9 +231,8 @@ sfk_status sfk_op_set_schedule(sfk_op *op, const sfk_schedule *s)
     TUNE_FAIL(SFK_ERR_INVALID_ARG, "tile_shape out of range");
   if (s->z_cells < 0) TUNE_FAIL(SFK_ERR_INVALID_ARG, "z_cells must be >= 0");
   if (s->cont_scatter == 2 || s->cont_scatter == -1) {
-    const size_t need = tp_lds_bytes(op->d.degree + 1, s->tile_shape, op->d.precision == SFK_FP32);
-    if (tp_ok(op) && need > (size_t)lds_limit())
-      TUNE_FAIL(SFK_ERR_UNSUPPORTED, "tile shape needs more LDS than the device has per workgroup");
+    if (tp_ok(op) && !tp_shape_fits(op->d.degree + 1, s->tile_shape, op->d.precision == SFK_FP32, lds_limit()))
+      TUNE_FAIL(SFK_ERR_UNSUPPORTED, "tile shape needs more LDS than leaves room for two workgroups per CU");
   }
   op->sched_cb = s->cells_per_block;
   op->sched_order = s->block_order;
@@ -320,20 +332,19 @@ sfk_status sfk_tune(sfk_op *op, int repeats, sfk_schedule *best, double *best_se
     if (tp_ok(op)) {
       // tensor-product kernel: tile shapes x cells in z per workgroup
       const int n = op->d.degree + 1, nz = op->d.n_cells[2];
-      const int lds_max = lds_limit();
-      std::vector<int> zcs;
-      for (int z = 1; z < nz; z *= 2) zcs.push_back(z);
-      zcs.push_back(nz);
-      for (int sh = 0; sh < tp_shape_count(n) && status == SFK_OK; ++sh) {
-        if (tp_lds_bytes(n, sh, op->d.precision == SFK_FP32) > (size_t)lds_max) continue;
+      const double tp_best = tp_best_cost(op);
+      const int win_cb = saved_cb > 0 ? saved_cb : default_cb(op); // (unused by this kernel)
+      for (int sh = 1; sh < tp_shape_count(n) && status == SFK_OK; ++sh) {
+        if (!tp_shape_fits(n, sh, op->d.precision == SFK_FP32, lds_limit())) continue;
         for (int order = 0; order <= 1 && status == SFK_OK; ++order)
-          for (int zc : zcs) {
+          for (int zc : tp_zc_candidates(nz)) {
             if (status != SFK_OK) break;
+            if (tp_cost(n, op->d.n_cells, sh, zc) > kTpTry * tp_best) continue;
             op->sched_order = order;
             op->cont_scatter = 2;
             op->tp_shape = sh;
             op->tp_zc = zc;
-            trial(sfk_schedule{saved_cb, order, 2, sh, zc});
+            trial(sfk_schedule{win_cb, order, 2, sh, zc});
           }
       }
     }
@@ -352,14 +363,13 @@ sfk_status sfk_tune(sfk_op *op, int repeats, sfk_schedule *best, double *best_se
     if (status == SFK_OK) status = sfk_vec_fill(op->d.precision, pv, op->nvec * op->d.n_rhs, 0.0, stream);
     if (status == SFK_OK) status = ensure_device_tables(op);
     const int n = op->d.degree + 1, nz = op->d.n_cells[2];
-    std::vector<int> zcs;
-    for (int z = 1; z < nz; z *= 2) zcs.push_back(z);
-    zcs.push_back(nz);
-    for (int sh = 0; sh < tp_shape_count(n) && status == SFK_OK; ++sh) {
-      if (tp_lds_bytes(n, sh, op->d.precision == SFK_FP32) > (size_t)lds_limit()) continue;
+    const double tp_best = tp_best_cost(op);
+    for (int sh = 1; sh < tp_shape_count(n) && status == SFK_OK; ++sh) {
+      if (!tp_shape_fits(n, sh, op->d.precision == SFK_FP32, lds_limit())) continue;
       for (int order = 0; order <= 1 && status == SFK_OK; ++order)
-        for (int zc : zcs) {
+        for (int zc : tp_zc_candidates(nz)) {
           if (status != SFK_OK) break;
+          if (tp_cost(n, op->d.n_cells, sh, zc) > kTpTry * tp_best) continue;
           op->cheby_shape = sh;
           op->cheby_order = order;
           op->cheby_zc = zc;
