@@ -201,34 +201,6 @@ __device__ __forceinline__ void line_one(const void *tab, const T (&in)[2 * N - 
 }
 
 
-// Buffer accesses: a uniform base, a 32-bit offset per lane and a uniform
-// offset.  A lane offset of kOob lies beyond every buffer described here
-// (fewer than 2^31 bytes): such lanes read 0 and store nothing.
-constexpr unsigned kOob = 0x80000000u, kAll = 0x7fffffffu;
-typedef unsigned sfk_u2 __attribute__((ext_vector_type(2)));
-using Rsrc = __amdgpu_buffer_rsrc_t;
-template <typename T>
-__device__ __forceinline__ Rsrc make_rsrc(const T *p, unsigned bytes = kAll)
-{
-  return __builtin_amdgcn_make_buffer_rsrc(const_cast<T *>(p), 0, (int)bytes, 0x00027000);
-}
-template <typename T>
-__device__ __forceinline__ T buf_load(Rsrc r, unsigned voff, unsigned soff)
-{
-  if constexpr (sizeof(T) == 8)
-    return __builtin_bit_cast(T, __builtin_amdgcn_raw_buffer_load_b64(r, (int)voff, (int)soff, 0));
-  else
-    return __builtin_bit_cast(T, __builtin_amdgcn_raw_buffer_load_b32(r, (int)voff, (int)soff, 0));
-}
-template <int NT, typename T>
-__device__ __forceinline__ void buf_store(Rsrc r, unsigned voff, unsigned soff, T v)
-{
-  constexpr int aux = NT ? 2 : 0; // non-temporal
-  if constexpr (sizeof(T) == 8)
-    __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(sfk_u2, v), r, (int)voff, (int)soff, aux);
-  else
-    __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, v), r, (int)voff, (int)soff, aux);
-}
 // the same value, unknown to the compiler: keeps multiples of a stride from
 // being hoisted out of the layer loop into scalar registers it then spills
 __device__ __forceinline__ unsigned opaque_s(unsigned v)

@@ -13,15 +13,25 @@
 //
 // One workgroup = cb consecutive cells, n^2 threads per cell; thread l owns
 // line l of every direction.  Phases (barrier between):
-//   0  cell block -> LDS U (coalesced), neighbour layers -> registers
-//   1  p = L~_x u (x line) -> P, q = L~_y u (y line) -> Q, r = L~_z u (z line, registers)
-//   2  P <- M_z P, Q <- M_z Q (z lines), U <- r
+//   0  z line of u from global memory; U <- u, P <- L~_z u (z lines)
+//   1  r = L~_x u (x line, registers), Q <- L~_y u (y line)
+//   2  P <- M_x P, Q <- M_x Q, U <- r (x lines)
 //   3  P <- M_y P, Q <- Q + M_y U (y lines)
-//   4  U <- M_x Q + P (x lines)
-//   5  U -> dst (coalesced), or the fused Chebyshev update of
+//   4  z line of M_z Q + P -> dst, or the fused Chebyshev update of
 //      evaluation_dg_laplacian.h:485-502 on the way out.
-// The same order of sums as the reference: f_x M_z M_y L~_x + M_x (M_z
-// f_y L~_y + M_y f_z L~_z).
+// (f_z M_y M_x L~_z + M_z (M_x f_y L~_y + M_y f_x L~_x); the factors f_d are
+// in the tables of L.)
+//
+// What bounds it: LDS accesses and HBM about equally.  Starting and ending on
+// z lines, whose lanes touch consecutive dofs, both the block load and the
+// store go straight between registers and memory: 17 LDS accesses per point
+// and 4 barriers, where a coalesced copy through LDS on both ends took 20 and
+// 5.  Measured, before -> after,
+// matvec: p = 3 56x50x55 FP64 44 -> 38 us (4.1 TB/s), FP32 24 -> 19.6 us; p = 5
+// 31x37x29 FP64 33.3 -> 29.3 us, FP32 18.4 -> 16 us; p = 7 22x25x24 FP32 21.4
+// -> 15.8 us; Chebyshev step p = 5 FP64 80 -> 70 us, p = 8 20x21x22 78 -> 62 us.
+// Tried and not kept: workgroups that loop over several blocks and load the
+// next one early (no faster at 4 to 64 workgroups per CU).
 #include "sfk_device.h"
 #include "sfk_kernels.h"
 
@@ -33,11 +43,45 @@ constexpr int kPcMaxThreads = 256;
 
 template <int N, typename T>
 struct PcTab {
-  Eo<N, T> L, M;  // symmetric: the same table serves both contraction directions
-  T v1, v2;       // neighbour coupling
-  T f[3];         // direction factors
-  T ld[N], md[N]; // diagonals of L and M (operator diagonal)
+  Eo<N, T> L[3], M; // f_d L, M; symmetric: the same table serves both contraction directions
+  T v1[3], v2[3];   // neighbour coupling, times f_d
+  T f[3];           // direction factors
+  T ld[N], md[N];   // diagonals of L and M (operator diagonal)
 };
+
+// LDS block of a cell (x fastest): for n = 4, 8 rows are padded by one
+// value, so that the x lines of consecutive rows, and with the plane pitch
+// the y lines too, fall on different banks (passes per access relative to the
+// conflict-free count, over the kernel's mix: n = 4 FP64 1.76 -> 1.24, n = 8
+// 3.88 -> 1.24).  Odd n gains nothing from it, and for n = 6 the workgroup
+// per CU that the larger block costs outweighs 1.84 -> 1.61 (p = 5 FP64 29.3
+// us unpadded, 32.4 us padded).
+template <int N>
+struct PcLds {
+  static constexpr int NP = N == 4 || N == 8 ? N + 1 : N, PP = N * NP, CS = N * PP;
+};
+template <int N, int DIR>
+__device__ __forceinline__ int pc_base(int l)
+{
+  using C = PcLds<N>;
+  return DIR == 0 ? (l / N) * C::PP + (l % N) * C::NP : (DIR == 1 ? (l / N) * C::PP + l % N : (l / N) * C::NP + l % N);
+}
+template <int N, int DIR, typename T>
+__device__ __forceinline__ void pc_read(const T *cell, int l, T (&v)[N])
+{
+  constexpr int st = DIR == 0 ? 1 : (DIR == 1 ? PcLds<N>::NP : PcLds<N>::PP);
+  const T *q = cell + pc_base<N, DIR>(l);
+#pragma unroll
+  for (int i = 0; i < N; ++i) v[i] = q[i * st];
+}
+template <int N, int DIR, typename T>
+__device__ __forceinline__ void pc_write(T *cell, int l, const T (&v)[N])
+{
+  constexpr int st = DIR == 0 ? 1 : (DIR == 1 ? PcLds<N>::NP : PcLds<N>::PP);
+  T *q = cell + pc_base<N, DIR>(l);
+#pragma unroll
+  for (int i = 0; i < N; ++i) q[i * st] = v[i];
+}
 
 template <int N, typename T>
 __device__ __forceinline__ const SFK_CONST_AS PcTab<N, T> &pctab(const PcTab<N, T> *p)
@@ -55,7 +99,7 @@ template <int N, typename T>
 constexpr int pc_waves()
 {
   constexpr int cb = pc_cells_per_block<N>();
-  return lds_waves_per_simd(3 * cb * CellLds<N, T>::CS * (int)sizeof(T), cb * N * N);
+  return lds_waves_per_simd(3 * cb * PcLds<N>::CS * (int)sizeof(T), cb * N * N);
 }
 
 template <int N, typename T>
@@ -89,16 +133,28 @@ __device__ __forceinline__ void pc_couple(T (&o)[N], const T (&nb)[4], T v1, T v
   o[N - 2] += v2 * nb[2];
 }
 
+// the two face layers of the lower and of the upper neighbour at face point l
 template <int N, int DIR, typename T>
 __device__ __forceinline__ void pc_load_layers(const T *src, const int (&nbr)[6], int l, T (&nb)[4])
 {
   constexpr long long N3 = N * N * N;
-  const T *lo = src + nbr[2 * DIR] * N3;
-  const T *hi = src + nbr[2 * DIR + 1] * N3;
-  nb[0] = lo[pc_idx<N, DIR>(l, N - 1)];
-  nb[1] = lo[pc_idx<N, DIR>(l, N - 2)];
-  nb[2] = hi[pc_idx<N, DIR>(l, 0)];
-  nb[3] = hi[pc_idx<N, DIR>(l, 1)];
+  const T *lo = src + nbr[2 * DIR] * N3 + pc_idx<N, DIR>(l, N - 2);
+  const T *hi = src + nbr[2 * DIR + 1] * N3 + pc_idx<N, DIR>(l, 0);
+  if constexpr (DIR == 0 && N % 2 == 0) {
+    // adjacent in memory, at even positions: one load each
+    typedef T T2 __attribute__((ext_vector_type(2), aligned(sizeof(T))));
+    const T2 a = *(const T2 *)lo, b = *(const T2 *)hi;
+    nb[0] = a.y;
+    nb[1] = a.x;
+    nb[2] = b.x;
+    nb[3] = b.y;
+  } else {
+    constexpr int st = line_stride<N, N, DIR>();
+    nb[0] = lo[st];
+    nb[1] = lo[0];
+    nb[2] = hi[0];
+    nb[3] = hi[st];
+  }
 }
 
 template <int N, typename T, bool COUPLE, bool CHEBY>
@@ -107,121 +163,148 @@ precomp_kernel(PcArgs<N, T> a)
 {
   constexpr int N2 = N * N, N3 = N2 * N;
   const int cb = a.cb;
-  constexpr int CS = CellLds<N, T>::CS;
-  T *U = dyn_lds<T>();
-  T *P = U + cb * CS, *Q = P + cb * CS;
+  constexpr int CS = PcLds<N>::CS;
+  // n <= 3: a z line's lanes cover less than a cache line, and six streams of
+  // such pieces cost more than coalesced copies through LDS on both ends (p = 2
+  // FP32 Chebyshev step 30 us flat, 36 us on z lines)
+  constexpr bool FLAT = CHEBY && N <= 3;
   const long long c0 = (long long)logical_block(blockIdx.x, gridDim.x, a.order) * cb;
   const long long voff = (long long)blockIdx.y * a.nvec;
   const T *src = a.src + voff;
   const int t = threadIdx.x, c = t / N2, l = t - c * N2;
-  const long long cell = c0 + c;
-  const bool act = c < cb && cell < a.ncells;
+  const bool act = c < cb && c0 + c < a.ncells;
+  // (the divisions of the cell's coordinates on the scalar unit)
+  int nbr[6] = {0, 0, 0, 0, 0, 0};
+  const long long cell = act ? locate_cell((unsigned)c0, (unsigned)c, a.nx, a.ny, a.nz, 0, nbr) : 0;
+  T *U = dyn_lds<T>() + (act ? c : 0) * CS;
+  T *P = U + cb * CS, *Q = P + cb * CS;
+  const long long g0 = cell * N3 + l; // this thread's z line: g0 + k N2
+  // FLAT: the block's nval consecutive values lie in LDS as in memory
+  static_assert(!FLAT || CS == N3, "unpadded");
   const long long rem = a.ncells - c0;
   const int nval = (rem < cb ? (int)rem : cb) * N3;
-  const T *sb = src + c0 * N3;
 
-  T nb[3][4];
-  if (COUPLE && act) {
-    int nbr[6];
-    periodic_neighbors((int)cell, a.nx, a.ny, a.nz, nbr);
-    pc_load_layers<N, 0>(src, nbr, l, nb[0]);
-    pc_load_layers<N, 1>(src, nbr, l, nb[1]);
-    pc_load_layers<N, 2>(src, nbr, l, nb[2]);
-  }
-  // blockDim.x >= cb n^2, so n rounds cover the cb n^3 values of the block;
-  // the loads are branch-free (index clamped into the block) so that all n
-  // are in flight together, and only the LDS writes are guarded
-  T keep[N];
+  T u[N], nb[3][4], keep[FLAT ? N : 1];
+  if constexpr (FLAT) {
+    // blockDim.x >= cb n^2: n rounds cover the block
 #pragma unroll
-  for (int k = 0; k < N; ++k) {
-    const int i = t + k * (int)blockDim.x;
-    keep[k] = sb[i < nval ? i : nval - 1];
-  }
+    for (int k = 0; k < N; ++k) {
+      const int i = t + k * (int)blockDim.x;
+      keep[k] = src[c0 * N3 + (i < nval ? i : nval - 1)];
+    }
 #pragma unroll
-  for (int k = 0; k < N; ++k) {
-    const int i = t + k * (int)blockDim.x;
-    if (i < nval) U[(i / N3) * CS + cl_off<N, T>(i % N3)] = keep[k];
+    for (int k = 0; k < N; ++k) {
+      const int i = t + k * (int)blockDim.x;
+      if (i < nval) dyn_lds<T>()[i] = keep[k];
+    }
+    __syncthreads();
+  }
+  if (act) {
+    if constexpr (FLAT) pc_read<N, 2>(U, l, u);
+    else
+#pragma unroll
+      for (int k = 0; k < N; ++k) u[k] = src[g0 + k * N2];
+    if constexpr (COUPLE) {
+      pc_load_layers<N, 2>(src, nbr, l, nb[2]);
+      pc_load_layers<N, 1>(src, nbr, l, nb[1]);
+      pc_load_layers<N, 0>(src, nbr, l, nb[0]);
+    }
+    if constexpr (!FLAT) pc_write<N, 2>(U, l, u);
+    const auto &pt = pctab(a.pt);
+    T o[N];
+    eo_apply<N, 1>(pt.L[2], u, o);
+    if constexpr (COUPLE) pc_couple(o, nb[2], pt.v1[2], pt.v2[2]);
+    pc_write<N, 2>(P, l, o);
   }
   __syncthreads();
-
-  T *Uc = U + c * CS, *Pc = P + c * CS, *Qc = Q + c * CS;
   T r[N];
   if (act) {
     const auto &pt = pctab(a.pt);
     T v[N], o[N];
-    cl_read<N, 0>(Uc, l, v);
-    eo_apply<N, 1>(pt.L, v, o);
-    if constexpr (COUPLE) pc_couple(o, nb[0], pt.v1, pt.v2);
-#pragma unroll
-    for (int i = 0; i < N; ++i) o[i] *= pt.f[0];
-    cl_write<N, 0>(Pc, l, o);
-    cl_read<N, 1>(Uc, l, v);
-    eo_apply<N, 1>(pt.L, v, o);
-    if constexpr (COUPLE) pc_couple(o, nb[1], pt.v1, pt.v2);
-#pragma unroll
-    for (int i = 0; i < N; ++i) o[i] *= pt.f[1];
-    cl_write<N, 1>(Qc, l, o);
-    cl_read<N, 2>(Uc, l, v);
-    eo_apply<N, 1>(pt.L, v, r);
-    if constexpr (COUPLE) pc_couple(r, nb[2], pt.v1, pt.v2);
-#pragma unroll
-    for (int i = 0; i < N; ++i) r[i] *= pt.f[2];
+    pc_read<N, 0>(U, l, v);
+    eo_apply<N, 1>(pt.L[0], v, r);
+    if constexpr (COUPLE) pc_couple(r, nb[0], pt.v1[0], pt.v2[0]);
+    pc_read<N, 1>(U, l, v);
+    eo_apply<N, 1>(pt.L[1], v, o);
+    if constexpr (COUPLE) pc_couple(o, nb[1], pt.v1[1], pt.v2[1]);
+    pc_write<N, 1>(Q, l, o);
   }
   __syncthreads();
   if (act) {
     const auto &pt = pctab(a.pt);
     T v[N], o[N];
-    cl_read<N, 2>(Pc, l, v);
+    pc_read<N, 0>(P, l, v);
     eo_apply<N, 1>(pt.M, v, o);
-    cl_write<N, 2>(Pc, l, o);
-    cl_read<N, 2>(Qc, l, v);
+    pc_write<N, 0>(P, l, o);
+    pc_read<N, 0>(Q, l, v);
     eo_apply<N, 1>(pt.M, v, o);
-    cl_write<N, 2>(Qc, l, o);
-    cl_write<N, 2>(Uc, l, r);
+    pc_write<N, 0>(Q, l, o);
+    pc_write<N, 0>(U, l, r);
   }
   __syncthreads();
+  // fused update: its streams are loaded one phase ahead (n <= 3: see below)
+  T s_rhs[CHEBY ? N : 1], s_diag[CHEBY ? N : 1], s_tm[CHEBY ? N : 1];
   if (act) {
+    if constexpr (CHEBY && !FLAT) {
+#pragma unroll
+      for (int k = 0; k < N; ++k) {
+        s_rhs[k] = a.rhs[g0 + k * N2];
+        s_diag[k] = a.diag[g0 + k * N2];
+        s_tm[k] = a.c_tm != T(0) ? a.tm[g0 + k * N2] : T(0); // c_tm == 0: tm not read
+      }
+    }
     const auto &pt = pctab(a.pt);
     T v[N], o[N];
-    cl_read<N, 1>(Pc, l, v);
+    pc_read<N, 1>(P, l, v);
     eo_apply<N, 1>(pt.M, v, o);
-    cl_write<N, 1>(Pc, l, o);
-    cl_read<N, 1>(Uc, l, v);
+    pc_write<N, 1>(P, l, o);
+    pc_read<N, 1>(U, l, v);
     eo_apply<N, 1>(pt.M, v, o);
-    cl_read<N, 1>(Qc, l, v);
+    pc_read<N, 1>(Q, l, v);
 #pragma unroll
     for (int i = 0; i < N; ++i) o[i] = v[i] + o[i];
-    cl_write<N, 1>(Qc, l, o);
+    pc_write<N, 1>(Q, l, o);
   }
   __syncthreads();
   if (act) {
     const auto &pt = pctab(a.pt);
     T v[N], o[N];
-    cl_read<N, 0>(Qc, l, v);
+    pc_read<N, 2>(Q, l, v);
     eo_apply<N, 1>(pt.M, v, o);
-    cl_read<N, 0>(Pc, l, v);
+    pc_read<N, 2>(P, l, v);
+    if constexpr (FLAT) {
 #pragma unroll
-    for (int i = 0; i < N; ++i) o[i] = o[i] + v[i];
-    cl_write<N, 0>(Uc, l, o);
-  }
-  __syncthreads();
-  const long long g0 = voff + c0 * N3;
+      for (int k = 0; k < N; ++k) o[k] += v[k];
+      pc_write<N, 2>(U, l, o);
+    }
 #pragma unroll
-  for (int k = 0; k < N; ++k) {
-    const int i = t + k * (int)blockDim.x;
-    if (i < nval) {
-      const T au = U[(i / N3) * CS + cl_off<N, T>(i % N3)];
+    for (int k = 0; k < (FLAT ? 0 : N); ++k) {
+      const long long g = g0 + k * N2;
+      const T au = o[k] + v[k];
       if constexpr (CHEBY) {
-        // r = A u - rhs; tm = c_tm tm + c_np diag r; dst = u - tm (tm not
-        // read when c_tm == 0)
-        const long long gi = g0 + i;
-        const T res = au - a.rhs[gi];
-        T tmv = a.c_np * a.diag[gi] * res;
-        if (a.c_tm != T(0)) tmv = a.c_tm * a.tm[gi] + tmv;
-        a.tm[gi] = tmv;
-        a.dst[gi] = keep[k] - tmv;
+        // r = A u - rhs; tm = c_tm tm + c_np diag r; dst = u - tm
+        const T res = au - s_rhs[k];
+        T tmv = a.c_np * s_diag[k] * res;
+        if (a.c_tm != T(0)) tmv = a.c_tm * s_tm[k] + tmv;
+        a.tm[g] = tmv;
+        a.dst[g] = u[k] - tmv;
       } else {
-        __builtin_nontemporal_store(au, a.dst + g0 + i); // written once
+        __builtin_nontemporal_store(au, a.dst + voff + g); // written once
+      }
+    }
+  }
+  if constexpr (FLAT) {
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < N; ++k) {
+      const int i = t + k * (int)blockDim.x;
+      if (i < nval) {
+        const long long g = c0 * N3 + i;
+        const T res = dyn_lds<T>()[i] - a.rhs[g];
+        T tmv = a.c_np * a.diag[g] * res;
+        if (a.c_tm != T(0)) tmv = a.c_tm * a.tm[g] + tmv;
+        a.tm[g] = tmv;
+        a.dst[g] = keep[k] - tmv;
       }
     }
   }
@@ -264,7 +347,7 @@ hipError_t launch_precomp_n(const PrecompLaunch &L, hipStream_t s)
   if (L.cheby && L.nrhs != 1) return hipErrorInvalidValue;
   a.cb = CB;
   a.order = L.order;
-  const size_t lds = size_t(3) * CB * CellLds<N, T>::CS * sizeof(T);
+  const size_t lds = size_t(3) * CB * PcLds<N>::CS * sizeof(T);
   const dim3 grid((unsigned)((L.ncells + CB - 1) / CB), (unsigned)L.nrhs), block(((CB * N * N + 63) / 64) * 64);
   decltype(&precomp_kernel<N, T, true, false>) kern;
   if (L.couple) kern = L.cheby ? precomp_kernel<N, T, true, true> : precomp_kernel<N, T, true, false>;
@@ -278,7 +361,7 @@ hipError_t launch_precomp_n(const PrecompLaunch &L, hipStream_t s)
 template <int N, typename T>
 size_t precomp_lds_per_cell_n()
 {
-  return size_t(3) * CellLds<N, T>::CS * sizeof(T);
+  return size_t(3) * PcLds<N>::CS * sizeof(T);
 }
 
 template <int N, typename T>
@@ -296,11 +379,15 @@ template <int N, typename T>
 hipError_t upload_pctab(const Precomp1D &pc, const double f[3], void **dev)
 {
   PcTab<N, T> h{};
-  h.L = make_eo<N, T>(pc.lap, true);
   h.M = make_eo<N, T>(pc.mass, true);
-  h.v1 = T(pc.v1);
-  h.v2 = T(pc.v2);
-  for (int d = 0; d < 3; ++d) h.f[d] = T(f[d]);
+  for (int d = 0; d < 3; ++d) {
+    std::vector<double> L(pc.lap);
+    for (double &v : L) v *= f[d];
+    h.L[d] = make_eo<N, T>(L, true);
+    h.v1[d] = T(f[d] * pc.v1);
+    h.v2[d] = T(f[d] * pc.v2);
+    h.f[d] = T(f[d]);
+  }
   for (int i = 0; i < N; ++i) {
     h.ld[i] = T(pc.lap[i * N + i]);
     h.md[i] = T(pc.mass[i * N + i]);
