@@ -5,7 +5,8 @@
 //                homogeneous Dirichlet rows (colored stores or atomic scatter-add),
 //   Mode::DG     DG-SIPG on a Cartesian periodic mesh with the fused
 //                Chebyshev update (EvaluationDGLaplacian::do_inner_loop,
-//                legacy/include/evaluation_dg_laplacian.h:129-510).
+//                legacy/include/evaluation_dg_laplacian.h:129-510): degrees
+//                above 8 and the reference-compatible x sweep.
 //
 // One workgroup processes CB cells; each cell gets N*N threads.  Thread l of
 // a cell owns line l of every direction (x-line (j,k), y-line (i,k), z-line
@@ -769,11 +770,14 @@ static hipError_t launch_cell_n(const CellLaunch &L, hipStream_t stream)
     }
     return hipSuccess;
   }
-  if (L.cheby)
-    return launch(L.refx ? cell_kernel<N, T, Mode::DG, true, true, false> : cell_kernel<N, T, Mode::DG, true, false, false>,
+  if (L.refx)
+    return launch(L.cheby ? cell_kernel<N, T, Mode::DG, true, true, false> : cell_kernel<N, T, Mode::DG, false, true, false>,
                   grid);
-  return launch(L.refx ? cell_kernel<N, T, Mode::DG, false, true, false> : cell_kernel<N, T, Mode::DG, false, false, false>,
-                grid);
+  // (up to degree 8 the operator runs as a sum of Kronecker products)
+  if constexpr (N - 1 > kMaxDegreeTp)
+    return launch(L.cheby ? cell_kernel<N, T, Mode::DG, true, false, false> : cell_kernel<N, T, Mode::DG, false, false, false>,
+                  grid);
+  else return hipErrorInvalidValue;
 }
 
 template <int N, typename T>

@@ -11,7 +11,12 @@
 // inv_jac_d^2 / (inv_jac_x inv_jac_y inv_jac_z) (1 on the reference's unit
 // cells).  Periodic in every direction.
 //
-// One workgroup = cb consecutive cells, n^2 threads per cell; thread l owns
+// The Cartesian DG-SIPG operator is the same sum with the penalty (p+1)^2/h
+// instead of p(p+1)/h and runs here too (degree <= 8): (p+1)-point Gauss
+// quadrature integrates its 1D mass and stiffness exactly.
+//
+// One workgroup = cb cells in a row of the traversal (block order 2: slabs of
+// z-layers), n^2 threads per cell; thread l owns
 // line l of every direction.  Phases (barrier between):
 //   0  z line of u from global memory; U <- u, P <- L~_z u (z lines)
 //   1  r = L~_x u (x line, registers), Q <- L~_y u (y line)
@@ -175,7 +180,7 @@ precomp_kernel(PcArgs<N, T> a)
   const bool act = c < cb && c0 + c < a.ncells;
   // (the divisions of the cell's coordinates on the scalar unit)
   int nbr[6] = {0, 0, 0, 0, 0, 0};
-  const long long cell = act ? locate_cell((unsigned)c0, (unsigned)c, a.nx, a.ny, a.nz, 0, nbr) : 0;
+  const long long cell = act ? locate_cell((unsigned)c0, (unsigned)c, a.nx, a.ny, a.nz, FLAT ? 0 : a.order, nbr) : 0;
   T *U = dyn_lds<T>() + (act ? c : 0) * CS;
   T *P = U + cb * CS, *Q = P + cb * CS;
   const long long g0 = cell * N3 + l; // this thread's z line: g0 + k N2

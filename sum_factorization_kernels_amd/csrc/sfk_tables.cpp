@@ -231,7 +231,7 @@ std::vector<double> gll_points(int n)
   return p;
 }
 
-bool build_precomp_1d(int degree, bool ref_coupling, Precomp1D &pc)
+bool build_precomp_1d(int degree, double sigma, bool ref_coupling, Precomp1D &pc)
 {
   if (degree < 1 || degree > kMaxDegree) return false;
   const int n = degree + 1;
@@ -249,7 +249,6 @@ bool build_precomp_1d(int degree, bool ref_coupling, Precomp1D &pc)
     d0[i] = hb.derivative(i, 0.);
     d1[i] = hb.derivative(i, 1.);
   }
-  const double sigma = double(degree) * n;
   pc.mass.assign(n * n, 0.);
   pc.lap.assign(n * n, 0.);
   for (int i = 0; i < n; ++i)
