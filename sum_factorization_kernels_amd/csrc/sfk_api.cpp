@@ -315,7 +315,15 @@ sfk_status sfk_op_set_coefficient(sfk_op *op, const double *host, size_t count)
 {
   SFK_REQUIRE(op, SFK_ERR_INVALID_ARG, "null handle");
   SFK_REQUIRE(op->d.flags & SFK_FLAG_VARIABLE_COEF, SFK_ERR_INVALID_ARG, "operator lacks SFK_FLAG_VARIABLE_COEF");
-  return upload(op, &op->coef, host, count, (size_t)op->ncq, "coefficient");
+  SFK_REQUIRE(host != nullptr, SFK_ERR_INVALID_ARG, "coefficient: null host pointer");
+  SFK_REQUIRE(count == (size_t)op->ncq, SFK_ERR_INVALID_ARG,
+              "coefficient: expected " + std::to_string(op->ncq) + " values, got " + std::to_string(count));
+  // stored times the quadrature weight of its point
+  const std::vector<double> &w = op->tab.weights;
+  const size_t n = w.size();
+  std::vector<double> kw(count);
+  for (size_t i = 0; i < count; ++i) kw[i] = host[i] * w[i % n] * (w[i / n % n] * w[i / (n * n) % n]);
+  return upload(op, &op->coef, kw.data(), count, (size_t)op->ncq, "coefficient");
 }
 
 sfk_status sfk_op_set_velocity(sfk_op *op, const double *cell_host, size_t cell_count, const double *face_host,
@@ -350,7 +358,19 @@ sfk_status sfk_op_set_coefficient_device(sfk_op *op, const void *dev, size_t cou
 {
   SFK_REQUIRE(op, SFK_ERR_INVALID_ARG, "null handle");
   SFK_REQUIRE(op->d.flags & SFK_FLAG_VARIABLE_COEF, SFK_ERR_INVALID_ARG, "operator lacks SFK_FLAG_VARIABLE_COEF");
-  return copy_device(op, &op->coef, dev, count, (size_t)op->ncq, "coefficient", (hipStream_t)stream);
+  SFK_REQUIRE(dev != nullptr, SFK_ERR_INVALID_ARG, "coefficient: null device pointer");
+  SFK_REQUIRE(count == (size_t)op->ncq, SFK_ERR_INVALID_ARG,
+              "coefficient: expected " + std::to_string(op->ncq) + " values, got " + std::to_string(count));
+  SFK_ENSURE_TABLES(op);
+  if (op->coef == nullptr && hipMalloc(&op->coef, count * elem_size(op)) != hipSuccess) {
+    op->coef = nullptr;
+    set_error("coefficient: hipMalloc failed");
+    return SFK_ERR_ALLOC;
+  }
+  // stored times the quadrature weight of its point
+  SFK_CHECK_HIP(weight_qdata(op->d.degree + 1, op->d.precision == SFK_FP32, op->dtab, dev, op->coef,
+                             (long long)count, (hipStream_t)stream));
+  return SFK_OK;
 }
 
 sfk_status sfk_op_set_velocity_device(sfk_op *op, const void *cell_dev, size_t cell_count, const void *face_dev,

@@ -56,7 +56,7 @@ struct CellArgs {
   const T *rhs, *diag; // Chebyshev
   T *tm;
   T c_np, c_tm;
-  const T *coef;   // per cell q-point coefficient (optional)
+  const T *coef;   // coefficient times quadrature weight per cell q-point (optional)
   long long ncells;
   int nx, ny, nz;  // cells per direction
   int gx, gy, gz;  // node grid (continuous)
@@ -119,11 +119,9 @@ __device__ __forceinline__ void grad_phase(const CellArgs<N, T> &a, const T *Ace
   const T c = a.cdiag[DIR];
 #pragma unroll
   for (int i = 0; i < N; ++i) {
-    T f = c * line_weight<N, DIR>(tb.w, l, i);
-    if constexpr (COEF) {
-      const int dof = line_base<N, N, DIR>(l) + i * line_stride<N, N, DIR>();
-      f *= a.coef[cell * (N * N * N) + dof];
-    }
+    T f;
+    if constexpr (COEF) f = c * a.coef[cell * (N * N * N) + line_base<N, N, DIR>(l) + i * line_stride<N, N, DIR>()];
+    else f = c * line_weight<N, DIR>(tb.w, l, i);
     g[i] *= f;
   }
   eo_apply<N, -1>(tb.Db, g, r);
@@ -146,18 +144,24 @@ __device__ __forceinline__ void grad_phase(const CellArgs<N, T> &a, const T *Ace
 // instead of one row per lane.  Values added to are all loaded before the
 // first store.  Called by every thread of the workgroup (barrier inside);
 // sA (the A sweep array, dead at this point) holds the rows.
-template <int N, typename T>
-__device__ __forceinline__ void cont_store_colored(const CellArgs<N, T> &a, T (&o)[N], T *sA, const T *sB, bool act,
-                                                   int c, int l, int cy, int cz, int seg, int cx0, int cx_end, T *dst)
+// NR right-hand sides (nr of them present) share the index arithmetic: arrays
+// of right-hand side r at sA + r rs, its vector at dst + r a.vstride.
+template <int N, typename T, int NR = 1>
+__device__ __forceinline__ void cont_store_colored(const CellArgs<N, T> &a, T (&o)[NR][N], T *sA, const T *sB, int rs,
+                                                   int nr, bool act, int c, int l, int cy, int cz, int seg, int cx0,
+                                                   int cx_end, T *dst)
 {
   constexpr int p = N - 1, N2 = N * N, N3 = N2 * N;
   const int ncs = cx_end - cx0, Lx = ncs * p + 1;
   if (act) {
-    if (c + 1 < ncs) o[p] += sB[(c + 1) * N3 + l];
-    T *row = sA + l * Lx + c * p;
 #pragma unroll
-    for (int i = 0; i < N; ++i)
-      if (i > 0 || c == 0) row[i] = o[i];
+    for (int r = 0; r < NR; ++r) {
+      if (c + 1 < ncs) o[r][p] += sB[r * rs + (c + 1) * N3 + l];
+      T *row = sA + r * rs + l * Lx + c * p;
+#pragma unroll
+      for (int i = 0; i < N; ++i)
+        if (i > 0 || c == 0) row[i] = o[r][i];
+    }
   }
   // per-row terms of the segment's N2 node rows, made once per row instead
   // of once per node: the index of the row's first node, a Dirichlet-row
@@ -185,14 +189,14 @@ __device__ __forceinline__ void cont_store_colored(const CellArgs<N, T> &a, T (&
   const unsigned mlx = ((1u << 20) + unsigned(Lx) - 1u) / unsigned(Lx);
   int mode[N]; // 0 nothing, 1 store, 2 add
   long long gi[N];
-  T val[N], old[N];
+  T val[NR][N], old[NR][N];
 #pragma unroll
   for (int r = 0; r < N; ++r) {
     const int idx = (int)threadIdx.x + r * (int)blockDim.x;
     mode[r] = 0;
     gi[r] = 0;
-    val[r] = T(0);
-    old[r] = T(0);
+#pragma unroll
+    for (int q = 0; q < NR; ++q) val[q][r] = old[q][r] = T(0);
     if (idx < total) {
       const int rw = (int)((unsigned(idx) * mlx) >> 20), xi = idx - rw * Lx;
       const int fl = s_rflag[rw];
@@ -202,7 +206,8 @@ __device__ __forceinline__ void cont_store_colored(const CellArgs<N, T> &a, T (&
       const int X = cx0 * p + xi;
       const bool bd = (fl & 4) || X == 0 || X == a.gx - 1;
       gi[r] = s_rbase[rw] + xi;
-      val[r] = bd ? T(0) : sA[idx];
+#pragma unroll
+      for (int q = 0; q < NR; ++q) val[q][r] = bd ? T(0) : sA[q * rs + idx];
       mode[r] = m == a.color ? 1 : (bd ? 0 : 2);
     }
   }
@@ -210,13 +215,57 @@ __device__ __forceinline__ void cont_store_colored(const CellArgs<N, T> &a, T (&
   // together (interleaved with the index arithmetic above, the compiler
   // waited for each before the next)
 #pragma unroll
-  for (int r = 0; r < N; ++r)
-    if (mode[r] == 2) old[r] = dst[gi[r]];
+  for (int q = 0; q < NR; ++q)
+    if (q < nr)
 #pragma unroll
-  for (int r = 0; r < N; ++r) {
-    if (mode[r] == 1) dst[gi[r]] = val[r];
-    else if (mode[r] == 2) dst[gi[r]] = old[r] + val[r];
+      for (int r = 0; r < N; ++r)
+        if (mode[r] == 2) old[q][r] = dst[q * a.vstride + gi[r]];
+#pragma unroll
+  for (int q = 0; q < NR; ++q)
+    if (q < nr)
+#pragma unroll
+      for (int r = 0; r < N; ++r) {
+        if (mode[r] == 1) dst[q * a.vstride + gi[r]] = val[q][r];
+        else if (mode[r] == 2) dst[q * a.vstride + gi[r]] = old[q][r] + val[q][r];
+      }
+}
+
+// A workgroup's cells of the continuous operator: the row-segment
+// decomposition of a colour >= 0, or cells in index order (atomic scatter)
+struct ContPos {
+  int seg, cx, cy, cz, cx0, cx_end;
+  long long cell0;
+  bool act;
+};
+template <int N, typename T>
+__device__ __forceinline__ ContPos cont_position(const CellArgs<N, T> &a, unsigned blk, int c)
+{
+  const int CB = a.cb;
+  ContPos q{};
+  if (a.color >= 0) {
+    const int si = (int)(blk % a.nss);
+    const int rest = (int)(blk / a.nss);
+    q.seg = (a.color >> 2 & 1) + 2 * si;
+    q.cy = (a.color & 1) + 2 * (rest % a.nry);
+    q.cz = (a.color >> 1 & 1) + 2 * (rest / a.nry);
+    q.cx0 = q.seg * CB;
+    q.cx_end = q.cx0 + CB < a.nx ? q.cx0 + CB : a.nx;
+    q.cx = q.cx0 + c;
+    q.cell0 = ((long long)q.cz * a.ny + q.cy) * a.nx + q.cx0;
+    q.act = c < CB && q.cx < q.cx_end;
+  } else {
+    // cell0's coordinates are uniform; cell0 + c is c steps further in x
+    // unless that crosses the end of the row
+    q.cell0 = (long long)blk * CB;
+    q.act = c < CB && q.cell0 + c < a.ncells;
+    CellXYZ x = traverse_xyz((unsigned)q.cell0, a.nx, a.ny, a.nz, 0);
+    if (x.x + c < (unsigned)a.nx) x.x += c;
+    else x = traverse_xyz((unsigned)(q.cell0 + c), a.nx, a.ny, a.nz, 0);
+    q.cx = (int)x.x;
+    q.cy = (int)x.y;
+    q.cz = (int)x.z;
   }
+  return q;
 }
 
 template <int N, typename T, Mode MODE, bool CHEBY, bool REFX, bool COEF>
@@ -235,32 +284,12 @@ cell_kernel(const CellArgs<N, T> a)
   const int c = t / N2, l = t % N2;
   const unsigned blk = logical_block(blockIdx.x, gridDim.x, a.order);
   long long cell0 = (long long)blk * CB;
-  // continuous: coordinates of this thread's cell; a colour >= 0 selects the
-  // row-segment decomposition, a negative one the cell-linear atomic variant
-  int seg = 0, ccx = 0, ccy = 0, ccz = 0, cx0 = 0, cx_end = 0;
+  ContPos q{};
   bool act = c < CB && cell0 + c < a.ncells;
   if constexpr (MODE == Mode::Cont) {
-    if (a.color >= 0) {
-      const int si = (int)(blk % a.nss);
-      const int rest = (int)(blk / a.nss);
-      seg = (a.color >> 2 & 1) + 2 * si;
-      ccy = (a.color & 1) + 2 * (rest % a.nry);
-      ccz = (a.color >> 1 & 1) + 2 * (rest / a.nry);
-      cx0 = seg * CB;
-      cx_end = cx0 + CB < a.nx ? cx0 + CB : a.nx;
-      ccx = cx0 + c;
-      cell0 = ((long long)ccz * a.ny + ccy) * a.nx + cx0;
-      act = c < CB && ccx < cx_end;
-    } else {
-      // cell0's coordinates are uniform; cell0 + c is c steps further in x
-      // unless that crosses the end of the row
-      CellXYZ q = traverse_xyz((unsigned)cell0, a.nx, a.ny, a.nz, 0);
-      if (q.x + c < (unsigned)a.nx) q.x += c;
-      else q = traverse_xyz((unsigned)(cell0 + c), a.nx, a.ny, a.nz, 0);
-      ccx = (int)q.x;
-      ccy = (int)q.y;
-      ccz = (int)q.z;
-    }
+    q = cont_position(a, blk, c);
+    cell0 = q.cell0;
+    act = q.act;
   }
   // DG: the cell at this traversal position and its periodic face neighbours
   int nbr[6] = {0, 0, 0, 0, 0, 0};
@@ -285,12 +314,12 @@ cell_kernel(const CellArgs<N, T> a)
       if constexpr (MODE == Mode::Cont) {
         // (staging the segment's node rows through LDS for coalesced loads
         // measured slower: the extra barrier costs more than it saves)
-        const int X = ccx * p + l % N, Y = ccy * p + l / N;
+        const int X = q.cx * p + l % N, Y = q.cy * p + l / N;
         const bool bxy = X == 0 || Y == 0 || X == a.gx - 1 || Y == a.gy - 1;
-        const long long g0 = (long long)ccz * p * a.gy * a.gx + (long long)Y * a.gx + X;
+        const long long g0 = (long long)q.cz * p * a.gy * a.gx + (long long)Y * a.gx + X;
 #pragma unroll
         for (int k = 0; k < N; ++k) {
-          const int Z = ccz * p + k;
+          const int Z = q.cz * p + k;
           const bool bd = bxy || Z == 0 || Z == a.gz - 1;
           u[k] = bd ? T(0) : src[g0 + (long long)k * a.gy * a.gx];
         }
@@ -419,7 +448,8 @@ cell_kernel(const CellArgs<N, T> a)
     }
     __syncthreads();
     // --------------------------------------------------------------- Bx
-    T o[N];
+    T oo[1][N];
+    T(&o)[N] = oo[0];
     if (act) {
       const auto &tb = ctab(a.dt);
       T u[N];
@@ -436,14 +466,14 @@ cell_kernel(const CellArgs<N, T> a)
     if constexpr (MODE == Mode::Cont) {
       if (a.color >= 0) {
         __syncthreads();
-        cont_store_colored<N, T>(a, o, sA, sB, act, c, l, ccy, ccz, seg, cx0, cx_end, dst);
+        cont_store_colored<N, T>(a, oo, sA, sB, 0, 1, act, c, l, q.cy, q.cz, q.seg, q.cx0, q.cx_end, dst);
       } else if (act) {
-        const int Y = ccy * p + l % N, Z = ccz * p + l / N;
+        const int Y = q.cy * p + l % N, Z = q.cz * p + l / N;
         const bool byz = Y == 0 || Z == 0 || Y == a.gy - 1 || Z == a.gz - 1;
-        const long long g0 = ((long long)Z * a.gy + Y) * a.gx + (long long)ccx * p;
+        const long long g0 = ((long long)Z * a.gy + Y) * a.gx + (long long)q.cx * p;
 #pragma unroll
         for (int i = 0; i < N; ++i) {
-          const int X = ccx * p + i;
+          const int X = q.cx * p + i;
           if (!(byz || X == 0 || X == a.gx - 1)) atomicAdd(dst + g0 + i, o[i]);
         }
       }
@@ -471,6 +501,171 @@ cell_kernel(const CellArgs<N, T> a)
         for (int i = 0; i < N; ++i) __builtin_nontemporal_store(o[i], dst + g0 + i);
       }
     }
+  }
+}
+
+// Continuous Laplacian with a coefficient per q-point, NR right-hand sides per
+// workgroup.  Phases (barrier between):
+//   L   z line of the input -> z value sweep -> A
+//   V1  x value sweep on A
+//   Gy  y value sweep -> A; y gradient, coefficient, transposed gradient -> B
+//   Gx  the same for x on A, B += ...
+//   Gz  the same for z, + B, transposed z value sweep -> A
+//   By  transposed y value sweep on A
+//   Bx  transposed x value sweep, colored stores or atomic adds
+// What bounds it: VALU issue and the latency between the phases.  Two
+// right-hand sides share the coefficient, the table loads, the index
+// arithmetic of the colored store and the barriers; the coefficient holds the
+// quadrature weight (one product per point and direction instead of four) and
+// the y gradient follows its value sweep in registers (15 LDS accesses per
+// point instead of 16, 7 phases instead of 8).  Measured, before -> after (all
+// right-hand sides of one apply): p = 2 80x70x75, 8, FP32 401 -> 300 us; p = 4
+// 40x37x42, 3, FP64 181 -> 163 us; p = 5 24x26x28, 5, FP32 132 -> 114 us; p = 8
+// 24^3, 1, FP64 143 -> 134 us, but 8, FP32 467 -> 465 us: there the workgroups a
+// CU holds, and the tails of the 8 launches (15 %), set the time.
+template <int N, typename T, int NR>
+__global__ void __launch_bounds__(kCellMaxThreads)
+__attribute__((amdgpu_waves_per_eu(1, lds_waves_per_simd(NR * cells_per_block<N>() * 2 * N * N * N * (int)sizeof(T), cells_per_block<N>() * N * N))))
+cont_coef_kernel(const CellArgs<N, T> a)
+{
+  constexpr int N2 = N * N, N3 = N2 * N, p = N - 1;
+  const int CB = a.cb, rs = 2 * CB * N3; // arrays of one right-hand side
+  T *sA = dyn_lds<T>(), *sB = sA + CB * N3;
+  const int t = threadIdx.x, c = t / N2, l = t % N2;
+  const ContPos q = cont_position(a, logical_block(blockIdx.x, gridDim.x, a.order), c);
+  const bool act = q.act;
+  T *A = sA + (act ? c : 0) * N3, *B = sB + (act ? c : 0) * N3;
+  const int r0 = (int)blockIdx.y * NR, nr = a.nrhs - r0 < NR ? a.nrhs - r0 : NR;
+  const T *src = a.src + r0 * a.vstride;
+  T *dst = a.dst + r0 * a.vstride;
+  const T *coef = a.coef + (q.cell0 + (act ? c : 0)) * N3;
+
+  if (act) {
+    const int X = q.cx * p + l % N, Y = q.cy * p + l / N;
+    const bool bxy = X == 0 || Y == 0 || X == a.gx - 1 || Y == a.gy - 1;
+    const long long plane = (long long)a.gy * a.gx, g0 = (long long)q.cz * p * plane + (long long)Y * a.gx + X;
+    T u[NR][N], v[N];
+#pragma unroll
+    for (int r = 0; r < NR; ++r)
+#pragma unroll
+      for (int k = 0; k < N; ++k) {
+        const int Z = q.cz * p + k;
+        u[r][k] = bxy || Z == 0 || Z == a.gz - 1 || r >= nr ? T(0) : src[r * a.vstride + g0 + k * plane];
+      }
+#pragma unroll
+    for (int r = 0; r < NR; ++r) {
+      eo_apply<N, 1>(ctab(a.dt).Sf, u[r], v);
+      lds_write_line<N, N, 2>(A + r * rs, l, v);
+    }
+  }
+  __syncthreads();
+  if (act) {
+#pragma unroll
+    for (int r = 0; r < NR; ++r) {
+      T u[N], v[N];
+      lds_read_line<N, N, 0>(A + r * rs, l, u);
+      eo_apply<N, 1>(ctab(a.dt).Sf, u, v);
+      lds_write_line<N, N, 0>(A + r * rs, l, v);
+    }
+  }
+  // the coefficient of this thread's line of direction DIR
+  auto load_coef = [&](auto dirc, T(&k)[N]) {
+    constexpr int DIR = decltype(dirc)::value;
+    const T *kl = coef + line_base<N, N, DIR>(l);
+#pragma unroll
+    for (int i = 0; i < N; ++i) k[i] = kl[i * line_stride<N, N, DIR>()];
+  };
+  // r = D^T (cdiag k) D v
+  auto grad = [&](int dir, const T(&k)[N], const T(&v)[N], T(&r)[N]) {
+    T g[N];
+    eo_apply<N, -1>(ctab(a.dt).Df, v, g);
+#pragma unroll
+    for (int i = 0; i < N; ++i) g[i] *= a.cdiag[dir] * k[i];
+    eo_apply<N, -1>(ctab(a.dt).Db, g, r);
+  };
+  using dir0 = std::integral_constant<int, 0>;
+  using dir1 = std::integral_constant<int, 1>;
+  using dir2 = std::integral_constant<int, 2>;
+  T k[N];
+  if (act) load_coef(dir1(), k);
+  __syncthreads();
+  if (act) {
+#pragma unroll
+    for (int r = 0; r < NR; ++r) {
+      T u[N], v[N], w[N];
+      lds_read_line<N, N, 1>(A + r * rs, l, u);
+      eo_apply<N, 1>(ctab(a.dt).Sf, u, v);
+      lds_write_line<N, N, 1>(A + r * rs, l, v);
+      grad(1, k, v, w);
+      lds_write_line<N, N, 1>(B + r * rs, l, w);
+    }
+    load_coef(dir0(), k);
+  }
+  __syncthreads();
+  if (act) {
+#pragma unroll
+    for (int r = 0; r < NR; ++r) {
+      T v[N], w[N], b[N];
+      lds_read_line<N, N, 0>(A + r * rs, l, v);
+      grad(0, k, v, w);
+      lds_read_line<N, N, 0>(B + r * rs, l, b);
+#pragma unroll
+      for (int i = 0; i < N; ++i) w[i] += b[i];
+      lds_write_line<N, N, 0>(B + r * rs, l, w);
+    }
+    load_coef(dir2(), k);
+  }
+  __syncthreads();
+  if (act) {
+#pragma unroll
+    for (int r = 0; r < NR; ++r) {
+      T v[N], w[N], b[N];
+      lds_read_line<N, N, 2>(A + r * rs, l, v);
+      grad(2, k, v, w);
+      lds_read_line<N, N, 2>(B + r * rs, l, b);
+#pragma unroll
+      for (int i = 0; i < N; ++i) w[i] += b[i];
+      eo_apply<N, 1>(ctab(a.dt).Sb, w, v);
+      lds_write_line<N, N, 2>(A + r * rs, l, v);
+    }
+  }
+  __syncthreads();
+  if (act) {
+#pragma unroll
+    for (int r = 0; r < NR; ++r) {
+      T u[N], v[N];
+      lds_read_line<N, N, 1>(A + r * rs, l, u);
+      eo_apply<N, 1>(ctab(a.dt).Sb, u, v);
+      lds_write_line<N, N, 1>(A + r * rs, l, v);
+    }
+  }
+  __syncthreads();
+  T o[NR][N];
+  if (act) {
+#pragma unroll
+    for (int r = 0; r < NR; ++r) {
+      T u[N];
+      lds_read_line<N, N, 0>(A + r * rs, l, u);
+      eo_apply<N, 1>(ctab(a.dt).Sb, u, o[r]);
+      // x-merge: the first x-plane of cell c+1 is the last one of cell c
+      if (a.color >= 0) B[r * rs + l] = o[r][0];
+    }
+  }
+  if (a.color >= 0) {
+    __syncthreads();
+    cont_store_colored<N, T, NR>(a, o, sA, sB, rs, nr, act, c, l, q.cy, q.cz, q.seg, q.cx0, q.cx_end, dst);
+  } else if (act) {
+    const int Y = q.cy * p + l % N, Z = q.cz * p + l / N;
+    const bool byz = Y == 0 || Z == 0 || Y == a.gy - 1 || Z == a.gz - 1;
+    const long long g0 = ((long long)Z * a.gy + Y) * a.gx + (long long)q.cx * p;
+#pragma unroll
+    for (int r = 0; r < NR; ++r)
+      if (r < nr)
+#pragma unroll
+        for (int i = 0; i < N; ++i) {
+          const int X = q.cx * p + i;
+          if (!(byz || X == 0 || X == a.gx - 1)) atomicAdd(dst + r * a.vstride + g0 + i, o[r][i]);
+        }
   }
 }
 
@@ -511,9 +706,9 @@ __global__ void __launch_bounds__(threads_per_block<N>()) diag_kernel(const Diag
       T u[N], v[N];
 #pragma unroll
       for (int i = 0; i < N; ++i) {
-        T f = (a.load ? a.fval * a.jxw : a.cdiag[d]) * line_weight<N, 0>(a.w, l, i);
-        if (a.coef && !a.load) f *= a.coef[cell * N3 + l * N + i];
-        u[i] = f;
+        // (the coefficient holds the quadrature weight)
+        const T w = a.coef && !a.load ? a.coef[cell * N3 + l * N + i] : line_weight<N, 0>(a.w, l, i);
+        u[i] = (a.load ? a.fval * a.jxw : a.cdiag[d]) * w;
       }
       if (a.load) eo_apply<N, 1>(a.S1b, u, v);
       else if (d == 0) eo_apply<N, 1>(a.G2b, u, v);
@@ -577,6 +772,17 @@ struct CoefGradArgs {
   long long vstride;
 };
 
+// Phases per right-hand side (barrier between): z lines of u and lambda (the
+// next pair's loads are in flight meanwhile), value sweeps in z -> U, Lm; x
+// value sweeps; y value sweeps, y derivatives; x and z derivatives.  Each
+// thread sums the products of its own lines in registers over all right-hand
+// sides, one accumulator line per direction; they meet in LDS once at the end,
+// where the quadrature weight is applied.  What bounds it: VALU issue and LDS.
+// 14 LDS accesses per point and pair and 4 barriers, where accumulating in LDS
+// direction by direction took 21 and 7, and one product per point and
+// direction instead of four.  Measured, before -> after: p = 8 24^3, 8 pairs,
+// FP32 360 -> 231 us, FP64 585 -> 451 us; p = 2 80x70x75, 8 pairs, FP64 449 -> 265
+// us; p = 4 40x37x42, 3 pairs, FP32 123 -> 77 us.
 template <int N, typename T>
 __global__ void __launch_bounds__(threads_per_block<N>()) coef_grad_kernel(const CoefGradArgs<N, T> a)
 {
@@ -584,82 +790,100 @@ __global__ void __launch_bounds__(threads_per_block<N>()) coef_grad_kernel(const
   constexpr int N2 = N * N, N3 = N * N * N, p = N - 1;
   __shared__ T sU[CB * N3];
   __shared__ T sL[CB * N3];
-  __shared__ T sG[CB * N3];
   const int t = threadIdx.x, c = t / N2, l = t % N2;
-  const long long cell = (long long)blockIdx.x * CB + c;
-  const bool act = c < CB && cell < a.ncells;
+  const unsigned cell0 = blockIdx.x * (unsigned)CB;
+  const bool act = c < CB && cell0 + c < a.ncells;
   T *U = sU + (act ? c : 0) * N3;
   T *Lm = sL + (act ? c : 0) * N3;
-  T *G = sG + (act ? c : 0) * N3;
-  const int cx = act ? (int)(cell % a.nx) : 0;
-  const long long rr0 = act ? cell / a.nx : 0;
-  const int cy = (int)(rr0 % a.ny), cz = (int)(rr0 / a.ny);
+  CellXYZ q = traverse_xyz(cell0, a.nx, a.ny, a.nz, 0);
+  if (q.x + c < (unsigned)a.nx) q.x += c;
+  else q = traverse_xyz(act ? cell0 + c : cell0, a.nx, a.ny, a.nz, 0);
+  const int X = (int)q.x * p + l % N, Y = (int)q.y * p + l / N, Z0 = (int)q.z * p;
+  const bool bxy = !act || X == 0 || Y == 0 || X == a.gx - 1 || Y == a.gy - 1;
+  const long long plane = (long long)a.gy * a.gx, g0 = (long long)Z0 * plane + (long long)Y * a.gx + X;
+  T u[N], w[N];
+  auto load = [&](int r) {
+#pragma unroll
+    for (int k = 0; k < N; ++k) {
+      const bool bd = bxy || Z0 + k == 0 || Z0 + k == a.gz - 1;
+      const long long g = r * a.vstride + g0 + k * plane;
+      u[k] = bd ? T(0) : a.u[g];
+      w[k] = bd ? T(0) : a.lam[g];
+    }
+  };
+  T ax[N], ay[N], az[N];
+#pragma unroll
+  for (int i = 0; i < N; ++i) ax[i] = ay[i] = az[i] = T(0);
+  auto add = [&](const T(&x)[N], const T(&y)[N], T(&acc)[N]) {
+    T gx[N], gy[N];
+    eo_apply<N, -1>(ctab(a.dt).Df, x, gx);
+    eo_apply<N, -1>(ctab(a.dt).Df, y, gy);
+#pragma unroll
+    for (int i = 0; i < N; ++i) acc[i] = gx[i] * gy[i] + acc[i];
+  };
+  load(0);
   for (int r = 0; r < a.nrhs; ++r) {
     if (act) {
-      T u[N], v[N], w[N], z[N];
-#pragma unroll
-      for (int k = 0; k < N; ++k) {
-        const int X = cx * p + l % N, Y = cy * p + l / N, Z = cz * p + k;
-        const bool bd = X == 0 || Y == 0 || Z == 0 || X == a.gx - 1 || Y == a.gy - 1 || Z == a.gz - 1;
-        const long long g = ((long long)Z * a.gy + Y) * a.gx + X + r * a.vstride;
-        u[k] = bd ? T(0) : a.u[g];
-        w[k] = bd ? T(0) : a.lam[g];
-      }
+      T v[N], z[N];
       eo_apply<N, 1>(ctab(a.dt).Sf, u, v);
       eo_apply<N, 1>(ctab(a.dt).Sf, w, z);
       lds_write_line<N, N, 2>(U, l, v);
       lds_write_line<N, N, 2>(Lm, l, z);
     }
     __syncthreads();
+    if (r + 1 < a.nrhs) load(r + 1);
     if (act) {
-      T u[N], v[N];
-      lds_read_line<N, N, 0>(U, l, u);
-      eo_apply<N, 1>(ctab(a.dt).Sf, u, v);
+      T x[N], v[N];
+      lds_read_line<N, N, 0>(U, l, x);
+      eo_apply<N, 1>(ctab(a.dt).Sf, x, v);
       lds_write_line<N, N, 0>(U, l, v);
-      lds_read_line<N, N, 0>(Lm, l, u);
-      eo_apply<N, 1>(ctab(a.dt).Sf, u, v);
+      lds_read_line<N, N, 0>(Lm, l, x);
+      eo_apply<N, 1>(ctab(a.dt).Sf, x, v);
       lds_write_line<N, N, 0>(Lm, l, v);
     }
     __syncthreads();
     if (act) {
-      T u[N], v[N];
-      lds_read_line<N, N, 1>(U, l, u);
-      eo_apply<N, 1>(ctab(a.dt).Sf, u, v);
+      T x[N], v[N], z[N];
+      lds_read_line<N, N, 1>(U, l, x);
+      eo_apply<N, 1>(ctab(a.dt).Sf, x, v);
       lds_write_line<N, N, 1>(U, l, v);
-      lds_read_line<N, N, 1>(Lm, l, u);
-      eo_apply<N, 1>(ctab(a.dt).Sf, u, v);
-      lds_write_line<N, N, 1>(Lm, l, v);
+      lds_read_line<N, N, 1>(Lm, l, x);
+      eo_apply<N, 1>(ctab(a.dt).Sf, x, z);
+      lds_write_line<N, N, 1>(Lm, l, z);
+      add(v, z, ay);
     }
     __syncthreads();
-    auto dir_term = [&](auto dirc, bool first) {
-      constexpr int DIR = decltype(dirc)::value;
-      T u[N], w[N], gu[N], gw[N], acc[N];
-      lds_read_line<N, N, DIR>(U, l, u);
-      lds_read_line<N, N, DIR>(Lm, l, w);
-      eo_apply<N, -1>(ctab(a.dt).Df, u, gu);
-      eo_apply<N, -1>(ctab(a.dt).Df, w, gw);
-      if (first) {
-#pragma unroll
-        for (int i = 0; i < N; ++i) acc[i] = T(0);
-      } else {
-        lds_read_line<N, N, DIR>(G, l, acc);
-      }
-#pragma unroll
-      for (int i = 0; i < N; ++i) acc[i] += a.cdiag[DIR] * line_weight<N, DIR>(ctab(a.dt).w, l, i) * gu[i] * gw[i];
-      lds_write_line<N, N, DIR>(G, l, acc);
-    };
-    if (act) dir_term(std::integral_constant<int, 0>(), r == 0);
-    __syncthreads();
-    if (act) dir_term(std::integral_constant<int, 1>(), false);
-    __syncthreads();
-    if (act) dir_term(std::integral_constant<int, 2>(), false);
+    if (act) {
+      T x[N], y[N];
+      lds_read_line<N, N, 0>(U, l, x);
+      lds_read_line<N, N, 0>(Lm, l, y);
+      add(x, y, ax);
+      lds_read_line<N, N, 2>(U, l, x);
+      lds_read_line<N, N, 2>(Lm, l, y);
+      add(x, y, az);
+    }
     __syncthreads();
   }
   if (act) {
-    T v[N];
-    lds_read_line<N, N, 0>(G, l, v);
 #pragma unroll
-    for (int i = 0; i < N; ++i) a.grad[cell * N3 + l * N + i] = v[i];
+    for (int i = 0; i < N; ++i) ax[i] *= a.cdiag[0];
+    lds_write_line<N, N, 0>(U, l, ax);
+  }
+  __syncthreads();
+  if (act) {
+    T v[N];
+    lds_read_line<N, N, 1>(U, l, v);
+#pragma unroll
+    for (int i = 0; i < N; ++i) v[i] = a.cdiag[1] * ay[i] + v[i];
+    lds_write_line<N, N, 1>(U, l, v);
+  }
+  __syncthreads();
+  if (act) {
+    T v[N];
+    lds_read_line<N, N, 2>(U, l, v);
+    T *out = a.grad + (long long)(cell0 + c) * N3 + l;
+#pragma unroll
+    for (int k = 0; k < N; ++k) out[k * N2] = (a.cdiag[2] * az[k] + v[k]) * line_weight<N, 2>(ctab(a.dt).w, l, k);
   }
 }
 
@@ -737,23 +961,32 @@ static hipError_t launch_cell_n(const CellLaunch &L, hipStream_t stream)
   const size_t lds = size_t(CB) * (2 * N3 + (L.mode == 2 ? 12 * N * N : 0)) * sizeof(T);
   const unsigned blocks = (unsigned)((L.ncells + CB - 1) / CB);
   const dim3 grid(blocks, L.nrhs), block(((CB * N * N + 63) / 64) * 64);
-  auto launch = [&](auto kern, dim3 g) {
-    const hipError_t e = allow_dynamic_lds((const void *)kern, lds);
+  auto launch = [&](auto kern, dim3 g, size_t bytes) {
+    const hipError_t e = allow_dynamic_lds((const void *)kern, bytes);
     if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(kern, g, block, lds, stream, a);
+    hipLaunchKernelGGL(kern, g, block, bytes, stream, a);
     return hipGetLastError();
   };
   if (L.mode == 0) {
     return launch(L.coef ? cell_kernel<N, T, Mode::Local, false, false, true>
-                         : cell_kernel<N, T, Mode::Local, false, false, false>, grid);
+                         : cell_kernel<N, T, Mode::Local, false, false, false>, grid, lds);
   } else if (L.mode == 1) {
-    auto kern = L.coef ? cell_kernel<N, T, Mode::Cont, false, false, true>
+    // two right-hand sides per workgroup at low degrees, where their shared
+    // index arithmetic and coefficient outweigh the halved number of resident
+    // workgroups (8 right-hand sides, p = 2 80x70x75 FP32: 370 -> 297 us, p = 4
+    // 40x37x42 156 -> 150 us, p = 8 24^3 462 -> 493 us; FP64 p = 1 227 -> 184 us,
+    // p = 3 50x52x55 263 -> 290 us)
+    constexpr int NR2 = N <= (std::is_same<T, float>::value ? 5 : 2) ? 2 : 1;
+    const bool two = L.coef && L.nrhs > 1 && NR2 == 2;
+    auto kern = L.coef ? (two ? cont_coef_kernel<N, T, NR2> : cont_coef_kernel<N, T, 1>)
                        : cell_kernel<N, T, Mode::Cont, false, false, false>;
+    const size_t klds = two ? 2 * lds : lds;
+    const unsigned ny = two ? (L.nrhs + 1) / 2 : L.nrhs;
     if (!cont_colored(L, CB)) {
       a.color = -1;
       const hipError_t e = vec_fill(std::is_same<T, float>::value, L.dst, L.vstride * L.nrhs, 0., stream);
       if (e != hipSuccess) return e;
-      return launch(kern, grid);
+      return launch(kern, dim3(blocks, ny), klds);
     }
     a.nseg = (a.nx + CB - 1) / CB;
     // colours in ascending order: the first unit to touch a node stores it
@@ -765,18 +998,18 @@ static hipError_t launch_cell_n(const CellLaunch &L, hipStream_t stream)
       a.nrz = (a.nz - pz + 1) / 2;
       const long long nb = (long long)a.nss * a.nry * a.nrz;
       if (nb == 0) continue;
-      const hipError_t e = launch(kern, dim3((unsigned)nb, L.nrhs));
+      const hipError_t e = launch(kern, dim3((unsigned)nb, ny), klds);
       if (e != hipSuccess) return e;
     }
     return hipSuccess;
   }
   if (L.refx)
     return launch(L.cheby ? cell_kernel<N, T, Mode::DG, true, true, false> : cell_kernel<N, T, Mode::DG, false, true, false>,
-                  grid);
+                  grid, lds);
   // (up to degree 8 the operator runs as a sum of Kronecker products)
   if constexpr (N - 1 > kMaxDegreeTp)
     return launch(L.cheby ? cell_kernel<N, T, Mode::DG, true, false, false> : cell_kernel<N, T, Mode::DG, false, false, false>,
-                  grid);
+                  grid, lds);
   else return hipErrorInvalidValue;
 }
 

@@ -163,6 +163,10 @@ struct CoefGradLaunch {
   const void *dtab = nullptr;
 };
 hipError_t launch_coef_gradient(const CoefGradLaunch &L, hipStream_t stream);
+// y = x times the quadrature weight, [cell][q] device arrays (dtab: the
+// operator's 1D tables)
+hipError_t weight_qdata(int n, bool fp32, const void *dtab, const void *x, void *y, long long count,
+                        hipStream_t stream);
 
 // sine-deformed mesh metric (cell and face), computed on the device
 hipError_t launch_sine_metric(const Tables1D &t, bool fp32, const int nc[3], double amp,

@@ -387,6 +387,59 @@ hipError_t layout_convert(int degree, const int nc[3], int lanes, const double *
   return hipGetLastError();
 }
 
+// y = x w_q: bound by memory; kWeightRounds coalesced values per thread, the
+// position in the cell of a workgroup's first value is uniform and the threads'
+// follow by 32-bit arithmetic.  Takes the place of a device copy when a
+// coefficient is set and saves every later apply one multiplication per q-point
+// (Q8 24^3: FP32 15.8 us, the copy 12.2 us; FP64 24.6 us, the copy 23.1 us).
+constexpr int kWeightRounds = 8;
+template <int N, typename T>
+__global__ void __launch_bounds__(kThreads) weight_kernel(const DevTab<N, T> *dt, const T *x, T *y, long long n)
+{
+  constexpr unsigned N3 = N * N * N;
+  const auto &w = ctab(dt).w;
+  __shared__ T sw[N];
+  if (threadIdx.x < N) sw[threadIdx.x] = w[threadIdx.x];
+  __syncthreads();
+  const long long i0 = blockIdx.x * (long long)(kThreads * kWeightRounds);
+  const unsigned q0 = (unsigned)(i0 % N3);
+  T v[kWeightRounds];
+#pragma unroll
+  for (int r = 0; r < kWeightRounds; ++r) {
+    const long long i = i0 + r * kThreads + threadIdx.x;
+    if (i < n) v[r] = x[i];
+  }
+#pragma unroll
+  for (int r = 0; r < kWeightRounds; ++r) {
+    const long long i = i0 + r * kThreads + threadIdx.x;
+    const unsigned q = (q0 + r * kThreads + threadIdx.x) % N3;
+    if (i < n) y[i] = v[r] * (sw[q % N] * (sw[q / N % N] * sw[q / (N * N)]));
+  }
+}
+
+hipError_t weight_qdata(int n, bool fp32, const void *dtab, const void *x, void *y, long long count, hipStream_t s)
+{
+  const long long blocks = (count + kThreads * kWeightRounds - 1) / (kThreads * kWeightRounds);
+  if (blocks <= 0 || blocks > 0x7fffffffLL) return hipErrorInvalidValue;
+  const unsigned g = (unsigned)blocks;
+  switch (n) {
+#define SFK_CASE(NN)                                                                                             \
+  case NN:                                                                                                       \
+    if (fp32)                                                                                                    \
+      hipLaunchKernelGGL((weight_kernel<NN, float>), dim3(g), dim3(kThreads), 0, s,                              \
+                         (const DevTab<NN, float> *)dtab, (const float *)x, (float *)y, count);                  \
+    else                                                                                                         \
+      hipLaunchKernelGGL((weight_kernel<NN, double>), dim3(g), dim3(kThreads), 0, s,                             \
+                         (const DevTab<NN, double> *)dtab, (const double *)x, (double *)y, count);               \
+    break;
+    SFK_CASE(2) SFK_CASE(3) SFK_CASE(4) SFK_CASE(5) SFK_CASE(6) SFK_CASE(7) SFK_CASE(8) SFK_CASE(9) \
+    SFK_CASE(10) SFK_CASE(11) SFK_CASE(12) SFK_CASE(13) SFK_CASE(14) SFK_CASE(15) SFK_CASE(16)
+#undef SFK_CASE
+  default: return hipErrorInvalidValue;
+  }
+  return hipGetLastError();
+}
+
 template <int N, typename T>
 static hipError_t upload_devtab(const Tables1D &t, void **dev)
 {
