@@ -12,7 +12,24 @@
 // kind 3  velocity gradient of mu^T L(a) u with mu = M^{-1} lambda:
 //         cell: (d mu/dx_d) u JxW at every q-point; face (upper face of each
 //         cell, normal velocity b = a.n):  -(mu^- - mu^+) u_upwind JxW_f.
-// Thread/phase organisation as in sfk_cell_kernels.hip.
+// One thread per line of N points of a cell (N^2 threads), cells_per_block
+// cells in a workgroup, the cell's values in LDS between the sweeps.
+//
+// What bounds it: the stored velocity and the vectors at large sizes, and for
+// N <= 4 as much the vector unit's issue slots (N = 4, FP32, 47x51x45 cells:
+// 693 vector instructions a thread were 30 of 41 us).  So no quadrature weight
+// is multiplied in the kernels: in the collocation space of the Gauss points
+// the tangential weights of every term cancel against those of W^{-1}, and what
+// is left (w_j / w_i, the cell size, the lifting l_i(0) / w_i of the face
+// fluxes) is folded into the 1D matrices on the host, one per direction; the
+// inverse mass matrix is one 1D matrix per direction instead of two.  The sweeps
+// end so that the first and the last run on the z lines that are loaded and
+// stored (consecutive dofs across lanes), and the y derivative starts from the
+// registers of the y value sweep: 7 phases instead of 10.  Measured, before ->
+// after: apply FP64 p = 3 48^3 62.7 -> 55.7 us (5.7 TB/s, as a large copy), p = 7
+// 24x25x26 74 -> 62, FP32 p = 3 47x51x45 29.3 -> 27.5; transpose FP64 p = 3 90 ->
+// 83; LSRK stage FP64 p = 3 95 -> 79, p = 8 22x21x20 104 -> 81; velocity gradient
+// FP64 p = 3 108 -> 74, FP32 51 -> 39.
 #include "sfk_device.h"
 #include "sfk_kernels.h"
 
@@ -24,23 +41,100 @@ constexpr int adv_cells_per_block()
   return 256 / (N * N) > 0 ? 256 / (N * N) : 1;
 }
 constexpr int kAdvMaxThreads = 256;
+
+// LDS values per cell: two blocks (A, B) and the six face layers, or one block
+template <int N, typename T, int KIND>
+constexpr int adv_lds_values()
+{
+  return KIND == 2 ? CellLds<N, T>::CS : 2 * CellLds<N, T>::CS + 6 * N * N;
+}
 template <int N, typename T, int KIND>
 constexpr int adv_waves()
 {
   constexpr int cb = adv_cells_per_block<N>();
-  return lds_waves_per_simd(cb * (2 * CellLds<N, T>::CS + (KIND == 2 ? 0 : 6 * N * N)) * (int)sizeof(T), cb * N * N);
+  return lds_waves_per_simd(cb * adv_lds_values<N, T, KIND>() * (int)sizeof(T), cb * N * N);
+}
+
+// face lifting of one direction, l_i(0) f0 + l_i(1) f1 at point i by parity:
+// e[i] (f0 + f1) + o[i] (f0 - f1), the mirrored point with - o[i]
+template <int N, typename T>
+struct AdvLift {
+  T e[(N + 1) / 2], o[(N + 1) / 2];
+};
+
+// 1D matrices of an advection operator, weights and cell size folded in
+template <int N, typename T>
+struct AdvTab {
+  Eo<N, T> Sf;       // GLL values -> Gauss points
+  Eo<N, T> If;       // Gauss points -> GLL values (inverse of Sf)
+  Eo<N, T> Sw;       // S^T W: Gauss points -> test functions
+  Eo<N, T> Mi, Mij;  // S^{-1} W^{-1} S^{-T}, and that divided by JxW's cell part
+  Eo<N, T> Dw[3];    // ij W^{-1} D^T W (forward)
+  Eo<N, T> Da[3];    // ij jxw D (adjoint)
+  Eo<N, T> Dg[3];    // ij jxw W D (velocity gradient)
+  AdvLift<N, T> tr;  // traces: v0, v1 = sum of l_i(0), l_i(1) times the values
+  AdvLift<N, T> Lw[3], La[3]; // -1/2 ij W^{-1} l, and that times jxw
+  T w[N];            // Gauss weights
+};
+
+template <int N, typename T>
+static AdvTab<N, T> make_advtab(const Tables1D &t, const double ij[3])
+{
+  AdvTab<N, T> a{};
+  // products in extended precision: one rounding per entry
+  using R = long double;
+  const R jxw = 1 / (R(ij[0]) * ij[1] * ij[2]);
+  const std::vector<R> w(t.weights.begin(), t.weights.end());
+  std::vector<double> m(N * N);
+  auto eo = [&](bool forward, auto entry) {
+    for (int i = 0; i < N; ++i)
+      for (int q = 0; q < N; ++q) m[i * N + q] = (double)entry(i, q);
+    return make_eo<N, T>(m, forward);
+  };
+  auto lift = [&](auto l0) { // l0(i): the factor of f0; that of f1 mirrors it
+    AdvLift<N, T> L{};
+    for (int i = 0; i < (N + 1) / 2; ++i) {
+      L.e[i] = T((l0(i) + l0(N - 1 - i)) / 2);
+      L.o[i] = T((l0(i) - l0(N - 1 - i)) / 2);
+    }
+    return L;
+  };
+  auto minv = [&](int i, int q) {
+    R v = 0;
+    for (int k = 0; k < N; ++k) v += (R)t.Sinv[k * N + i] * t.Sinv[k * N + q] / w[k];
+    return v;
+  };
+  a.Sf = make_eo<N, T>(t.S, true);
+  a.If = make_eo<N, T>(t.Sinv, true);
+  a.Sw = eo(false, [&](int i, int q) { return t.S[i * N + q] * w[q]; });
+  a.Mi = eo(true, minv);
+  a.Mij = eo(true, [&](int i, int q) { return minv(i, q) / jxw; });
+  a.tr = lift([&](int i) { return t.fv0[i]; });
+  for (int d = 0; d < 3; ++d) {
+    a.Dw[d] = eo(false, [&](int i, int q) { return ij[d] * (t.D[i * N + q] * w[q] / w[i]); });
+    a.Da[d] = eo(true, [&](int i, int q) { return ij[d] * jxw * t.D[i * N + q]; });
+    a.Dg[d] = eo(true, [&](int i, int q) { return ij[d] * jxw * (t.D[i * N + q] * w[q]); });
+    a.Lw[d] = lift([&](int i) { return -(R)ij[d] * (t.fv0[i] / w[i]) / 2; });
+    a.La[d] = lift([&](int i) { return -ij[d] * jxw * (t.fv0[i] / w[i]) / 2; });
+  }
+  for (int i = 0; i < N; ++i) a.w[i] = T(w[i]);
+  return a;
+}
+
+template <int N, typename T>
+__device__ __forceinline__ const SFK_CONST_AS AdvTab<N, T> &atab(const AdvTab<N, T> *p)
+{
+  return *(const SFK_CONST_AS AdvTab<N, T> *)opaque_ptr(p);
 }
 
 template <int N, typename T>
 struct AdvArgs {
-  const DevTab<N, T> *dt; // tables in device memory (read through ctab)
+  const AdvTab<N, T> *dt; // tables in device memory (read through atab)
   const T *src, *upd, *aux;
   T *dst, *tm, *dst2;
   T c_np, c_tm;
   const T *cell_vel, *face_vel;
   T vel[3];
-  T ij[3];
-  T jxw;
   T jxwf[3];
   long long ncells;
   int nx, ny, nz;
@@ -48,110 +142,183 @@ struct AdvArgs {
   int order; // block order (logical_block)
 };
 
-// normal velocity a.n (outward from the cell) at face point fa of face (d, s)
-// (the lower face's value is stored with the lower neighbour `lower`)
-template <int N, typename T, bool VAR>
-__device__ __forceinline__ T normal_velocity(const AdvArgs<N, T> &a, long long cell, int lower, int d, int s, int fa)
-{
-  constexpr int N2 = N * N;
-  if constexpr (!VAR) {
-    return s ? a.vel[d] : -a.vel[d];
-  } else {
-    if (s) return a.face_vel[((long long)d * a.ncells + cell) * N2 + fa];
-    return -a.face_vel[((long long)d * a.ncells + lower) * N2 + fa];
-  }
-}
-
-template <int N, int DIR, typename T, bool VAR>
-__device__ __forceinline__ T cell_velocity(const AdvArgs<N, T> &a, long long cell, int l, int i)
-{
-  if constexpr (!VAR) return a.vel[DIR];
-  else {
-    constexpr int N3 = N * N * N;
-    const int dof = line_base<N, N, DIR>(l) + i * line_stride<N, N, DIR>();
-    return a.cell_vel[(cell * 3 + DIR) * N3 + dof];
-  }
-}
-
-// value face layers of the 6 neighbours (GLL nodal: the face layer is the
-// trace) into this cell's F[f][fa]: thread l loads face point l of every
-// face (six independent loads, issued together)
+// velocity component DIR at the points of line l, and the normal velocities
+// a.n (outward from the cell) on its two ends: the lower face's value is stored
+// with the lower neighbour
 template <int N, typename T>
-__device__ __forceinline__ void load_face_layers(const T *src, T *F, const int (&nbr)[6], int l)
+struct AdvVel {
+  T v[N], n0, n1;
+};
+template <int N, int DIR, typename T, bool VAR>
+__device__ __forceinline__ void load_velocity(const AdvArgs<N, T> &a, long long cell, int lower, int l, AdvVel<N, T> &v)
 {
-  constexpr int N2 = N * N, N3 = N * N * N, p = N - 1;
-  T v[6];
+  if constexpr (VAR) {
+    constexpr int N2 = N * N, N3 = N2 * N;
+    const T *p = a.cell_vel + (cell * 3 + DIR) * N3 + line_base<N, N, DIR>(l);
 #pragma unroll
-  for (int f = 0; f < 6; ++f) {
-    const int d = f / 2, lf = f % 2 ? 0 : p;
-    const int of = d == 0 ? face_dof<N, 0>(lf, l) : (d == 1 ? face_dof<N, 1>(lf, l) : face_dof<N, 2>(lf, l));
-    v[f] = src[(long long)nbr[f] * N3 + of];
+    for (int i = 0; i < N; ++i) v.v[i] = p[i * line_stride<N, N, DIR>()];
+    const T *f = a.face_vel + (long long)DIR * a.ncells * N2 + l;
+    v.n0 = -f[(long long)lower * N2];
+    v.n1 = f[cell * N2];
+  } else {
+#pragma unroll
+    for (int i = 0; i < N; ++i) v.v[i] = a.vel[DIR];
+    v.n0 = -a.vel[DIR];
+    v.n1 = a.vel[DIR];
   }
-#pragma unroll
-  for (int f = 0; f < 6; ++f) F[f * N2 + l] = v[f];
 }
 
+// traces at both ends of a line of Gauss values
+template <int N, typename L, typename T>
+__device__ __forceinline__ void line_traces(const L &tr, const T (&q)[N], T &v0, T &v1)
+{
+  T e = 0, o = 0;
+#pragma unroll
+  for (int i = 0; i < N / 2; ++i) {
+    e += tr.e[i] * (q[i] + q[N - 1 - i]);
+    o += tr.o[i] * (q[i] - q[N - 1 - i]);
+  }
+  if constexpr (N % 2 == 1) e += tr.e[N / 2] * q[N / 2];
+  v0 = e + o;
+  v1 = e - o;
+}
+
+// r = D g plus the lifting of the end values f0, f1 (D odd: eo_apply<N, -1>
+// with the lifting added to its two parity sums)
+template <int N, typename E, typename L, typename T>
+__device__ __forceinline__ void derivative_lift(const E &t, const L &lw, const T (&g)[N], T f0, T f1, T (&r)[N])
+{
+  constexpr int mid = N / 2;
+  const T fs = f0 + f1, fd = f0 - f1;
+  T e[mid], o[mid];
+#pragma unroll
+  for (int k = 0; k < mid; ++k) {
+    e[k] = g[k] + g[N - 1 - k];
+    o[k] = g[k] - g[N - 1 - k];
+  }
+#pragma unroll
+  for (int q = 0; q < mid; ++q) {
+    T p = lw.o[q] * fd, s = lw.e[q] * fs;
+#pragma unroll
+    for (int k = 0; k < mid; ++k) {
+      p += t.A[k][q] * e[k];
+      s += t.B[k][q] * o[k];
+    }
+    if constexpr (N % 2 == 1) p += t.C[q] * g[mid];
+    r[q] = s + p;
+    r[N - 1 - q] = s - p;
+  }
+  if constexpr (N % 2 == 1) {
+    T m = lw.e[mid] * fs;
+#pragma unroll
+    for (int k = 0; k < mid; ++k) m += t.E[k] * o[k];
+    r[mid] = m;
+  }
+}
+
+// r = v r plus the lifting of the end values f0, f1
+template <int N, typename L, typename T>
+__device__ __forceinline__ void scale_lift(const L &lw, const T (&v)[N], T f0, T f1, T (&r)[N])
+{
+  const T fs = f0 + f1, fd = f0 - f1;
+#pragma unroll
+  for (int i = 0; i < N / 2; ++i) {
+    const T s = lw.e[i] * fs;
+    r[i] = v[i] * r[i] + (s + lw.o[i] * fd);
+    r[N - 1 - i] = v[N - 1 - i] * r[N - 1 - i] + (s - lw.o[i] * fd);
+  }
+  if constexpr (N % 2 == 1) r[N / 2] = v[N / 2] * r[N / 2] + lw.e[N / 2] * fs;
+}
+
+// One face layer line per item (6 N of them): the layer of neighbour f that
+// touches this cell (GLL nodal: the layer is the trace), swept in the second
+// tangential direction on its way into F[f][fa].  Adjacent items are adjacent
+// in the first, so that their loads share cache lines.
 template <int N, typename T, typename E>
-__device__ __forceinline__ void face_sweep_t(const E &M, T *F, int narr, int l, bool lo)
+__device__ __forceinline__ void face_lines(const E &S, const T *src, T *F, int item, int f, int d, int layer, int nbr)
+{
+  constexpr int N2 = N * N, N3 = N2 * N;
+  const int r = item % N;
+  const T *p = src + (long long)nbr * N3 + (d == 0 ? r * N + layer : (d == 1 ? layer * N + r : layer * N2 + r));
+  const int st = d == 2 ? N : N2;
+  T u[N], v[N];
+#pragma unroll
+  for (int i = 0; i < N; ++i) u[i] = p[i * st];
+  eo_apply<N, 1>(S, u, v);
+#pragma unroll
+  for (int i = 0; i < N; ++i) F[f * N2 + i * N + r] = v[i];
+}
+
+// sweep of the six layers in the first tangential direction
+template <int N, typename T, typename E>
+__device__ __forceinline__ void face_sweep(const E &S, T *F, int l)
+{
+  for (int it = l; it < 6 * N; it += N * N) {
+    T u[N], v[N];
+#pragma unroll
+    for (int i = 0; i < N; ++i) u[i] = F[it * N + i];
+    eo_apply<N, 1>(S, u, v);
+#pragma unroll
+    for (int i = 0; i < N; ++i) F[it * N + i] = v[i];
+  }
+}
+
+// Stores of results that no workgroup of the launch reads: non-temporal where
+// that pays, which is where one store instruction covers whole cache lines, and
+// for the velocity gradients in FP64 always.  Measured, plain -> non-temporal:
+// velocity gradient FP64 p = 3 48^3 105 -> 74 us, p = 4 130 -> 98, p = 6 112 ->
+// 86, FP32 p = 3 42 -> 39, but FP32 p = 1 126 -> 159, p = 6 47 -> 54; stage FP64
+// p = 3 85 -> 79 us, but p = 2 139 -> 197, p = 4 100 -> 109.
+template <int N, typename T>
+constexpr bool adv_nt_grad()
+{
+  return sizeof(T) == 8 || N * N * sizeof(T) % 64 == 0;
+}
+template <int N, typename T>
+constexpr bool adv_nt_stage()
+{
+  return N * N * sizeof(T) % 128 == 0;
+}
+template <bool NT, typename T>
+__device__ __forceinline__ void store_result(T v, T *p)
+{
+  if constexpr (NT) __builtin_nontemporal_store(v, p);
+  else *p = v;
+}
+
+template <int N, int DIR, typename E, typename T>
+__device__ __forceinline__ void sweep_line(const E &M, T *A, int l)
+{
+  T u[N], v[N];
+  cl_read<N, DIR>(A, l, u);
+  eo_apply<N, 1>(M, u, v);
+  cl_write<N, DIR>(A, l, v);
+}
+
+// forward (kind 0) and transposed weak form (kind 1) in direction DIR from the
+// line's Gauss values q
+template <int N, int DIR, bool ADJ, typename Tb, typename T>
+__device__ __forceinline__ void adv_dir(const Tb &tb, const T (&q)[N], const AdvVel<N, T> &v, const T *F, int l,
+                                        T (&r)[N])
 {
   constexpr int N2 = N * N;
-  for (int it = l; it < narr * N; it += N2) {
-    T u[N], v[N];
-    T *fl = F + (it / N) * N2 + (lo ? (it % N) * N : (it % N));
-    const int st = lo ? 1 : N;
-#pragma unroll
-    for (int i = 0; i < N; ++i) u[i] = fl[i * st];
-    eo_apply<N, 1>(M, u, v);
-#pragma unroll
-    for (int i = 0; i < N; ++i) fl[i * st] = v[i];
-  }
-}
-
-// forward (kind 0) and transposed weak form (kind 1): direction phase
-template <int N, int DIR, typename T, bool VAR, bool ADJ>
-__device__ __forceinline__ void adv_dir(const AdvArgs<N, T> &a, const T *Acell, const T *F, int l, long long cell,
-                                        int lower, T (&r)[N])
-{
-  const auto &tb = ctab(a.dt);
-  T q[N];
-  cl_read<N, DIR>(Acell, l, q);
-  const T c = a.ij[DIR] * a.jxw;
+  T v0, v1;
+  line_traces<N>(tb.tr, q, v0, v1);
+  const T d0 = v0 - F[2 * DIR * N2 + l], d1 = v1 - F[(2 * DIR + 1) * N2 + l];
   if constexpr (!ADJ) {
     T g[N];
 #pragma unroll
-    for (int i = 0; i < N; ++i)
-      g[i] = cell_velocity<N, DIR, T, VAR>(a, cell, l, i) * c * (line_weight<N, DIR>(tb.w, l, i) * q[i]);
-    eo_apply<N, -1>(tb.Db, g, r);
+    for (int i = 0; i < N; ++i) g[i] = v.v[i] * q[i];
+    // (u^- + u^+) a.n + |a.n| (u^- - u^+), evaluation_dg_advect.h:403-404 (the
+    // factor -1/2 is in the lifting)
+    const T s0 = v0 + F[2 * DIR * N2 + l], s1 = v1 + F[(2 * DIR + 1) * N2 + l];
+    derivative_lift<N>(tb.Dw[DIR], tb.Lw[DIR], g, s0 * v.n0 + fabs(v.n0) * d0, s1 * v.n1 + fabs(v.n1) * d1, r);
   } else {
-    T g[N];
-    eo_apply<N, -1>(tb.Df, q, g);
-#pragma unroll
-    for (int i = 0; i < N; ++i)
-      r[i] = cell_velocity<N, DIR, T, VAR>(a, cell, l, i) * c * (line_weight<N, DIR>(tb.w, l, i) * g[i]);
+    eo_apply<N, -1>(tb.Da[DIR], q, r);
+    // 2 max(a.n, 0) (y^- - y^+)
+    scale_lift<N>(tb.La[DIR], v.v, (v.n0 > T(0) ? T(2) * v.n0 : T(0)) * d0, (v.n1 > T(0) ? T(2) * v.n1 : T(0)) * d1,
+                  r);
   }
-  constexpr int N2 = N * N;
-  const T wf = tb.w[l % N] * tb.w[l / N] * a.jxwf[DIR];
-  T v0 = 0, v1 = 0;
-#pragma unroll
-  for (int i = 0; i < N; ++i) {
-    v0 += tb.fv0[i] * q[i];
-    v1 += tb.fv1[i] * q[i];
-  }
-  T fl[2];
-#pragma unroll
-  for (int s = 0; s < 2; ++s) {
-    const T um = s ? v1 : v0;
-    const T up = F[(2 * DIR + s) * N2 + l];
-    const T an = normal_velocity<N, T, VAR>(a, cell, lower, DIR, s, l);
-    if constexpr (!ADJ) {
-      // -0.5((u^- + u^+) a.n + |a.n| (u^- - u^+)), evaluation_dg_advect.h:403-404
-      fl[s] = T(-0.5) * ((um + up) * an + fabs(an) * (um - up)) * wf;
-    } else {
-      fl[s] = -(an > T(0) ? an : T(0)) * (um - up) * wf;
-    }
-  }
-#pragma unroll
-  for (int i = 0; i < N; ++i) r[i] += tb.fv0[i] * fl[0] + tb.fv1[i] * fl[1];
 }
 
 template <int N, typename T, int KIND, bool VAR, bool STAGE>
@@ -162,11 +329,9 @@ advect_kernel(const AdvArgs<N, T> a)
   constexpr bool ADJ = KIND == 1;
   const int CB = a.cb;
   // dynamic LDS: A [CB][CS], B [CB][CS] (padded cell blocks), F [CB][6][N2]
-  // (not for M^{-1})
+  // (M^{-1}: A only)
   constexpr int CS = CellLds<N, T>::CS;
   T *sA = dyn_lds<T>();
-  T *sB = sA + CB * CS;
-  T *sF = sB + CB * CS;
   const int t = threadIdx.x, c = t / N2, l = t % N2;
   const long long cell0 = (long long)logical_block(blockIdx.x, gridDim.x, a.order) * CB;
   const bool act = c < CB && cell0 + c < a.ncells;
@@ -174,143 +339,102 @@ advect_kernel(const AdvArgs<N, T> a)
   int nbr[6] = {0, 0, 0, 0, 0, 0};
   const long long cell = act ? locate_cell((unsigned)cell0, (unsigned)c, a.nx, a.ny, a.nz, a.order, nbr) : 0;
   T *A = sA + (act ? c : 0) * CS;
-  T *B = sB + (act ? c : 0) * CS;
-  T *F = sF + (KIND != 2 && act ? c * 6 * N2 : 0);
+  T *B = sA + (CB + (act ? c : 0)) * CS;
+  T *F = sA + 2 * CB * CS + (act ? c : 0) * 6 * N2;
 
   if constexpr (KIND == 2) {
-    // M^{-1} x = Sinv^T W^{-1} Sinv x
     if (act) {
-      const auto &tb = ctab(a.dt);
+      const auto &tb = atab(a.dt);
       T u[N], v[N];
 #pragma unroll
       for (int k = 0; k < N; ++k) u[k] = a.src[cell * N3 + k * N2 + l];
-      eo_apply<N, 1>(tb.Ib, u, v);
+      eo_apply<N, 1>(tb.Mij, u, v);
       cl_write<N, 2>(A, l, v);
     }
     __syncthreads();
-    if (act) {
-      const auto &tb = ctab(a.dt);
-      T u[N], v[N];
-      cl_read<N, 0>(A, l, u);
-      eo_apply<N, 1>(tb.Ib, u, v);
-      cl_write<N, 0>(A, l, v);
-    }
+    if (act) sweep_line<N, 0>(atab(a.dt).Mi, A, l);
+    __syncthreads();
+    if (act) sweep_line<N, 1>(atab(a.dt).Mi, A, l);
     __syncthreads();
     if (act) {
-      const auto &tb = ctab(a.dt);
-      T u[N], v[N];
-      cl_read<N, 1>(A, l, u);
-      eo_apply<N, 1>(tb.Ib, u, v);
-#pragma unroll
-      for (int i = 0; i < N; ++i) v[i] /= a.jxw * line_weight<N, 1>(tb.w, l, i);
-      eo_apply<N, 1>(tb.If, v, u);
-      cl_write<N, 1>(A, l, u);
-    }
-    __syncthreads();
-    if (act) {
-      const auto &tb = ctab(a.dt);
-      T u[N], v[N];
-      cl_read<N, 0>(A, l, u);
-      eo_apply<N, 1>(tb.If, u, v);
-      cl_write<N, 0>(A, l, v);
-    }
-    __syncthreads();
-    if (act) {
-      const auto &tb = ctab(a.dt);
-      T u[N], v[N];
+      T u[N];
       cl_read<N, 2>(A, l, u);
-      eo_apply<N, 1>(tb.If, u, v);
 #pragma unroll
-      for (int k = 0; k < N; ++k) a.dst[cell * N3 + k * N2 + l] = v[k];
+      for (int k = 0; k < N; ++k) a.dst[cell * N3 + k * N2 + l] = u[k];
     }
     return;
   } else if constexpr (KIND == 3) {
     // velocity gradient: A <- u at q-points, B <- mu at q-points,
     // F[0..2] <- u^+ on the upper faces, F[3..5] <- mu^+ on the upper faces
+    T bn[3] = {0, 0, 0}, wl = 0;
     if (act) {
-      const auto &tb = ctab(a.dt);
-      T u[N], v[N];
+      const auto &tb = atab(a.dt);
+      T u[N], m[N], v[N];
 #pragma unroll
       for (int k = 0; k < N; ++k) u[k] = a.src[cell * N3 + k * N2 + l];
-      eo_apply<N, 1>(tb.Sf, u, v);
-      cl_write<N, 2>(A, l, v);
 #pragma unroll
-      for (int k = 0; k < N; ++k) u[k] = a.aux[cell * N3 + k * N2 + l];
-      eo_apply<N, 1>(tb.Sf, u, v);
-      cl_write<N, 2>(B, l, v);
-    }
-    if (act) {
-      T v[6];
-#pragma unroll
-      for (int fi = 0; fi < 6; ++fi) {
-        const int d = fi % 3;
-        const T *vec = fi < 3 ? a.src : a.aux;
-        const int of = d == 0 ? face_dof<N, 0>(0, l) : (d == 1 ? face_dof<N, 1>(0, l) : face_dof<N, 2>(0, l));
-        v[fi] = vec[(long long)nbr[2 * d + 1] * N3 + of];
+      for (int k = 0; k < N; ++k) m[k] = a.aux[cell * N3 + k * N2 + l];
+      for (int it = l; it < 6 * N; it += N2) {
+        const int fi = it / N, d = fi % 3;
+        face_lines<N>(tb.Sf, fi < 3 ? a.src : a.aux, F, it, fi, d, 0, d == 0 ? nbr[1] : (d == 1 ? nbr[3] : nbr[5]));
       }
 #pragma unroll
-      for (int fi = 0; fi < 6; ++fi) F[fi * N2 + l] = v[fi];
+      for (int d = 0; d < 3; ++d) bn[d] = a.face_vel[((long long)d * a.ncells + cell) * N2 + l];
+      wl = a.dt->w[l % N] * a.dt->w[l / N];
+      eo_apply<N, 1>(tb.Sf, u, v);
+      cl_write<N, 2>(A, l, v);
+      eo_apply<N, 1>(tb.Sf, m, v);
+      cl_write<N, 2>(B, l, v);
     }
     __syncthreads();
     if (act) {
-      const auto &tb = ctab(a.dt);
-      T u[N], v[N];
-      cl_read<N, 0>(A, l, u);
-      eo_apply<N, 1>(tb.Sf, u, v);
-      cl_write<N, 0>(A, l, v);
-      cl_read<N, 0>(B, l, u);
-      eo_apply<N, 1>(tb.Sf, u, v);
-      cl_write<N, 0>(B, l, v);
-      face_sweep_t<N, T>(tb.Sf, F, 6, l, true);
-    }
-    __syncthreads();
-    if (act) {
-      const auto &tb = ctab(a.dt);
-      T u[N], v[N];
-      cl_read<N, 1>(A, l, u);
-      eo_apply<N, 1>(tb.Sf, u, v);
-      cl_write<N, 1>(A, l, v);
-      cl_read<N, 1>(B, l, u);
-      eo_apply<N, 1>(tb.Sf, u, v);
-      cl_write<N, 1>(B, l, v);
-      face_sweep_t<N, T>(tb.Sf, F, 6, l, false);
+      const auto &tb = atab(a.dt);
+      sweep_line<N, 0>(tb.Sf, A, l);
+      sweep_line<N, 0>(tb.Sf, B, l);
+      face_sweep<N>(tb.Sf, F, l);
     }
     __syncthreads();
     // cell gradients of line l in direction DIR: the x and y lines go
     // through LDS below, so that every store writes consecutive dofs across
     // lanes (FP64 p3 48^3: 168 -> 151 us)
     T gx[N], gy[N];
+    auto do_dir = [&](auto dirc, const T(&uq)[N], const T(&mq)[N], T(&g)[N]) {
+      constexpr int DIR = decltype(dirc)::value;
+      const auto &tb = atab(a.dt);
+      eo_apply<N, -1>(tb.Dg[DIR], mq, g);
+#pragma unroll
+      for (int i = 0; i < N; ++i) g[i] *= wl * uq[i];
+      T u0, um, m0, mm;
+      line_traces<N>(tb.tr, uq, u0, um);
+      line_traces<N>(tb.tr, mq, m0, mm);
+      const T up = F[DIR * N2 + l], mp = F[(3 + DIR) * N2 + l];
+      const T sg = bn[DIR] > T(0) ? T(1) : (bn[DIR] < T(0) ? T(-1) : T(0));
+      const T uh = T(0.5) * (um + up) + T(0.5) * sg * (um - up);
+      store_result<adv_nt_grad<N, T>()>(-(mm - mp) * uh * (wl * a.jxwf[DIR]),
+                                           a.dst2 + ((long long)DIR * a.ncells + cell) * N2 + l);
+    };
     if (act) {
-      const auto &tb = ctab(a.dt);
-      auto do_dir = [&](auto dirc) {
-        constexpr int DIR = decltype(dirc)::value;
-        T uq[N], mq[N], g[N];
-        cl_read<N, DIR>(A, l, uq);
-        cl_read<N, DIR>(B, l, mq);
-        eo_apply<N, -1>(tb.Df, mq, g);
+      const auto &tb = atab(a.dt);
+      T u[N], uq[N], mq[N];
+      cl_read<N, 1>(A, l, u);
+      eo_apply<N, 1>(tb.Sf, u, uq);
+      cl_write<N, 1>(A, l, uq);
+      cl_read<N, 1>(B, l, u);
+      eo_apply<N, 1>(tb.Sf, u, mq);
+      cl_write<N, 1>(B, l, mq);
+      do_dir(std::integral_constant<int, 1>(), uq, mq, gy);
+    }
+    __syncthreads();
+    if (act) {
+      T uq[N], mq[N], gz[N];
+      cl_read<N, 0>(A, l, uq);
+      cl_read<N, 0>(B, l, mq);
+      do_dir(std::integral_constant<int, 0>(), uq, mq, gx);
+      cl_read<N, 2>(A, l, uq);
+      cl_read<N, 2>(B, l, mq);
+      do_dir(std::integral_constant<int, 2>(), uq, mq, gz);
 #pragma unroll
-        for (int i = 0; i < N; ++i) {
-          const T gi = g[i] * a.ij[DIR] * uq[i] * (a.jxw * line_weight<N, DIR>(tb.w, l, i));
-          if constexpr (DIR == 0) gx[i] = gi;
-          else if constexpr (DIR == 1) gy[i] = gi;
-          else a.dst[(cell * 3 + DIR) * N3 + line_base<N, N, DIR>(l) + i * line_stride<N, N, DIR>()] = gi;
-        }
-        T um = 0, mm = 0;
-#pragma unroll
-        for (int i = 0; i < N; ++i) {
-          um += tb.fv1[i] * uq[i];
-          mm += tb.fv1[i] * mq[i];
-        }
-        const T up = F[DIR * N2 + l], mp = F[(3 + DIR) * N2 + l];
-        const T b = a.face_vel[((long long)DIR * a.ncells + cell) * N2 + l];
-        const T sg = b > T(0) ? T(1) : (b < T(0) ? T(-1) : T(0));
-        const T uh = T(0.5) * (um + up) + T(0.5) * sg * (um - up);
-        a.dst2[((long long)DIR * a.ncells + cell) * N2 + l] =
-            -(mm - mp) * uh * (tb.w[l % N] * tb.w[l / N] * a.jxwf[DIR]);
-      };
-      do_dir(std::integral_constant<int, 0>());
-      do_dir(std::integral_constant<int, 1>());
-      do_dir(std::integral_constant<int, 2>());
+      for (int m = 0; m < N; ++m) store_result<adv_nt_grad<N, T>()>(gz[m], a.dst + (cell * 3 + 2) * N3 + l + m * N2);
     }
     // x and y gradients: written into the cell blocks (their q-point values
     // are no longer needed) and stored as z lines, lane l at dof l + m N^2
@@ -324,111 +448,103 @@ advect_kernel(const AdvArgs<N, T> a)
       T v[N];
       cl_read<N, 2>(A, l, v);
 #pragma unroll
-      for (int m = 0; m < N; ++m) a.dst[(cell * 3 + 0) * N3 + l + m * N2] = v[m];
+      for (int m = 0; m < N; ++m) store_result<adv_nt_grad<N, T>()>(v[m], a.dst + (cell * 3 + 0) * N3 + l + m * N2);
       cl_read<N, 2>(B, l, v);
 #pragma unroll
-      for (int m = 0; m < N; ++m) a.dst[(cell * 3 + 1) * N3 + l + m * N2] = v[m];
+      for (int m = 0; m < N; ++m) store_result<adv_nt_grad<N, T>()>(v[m], a.dst + (cell * 3 + 1) * N3 + l + m * N2);
     }
     return;
   } else {
     // ------------------------------------------------ L: z values + faces
+    // The velocities of a direction are loaded two phases before their use.
+    AdvVel<N, T> vx, vy, vz;
     if (act) {
-      const auto &tb = ctab(a.dt);
+      const auto &tb = atab(a.dt);
       T u[N], v[N];
 #pragma unroll
       for (int k = 0; k < N; ++k) u[k] = a.src[cell * N3 + k * N2 + l];
+      for (int it = l; it < 6 * N; it += N2) {
+        const int f = it / N;
+        const int below = f == 0 ? nbr[0] : (f == 2 ? nbr[2] : nbr[4]);
+        const int above = f == 1 ? nbr[1] : (f == 3 ? nbr[3] : nbr[5]);
+        face_lines<N>(tb.Sf, a.src, F, it, f, f / 2, f % 2 ? 0 : N - 1, f % 2 ? above : below);
+      }
+      load_velocity<N, 1, T, VAR>(a, cell, nbr[2], l, vy);
       eo_apply<N, 1>(tb.Sf, u, v);
       cl_write<N, 2>(A, l, v);
     }
-    if (act) load_face_layers<N, T>(a.src, F, nbr, l);
     __syncthreads();
     if (act) {
-      const auto &tb = ctab(a.dt);
-      T u[N], v[N];
-      cl_read<N, 0>(A, l, u);
-      eo_apply<N, 1>(tb.Sf, u, v);
-      cl_write<N, 0>(A, l, v);
-      face_sweep_t<N, T>(tb.Sf, F, 6, l, true);
+      const auto &tb = atab(a.dt);
+      load_velocity<N, 2, T, VAR>(a, cell, nbr[4], l, vz);
+      sweep_line<N, 0>(tb.Sf, A, l);
+      face_sweep<N>(tb.Sf, F, l);
     }
     __syncthreads();
     if (act) {
-      const auto &tb = ctab(a.dt);
-      T u[N], v[N];
+      const auto &tb = atab(a.dt);
+      T u[N], q[N], r[N];
+      load_velocity<N, 0, T, VAR>(a, cell, nbr[0], l, vx);
       cl_read<N, 1>(A, l, u);
-      eo_apply<N, 1>(tb.Sf, u, v);
-      cl_write<N, 1>(A, l, v);
-      face_sweep_t<N, T>(tb.Sf, F, 6, l, false);
-    }
-    __syncthreads();
-    if (act) {
-      const auto &tb = ctab(a.dt);
-      T r[N];
-      adv_dir<N, 0, T, VAR, ADJ>(a, A, F, l, cell, nbr[0], r);
-      cl_write<N, 0>(B, l, r);
-    }
-    __syncthreads();
-    if (act) {
-      const auto &tb = ctab(a.dt);
-      T r[N], b[N];
-      adv_dir<N, 1, T, VAR, ADJ>(a, A, F, l, cell, nbr[2], r);
-      cl_read<N, 1>(B, l, b);
-#pragma unroll
-      for (int i = 0; i < N; ++i) r[i] += b[i];
+      eo_apply<N, 1>(tb.Sf, u, q);
+      cl_write<N, 1>(A, l, q);
+      adv_dir<N, 1, ADJ>(tb, q, vy, F, l, r);
       cl_write<N, 1>(B, l, r);
     }
     __syncthreads();
     if (act) {
-      const auto &tb = ctab(a.dt);
-      T r[N], b[N], o[N];
-      adv_dir<N, 2, T, VAR, ADJ>(a, A, F, l, cell, nbr[4], r);
+      const auto &tb = atab(a.dt);
+      T q[N], r[N], b[N];
+      cl_read<N, 2>(A, l, q);
+      adv_dir<N, 2, ADJ>(tb, q, vz, F, l, r);
       cl_read<N, 2>(B, l, b);
 #pragma unroll
       for (int i = 0; i < N; ++i) r[i] += b[i];
-      if constexpr (!ADJ) {
-        // inverse mass matrix by collocation, evaluation_dg_advect.h:619-624
+      cl_write<N, 2>(B, l, r);
+    }
+    __syncthreads();
+    // back to the dofs: forward by collocation (evaluation_dg_advect.h:619-624)
+    if (act) {
+      const auto &tb = atab(a.dt);
+      T q[N], r[N], b[N];
+      cl_read<N, 0>(A, l, q);
+      adv_dir<N, 0, ADJ>(tb, q, vx, F, l, r);
+      cl_read<N, 0>(B, l, b);
 #pragma unroll
-        for (int i = 0; i < N; ++i) r[i] /= a.jxw * line_weight<N, 2>(tb.w, l, i);
-        eo_apply<N, 1>(tb.If, r, o);
-      } else {
-        eo_apply<N, 1>(tb.Sb, r, o);
-      }
-      cl_write<N, 2>(A, l, o);
+      for (int i = 0; i < N; ++i) r[i] += b[i];
+      if constexpr (!ADJ) eo_apply<N, 1>(tb.If, r, b);
+      else eo_apply<N, 1>(tb.Sw, r, b);
+      cl_write<N, 0>(B, l, b);
     }
     __syncthreads();
     if (act) {
-      const auto &tb = ctab(a.dt);
-      T u[N], v[N];
-      cl_read<N, 1>(A, l, u);
-      if constexpr (!ADJ) eo_apply<N, 1>(tb.If, u, v);
-      else eo_apply<N, 1>(tb.Sb, u, v);
-      cl_write<N, 1>(A, l, v);
+      const auto &tb = atab(a.dt);
+      if constexpr (!ADJ) sweep_line<N, 1>(tb.If, B, l);
+      else sweep_line<N, 1>(tb.Sw, B, l);
     }
     __syncthreads();
     if (act) {
-      const auto &tb = ctab(a.dt);
+      const auto &tb = atab(a.dt);
       T u[N], o[N];
-      cl_read<N, 0>(A, l, u);
-      if constexpr (!ADJ) eo_apply<N, 1>(tb.If, u, o);
-      else eo_apply<N, 1>(tb.Sb, u, o);
-      cl_write<N, 0>(B, l, o);
-    }
-    // the x lines go back through LDS and leave as z lines: lane l holds
-    // dofs l + m N^2, so every store writes consecutive dofs across lanes
-    __syncthreads();
-    if (act) {
-      T o[N];
-      cl_read<N, 2>(B, l, o);
       const long long g0 = cell * N3 + l;
       if constexpr (STAGE) {
+        T up[N];
+#pragma unroll
+        for (int m = 0; m < N; ++m) up[m] = a.upd[g0 + m * N2];
+        cl_read<N, 2>(B, l, u);
+        eo_apply<N, 1>(tb.If, u, o);
         // evaluation_dg_advect.h:651-667
 #pragma unroll
         for (int m = 0; m < N; ++m) {
           const long long g = g0 + m * N2;
-          const T vnp = a.upd[g] + a.c_np * o[m];
-          a.dst[g] = vnp;
-          if (a.c_tm != T(0)) a.tm[g] = vnp + a.c_tm * o[m];
+          const T vnp = up[m] + a.c_np * o[m];
+          store_result<adv_nt_stage<N, T>()>(vnp, a.dst + g);
+          if (a.c_tm != T(0)) store_result<adv_nt_stage<N, T>()>(vnp + a.c_tm * o[m], a.tm + g);
         }
       } else {
+        cl_read<N, 2>(B, l, u);
+        if constexpr (!ADJ) eo_apply<N, 1>(tb.If, u, o);
+        else eo_apply<N, 1>(tb.Sw, u, o);
         // written once, read by nobody in this launch: non-temporal stores
         // keep L2 for the velocity and neighbour layers other workgroups
         // re-read (forward p = 3, 48^3: 73 -> 60 us on MI355X)
@@ -439,18 +555,17 @@ advect_kernel(const AdvArgs<N, T> a)
   }
 }
 
-
 template <int N, typename T>
 static size_t advect_lds_per_cell_n(bool minv)
 {
-  return size_t(2 * CellLds<N, T>::CS + (minv ? 0 : 6 * N * N)) * sizeof(T);
+  return size_t(minv ? adv_lds_values<N, T, 2>() : adv_lds_values<N, T, 0>()) * sizeof(T);
 }
 
 template <int N, typename T>
 static hipError_t launch_advect_n(const AdvectLaunch &L, hipStream_t s)
 {
   AdvArgs<N, T> a{};
-  a.dt = (const DevTab<N, T> *)L.dtab;
+  a.dt = (const AdvTab<N, T> *)L.dtab;
   a.src = (const T *)L.src;
   a.upd = (const T *)L.upd;
   a.aux = (const T *)L.aux;
@@ -464,10 +579,8 @@ static hipError_t launch_advect_n(const AdvectLaunch &L, hipStream_t s)
   const double jxw = 1. / (L.inv_jac[0] * L.inv_jac[1] * L.inv_jac[2]);
   for (int d = 0; d < 3; ++d) {
     a.vel[d] = T(L.vel[d]);
-    a.ij[d] = T(L.inv_jac[d]);
     a.jxwf[d] = T(jxw * L.inv_jac[d]);
   }
-  a.jxw = T(jxw);
   a.ncells = L.ncells;
   a.nx = L.nc[0];
   a.ny = L.nc[1];
@@ -502,6 +615,30 @@ static hipError_t dispatch_advect(const AdvectLaunch &L, hipStream_t s)
   switch (L.tables->n) {
 #define SFK_CASE(NN) \
   case NN: return launch_advect_n<NN, T>(L, s);
+    SFK_CASE(2) SFK_CASE(3) SFK_CASE(4) SFK_CASE(5) SFK_CASE(6) SFK_CASE(7) SFK_CASE(8) SFK_CASE(9) \
+    SFK_CASE(10) SFK_CASE(11) SFK_CASE(12) SFK_CASE(13) SFK_CASE(14) SFK_CASE(15) SFK_CASE(16)
+#undef SFK_CASE
+  default: return hipErrorInvalidValue;
+  }
+}
+
+template <int N, typename T>
+static hipError_t upload_advtab(const Tables1D &t, const double ij[3], void **dev)
+{
+  const AdvTab<N, T> h = make_advtab<N, T>(t, ij);
+  const hipError_t e = hipMalloc(dev, sizeof(h));
+  if (e != hipSuccess) {
+    *dev = nullptr;
+    return e;
+  }
+  return hipMemcpy(*dev, &h, sizeof(h), hipMemcpyHostToDevice);
+}
+
+hipError_t upload_advect_tables(const Tables1D &t, const double ij[3], bool fp32, void **dev)
+{
+  switch (t.n) {
+#define SFK_CASE(NN) \
+  case NN: return fp32 ? upload_advtab<NN, float>(t, ij, dev) : upload_advtab<NN, double>(t, ij, dev);
     SFK_CASE(2) SFK_CASE(3) SFK_CASE(4) SFK_CASE(5) SFK_CASE(6) SFK_CASE(7) SFK_CASE(8) SFK_CASE(9) \
     SFK_CASE(10) SFK_CASE(11) SFK_CASE(12) SFK_CASE(13) SFK_CASE(14) SFK_CASE(15) SFK_CASE(16)
 #undef SFK_CASE

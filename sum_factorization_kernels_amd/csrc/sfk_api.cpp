@@ -116,6 +116,8 @@ sfk_status ensure_device_tables(sfk_op *op)
   if (!op->dtab)
     e = op->d.kind == SFK_DG_PRECOMP || sipg_kron(op)
             ? upload_precomp(op, &op->dtab)
+        : op->d.kind == SFK_DG_ADVECT
+            ? upload_advect_tables(op->tab, op->d.inv_jac, op->d.precision == SFK_FP32, &op->dtab)
             : upload_device_tables(op->tab, op->d.precision == SFK_FP32, &op->dtab);
   if (e == hipSuccess && has_tp(op) && !op->tptab)
     e = upload_tp_tables(op->tab, op->d.inv_jac, op->d.precision == SFK_FP32, &op->tptab);

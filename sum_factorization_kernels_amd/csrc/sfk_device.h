@@ -322,9 +322,9 @@ __device__ __forceinline__ CellXYZ traverse_xyz(unsigned q, unsigned nx, unsigne
 
 // Cell c of a workgroup whose first position q0 is the same for all its
 // threads: q0's coordinates are uniform (scalar unit), and position q0 + c
-// of both traversals is q0's cell moved c steps in x unless that crosses
-// the end of the x row (then the divisions are done per thread).  Returns
-// the cell index; its periodic face neighbours go to nbr (as
+// of both traversals is q0's cell moved c steps in x, or where that crosses the
+// end of the x row, in the traversal's next row (rows shorter than c: the
+// divisions are done per thread).  Returns the cell index; its periodic face neighbours go to nbr (as
 // periodic_neighbors).
 __device__ __forceinline__ long long locate_cell(unsigned q0, unsigned c, int nx, int ny, int nz, int order,
                                                  int (&nbr)[6])
@@ -332,7 +332,18 @@ __device__ __forceinline__ long long locate_cell(unsigned q0, unsigned c, int nx
   const unsigned unx = (unsigned)nx, uny = (unsigned)ny, unz = (unsigned)nz;
   CellXYZ p = traverse_xyz(q0, unx, uny, unz, order);
   if (p.x + c < unx) p.x += c;
-  else p = traverse_xyz(q0 + c, unx, uny, unz, order);
+  else if (p.x + c - unx < unx) {
+    p.x += c - unx;
+    if (order != 2) {
+      if (++p.y == uny) p.y = 0, ++p.z;
+    } else {
+      const unsigned z0 = p.z / kSlab * kSlab;
+      if (++p.z == unz || p.z == z0 + kSlab) {
+        p.z = z0;
+        if (++p.y == uny) p.y = 0, p.z = z0 + kSlab;
+      }
+    }
+  } else p = traverse_xyz(q0 + c, unx, uny, unz, order);
   const int sy = nx, sz = nx * ny;
   const int ci = ((int)p.z * ny + (int)p.y) * nx + (int)p.x;
   nbr[0] = ci + (p.x == 0 ? nx - 1 : -1);

@@ -119,11 +119,13 @@ struct AdvectLaunch {
   int nc[3] = {1, 1, 1};
   double inv_jac[3] = {1., 1., 1.};
   int cb = 0, order = 1; // schedule
-  const void *dtab = nullptr;
+  const void *dtab = nullptr; // upload_advect_tables
 };
 hipError_t launch_advect(const AdvectLaunch &L, hipStream_t stream);
 // LDS bytes per cell of launch_advect's operator kernels (n points per direction)
 size_t advect_lds_per_cell(int n, bool fp32);
+// the advection operator's 1D matrices (AdvTab<n, T>) in a new device allocation
+hipError_t upload_advect_tables(const Tables1D &t, const double ij[3], bool fp32, void **dev);
 
 // DG Laplacian with precomputed 1D matrices (PrecomputedDGLaplacian)
 struct PrecompLaunch {
