@@ -167,6 +167,19 @@ sfk_status sfk_grad_velocity(sfk_op *op, const void *u, const void *lambda, void
 sfk_status sfk_grad_coefficient(sfk_op *op, const void *u, const void *lambda, void *grad_k,
                                 void *stream);
 
+/* Forward and reverse pass of the advection operator with a velocity that
+ * lives on the device (layouts, counts and precision of
+ * sfk_op_set_velocity_device), e.g. inside an autodiff graph: each is
+ * sfk_op_set_velocity_device followed by sfk_apply, or by
+ * sfk_apply_transpose(lambda) -> grad_u and sfk_grad_velocity(u, lambda), with
+ * the velocity read once.  The operator holds that velocity afterwards.  The
+ * outputs must not overlap the inputs. */
+sfk_status sfk_advect_forward(sfk_op *op, const void *cell_dev, size_t cell_count, const void *face_dev,
+                              size_t face_count, const void *src, void *dst, void *stream);
+sfk_status sfk_advect_backward(sfk_op *op, const void *cell_dev, size_t cell_count, const void *face_dev,
+                               size_t face_count, const void *u, const void *lambda, void *grad_u,
+                               void *grad_cell, void *grad_face, void *stream);
+
 /* b_i = integral of f phi_i (continuous Laplacian; Dirichlet rows 0) */
 sfk_status sfk_op_rhs_constant(sfk_op *op, double f, void *b, void *stream);
 

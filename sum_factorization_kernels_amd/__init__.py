@@ -90,6 +90,8 @@ def lib():
         L.sfk_op_rhs_constant.argtypes = [_vp, ctypes.c_double, _vp, _vp]
         L.sfk_grad_velocity.argtypes = [_vp, _vp, _vp, _vp, _vp, _vp]
         L.sfk_grad_coefficient.argtypes = [_vp, _vp, _vp, _vp, _vp]
+        L.sfk_advect_forward.argtypes = [_vp, _vp, ctypes.c_size_t, _vp, ctypes.c_size_t, _vp, _vp, _vp]
+        L.sfk_advect_backward.argtypes = [_vp, _vp, ctypes.c_size_t, _vp, ctypes.c_size_t] + [_vp] * 6
         L.sfk_solve_cg_cheby.argtypes = [_vp, _vp, _dp, _dp, ctypes.c_double, ctypes.c_int, ctypes.c_int,
                                          ctypes.c_int, ctypes.POINTER(SolveStats), _vp]
         L.sfk_apply_1d.argtypes = [ctypes.c_int, _dp, ctypes.c_int, ctypes.c_int, _ll, _ll, ctypes.c_int,
@@ -211,6 +213,11 @@ class Operator:
         import torch
         return torch.zeros(self.vector_size * self.n_rhs, dtype=self.dtype, device="cuda")
 
+    def _empty(self, n):
+        """n values that the call in hand writes all of"""
+        import torch
+        return torch.empty(n, dtype=self.dtype, device="cuda")
+
     def set_cell_metric(self, a):
         check(lib().sfk_op_set_cell_metric(self.handle, _np_ptr(a), a.size))
 
@@ -289,6 +296,28 @@ class Operator:
         gf = torch.zeros(3 * self.n_face_q, dtype=self.dtype, device="cuda")
         check(lib().sfk_grad_velocity(self.handle, _dptr(u), _dptr(lam), _dptr(gc), _dptr(gf), _stream(stream)))
         return gc, gf
+
+    def advect_forward(self, u, cell, face, stream=None):
+        """set_velocity_device(cell, face), then apply(u), in one pass over the velocity"""
+        self._check_data(cell, 3 * self.n_cell_q)
+        self._check_data(face, 3 * self.n_face_q)
+        self._check_vec(u)
+        y = self._empty(self.vector_size)
+        check(lib().sfk_advect_forward(self.handle, _dptr(cell), cell.numel(), _dptr(face), face.numel(), _dptr(u),
+                                       _dptr(y), _stream(stream)))
+        return y
+
+    def advect_backward(self, u, lam, cell, face, stream=None):
+        """set_velocity_device(cell, face), then (apply_transpose(lam), *grad_velocity(u, lam)) in one pass over
+        the velocity"""
+        self._check_data(cell, 3 * self.n_cell_q)
+        self._check_data(face, 3 * self.n_face_q)
+        self._check_vec(u)
+        self._check_vec(lam)
+        gu, gc, gf = (self._empty(n) for n in (self.vector_size, 3 * self.n_cell_q, 3 * self.n_face_q))
+        check(lib().sfk_advect_backward(self.handle, _dptr(cell), cell.numel(), _dptr(face), face.numel(), _dptr(u),
+                                        _dptr(lam), _dptr(gu), _dptr(gc), _dptr(gf), _stream(stream)))
+        return gu, gc, gf
 
     @property
     def schedule(self):

@@ -5,7 +5,8 @@ gradients are hand-written HIP kernels (no autodiff of the kernels):
       advection operator with per-point velocity a
       (legacy/include/evaluation_dg_advect.h:285-676 with a variable a);
       backward: u-bar = A^T y-bar (sfk_apply_transpose),
-      a-bar = d(y-bar^T A(a) u)/da (sfk_grad_velocity).
+      a-bar = d(y-bar^T A(a) u)/da (sfk_grad_velocity), both from
+      sfk_advect_backward where both are wanted.
   laplace_coef(u, k, op)   y = A(k) u, -div(k grad u) on the continuous
       Q_p mesh (n_rhs vectors); backward: u-bar = A(k) y-bar (symmetric),
       k-bar = d(y-bar^T A(k) u)/dk (sfk_grad_coefficient).
@@ -18,8 +19,7 @@ import torch
 class _Advect(torch.autograd.Function):
     @staticmethod
     def forward(ctx, u, vel_cell, vel_face, op):
-        op.set_velocity_device(vel_cell, vel_face)
-        y = op.apply(u)
+        y = op.advect_forward(u, vel_cell, vel_face)
         ctx.save_for_backward(u, vel_cell, vel_face)
         ctx.op = op
         return y
@@ -29,11 +29,12 @@ class _Advect(torch.autograd.Function):
         u, vc, vf = ctx.saved_tensors
         op = ctx.op
         gy = gy.contiguous()
+        velocity = ctx.needs_input_grad[1] or ctx.needs_input_grad[2]
+        if ctx.needs_input_grad[0] and velocity:
+            return *op.advect_backward(u, gy, vc, vf), None
         op.set_velocity_device(vc, vf)
         gu = op.apply_transpose(gy) if ctx.needs_input_grad[0] else None
-        gc = gf = None
-        if ctx.needs_input_grad[1] or ctx.needs_input_grad[2]:
-            gc, gf = op.grad_velocity(u, gy)
+        gc, gf = op.grad_velocity(u, gy) if velocity else (None, None)
         return gu, gc, gf, None
 
 

@@ -12,6 +12,10 @@
 // kind 3  velocity gradient of mu^T L(a) u with mu = M^{-1} lambda:
 //         cell: (d mu/dx_d) u JxW at every q-point; face (upper face of each
 //         cell, normal velocity b = a.n):  -(mu^- - mu^+) u_upwind JxW_f.
+// kind 4  kinds 1 and 3 of the same mu in one pass (they share the sweeps and
+//         derivatives of mu), the velocity read from the caller's arrays and
+//         stored into the operator's on the way (set_cell, set_face).
+// kind 5  kind 0 that reads and stores the velocity so.
 // One thread per line of N points of a cell (N^2 threads), cells_per_block
 // cells in a workgroup, the cell's values in LDS between the sweeps.
 //
@@ -42,11 +46,13 @@ constexpr int adv_cells_per_block()
 }
 constexpr int kAdvMaxThreads = 256;
 
-// LDS values per cell: two blocks (A, B) and the six face layers, or one block
+// LDS values per cell: two blocks (A, B) and six face layers; kind 2 one block,
+// kind 4 three blocks and nine layers
 template <int N, typename T, int KIND>
 constexpr int adv_lds_values()
 {
-  return KIND == 2 ? CellLds<N, T>::CS : 2 * CellLds<N, T>::CS + 6 * N * N;
+  if (KIND == 2) return CellLds<N, T>::CS;
+  return KIND == 4 ? 3 * CellLds<N, T>::CS + 9 * N * N : 2 * CellLds<N, T>::CS + 6 * N * N;
 }
 template <int N, typename T, int KIND>
 constexpr int adv_waves()
@@ -134,6 +140,7 @@ struct AdvArgs {
   T *dst, *tm, *dst2;
   T c_np, c_tm;
   const T *cell_vel, *face_vel;
+  T *set_cell, *set_face; // kinds 4 and 5: the velocity read is stored here
   T vel[3];
   T jxwf[3];
   long long ncells;
@@ -165,6 +172,87 @@ __device__ __forceinline__ void load_velocity(const AdvArgs<N, T> &a, long long 
     for (int i = 0; i < N; ++i) v.v[i] = a.vel[DIR];
     v.n0 = -a.vel[DIR];
     v.n1 = a.vel[DIR];
+  }
+}
+
+// Stores of results that no workgroup of the launch reads: non-temporal where
+// that pays, which for the stage is where one store instruction covers whole
+// cache lines, and for the velocity gradients also in FP64 from N = 4 on.
+// Measured, plain -> non-temporal: time step (5 stages) FP64 p = 3 47x51x45 396 ->
+// 374 us, but p = 2 72x70x68 659 -> 788, FP32 p = 4 40x37x42 214 -> 261; velocity
+// gradient repeated into the same arrays FP64 p = 3 48^3 105 -> 74 us, p = 4 130 ->
+// 98, p = 6 112 -> 86, FP32 p = 3 42 -> 39, but p = 1 126 -> 159, p = 6 47 -> 54;
+// within forward, loss and backward pass FP32 p = 3 254 -> 251, but p = 2 399 ->
+// 431, FP64 p = 2 688 -> 721.
+template <int N, typename T>
+constexpr bool adv_nt_grad()
+{
+  return (sizeof(T) == 8 && N >= 4) || N * N * sizeof(T) % 64 == 0;
+}
+template <int N, typename T>
+constexpr bool adv_nt_stage()
+{
+  return N * N * sizeof(T) % 128 == 0;
+}
+template <bool NT, typename T>
+__device__ __forceinline__ void store_result(T v, T *p)
+{
+  if constexpr (NT) __builtin_nontemporal_store(v, p);
+  else *p = v;
+}
+
+// How kinds 4 and 5 store the velocity: for N < 4 as a copy of its own
+// (copy_velocity: a second, contiguous load, non-temporal stores), else from the
+// registers that the lines are computed from.  Forward pass, loss and backward
+// pass, copy / registers: p = 1 90x85x80 FP32 232 / 259 us, FP64 395 / 420; p = 2
+// 72x70x68 FP32 399 / 442, FP64 721 / 746; but p = 3 47x51x45 FP32 264 / 253,
+// FP64 453 / 431; p = 6 28x27x29 FP32 290 / 274, FP64 520 / 474 (p = 4 FP32 303 /
+// 312).  With separate set, apply, transpose and gradient calls p = 3 took 345
+// (FP32) and 617 us.
+template <int N, typename T>
+constexpr bool adv_flat_copy()
+{
+  return N < 4;
+}
+
+template <int N, int DIR, typename T>
+__device__ __forceinline__ void store_velocity(const AdvArgs<N, T> &a, long long cell, int l, const AdvVel<N, T> &v)
+{
+  constexpr int N2 = N * N, N3 = N2 * N;
+  T *p = a.set_cell + (cell * 3 + DIR) * N3 + line_base<N, N, DIR>(l);
+#pragma unroll
+  for (int i = 0; i < N; ++i) p[i * line_stride<N, N, DIR>()] = v.v[i];
+  a.set_face[((long long)DIR * a.ncells + cell) * N2 + l] = v.n1;
+}
+
+// Part of three of the copy of the caller's velocity into the operator's: the
+// workgroup at traversal position cell0 copies the values of CB cells in index
+// order (which for block order 2 need not be the cells it computes), so that
+// loads and stores are contiguous over the workgroup.
+template <int N, typename T>
+struct AdvCopy {
+  T v[N], f;
+};
+template <int N, typename T, bool STORE>
+__device__ __forceinline__ void copy_velocity(const AdvArgs<N, T> &a, long long cell0, int CB, int t, int part,
+                                              AdvCopy<N, T> &c)
+{
+  constexpr int N2 = N * N, N3 = N2 * N;
+  if constexpr (!adv_flat_copy<N, T>()) return;
+  const int nt = CB * N2;
+  if (t >= nt) return;
+  const long long base = cell0 * (3 * N3) + (long long)part * N * nt + t, end = a.ncells * (3 * N3);
+#pragma unroll
+  for (int i = 0; i < N; ++i) {
+    if (base + i * nt < end) {
+      if constexpr (STORE) store_result<true>(c.v[i], a.set_cell + base + i * nt);
+      else c.v[i] = a.cell_vel[base + i * nt];
+    }
+  }
+  const long long fb = cell0 * N2 + t;
+  if (fb < a.ncells * N2) {
+    if constexpr (STORE) store_result<true>(c.f, a.set_face + part * a.ncells * N2 + fb);
+    else c.f = a.face_vel[part * a.ncells * N2 + fb];
   }
 }
 
@@ -249,11 +337,11 @@ __device__ __forceinline__ void face_lines(const E &S, const T *src, T *F, int i
   for (int i = 0; i < N; ++i) F[f * N2 + i * N + r] = v[i];
 }
 
-// sweep of the six layers in the first tangential direction
-template <int N, typename T, typename E>
+// sweep of NF layers in the first tangential direction
+template <int N, int NF, typename T, typename E>
 __device__ __forceinline__ void face_sweep(const E &S, T *F, int l)
 {
-  for (int it = l; it < 6 * N; it += N * N) {
+  for (int it = l; it < NF * N; it += N * N) {
     T u[N], v[N];
 #pragma unroll
     for (int i = 0; i < N; ++i) u[i] = F[it * N + i];
@@ -261,29 +349,6 @@ __device__ __forceinline__ void face_sweep(const E &S, T *F, int l)
 #pragma unroll
     for (int i = 0; i < N; ++i) F[it * N + i] = v[i];
   }
-}
-
-// Stores of results that no workgroup of the launch reads: non-temporal where
-// that pays, which is where one store instruction covers whole cache lines, and
-// for the velocity gradients in FP64 always.  Measured, plain -> non-temporal:
-// velocity gradient FP64 p = 3 48^3 105 -> 74 us, p = 4 130 -> 98, p = 6 112 ->
-// 86, FP32 p = 3 42 -> 39, but FP32 p = 1 126 -> 159, p = 6 47 -> 54; stage FP64
-// p = 3 85 -> 79 us, but p = 2 139 -> 197, p = 4 100 -> 109.
-template <int N, typename T>
-constexpr bool adv_nt_grad()
-{
-  return sizeof(T) == 8 || N * N * sizeof(T) % 64 == 0;
-}
-template <int N, typename T>
-constexpr bool adv_nt_stage()
-{
-  return N * N * sizeof(T) % 128 == 0;
-}
-template <bool NT, typename T>
-__device__ __forceinline__ void store_result(T v, T *p)
-{
-  if constexpr (NT) __builtin_nontemporal_store(v, p);
-  else *p = v;
 }
 
 template <int N, int DIR, typename E, typename T>
@@ -340,7 +405,7 @@ advect_kernel(const AdvArgs<N, T> a)
   const long long cell = act ? locate_cell((unsigned)cell0, (unsigned)c, a.nx, a.ny, a.nz, a.order, nbr) : 0;
   T *A = sA + (act ? c : 0) * CS;
   T *B = sA + (CB + (act ? c : 0)) * CS;
-  T *F = sA + 2 * CB * CS + (act ? c : 0) * 6 * N2;
+  T *F = sA + (KIND == 4 ? 3 : 2) * CB * CS + (act ? c : 0) * (KIND == 4 ? 9 : 6) * N2;
 
   if constexpr (KIND == 2) {
     if (act) {
@@ -391,7 +456,7 @@ advect_kernel(const AdvArgs<N, T> a)
       const auto &tb = atab(a.dt);
       sweep_line<N, 0>(tb.Sf, A, l);
       sweep_line<N, 0>(tb.Sf, B, l);
-      face_sweep<N>(tb.Sf, F, l);
+      face_sweep<N, 6>(tb.Sf, F, l);
     }
     __syncthreads();
     // cell gradients of line l in direction DIR: the x and y lines go
@@ -454,10 +519,135 @@ advect_kernel(const AdvArgs<N, T> a)
       for (int m = 0; m < N; ++m) store_result<adv_nt_grad<N, T>()>(v[m], a.dst + (cell * 3 + 1) * N3 + l + m * N2);
     }
     return;
+  } else if constexpr (KIND == 4) {
+    // A <- u, B <- mu at q-points, C <- the sum of L^T mu, F[0..5] <- mu of the
+    // six neighbours, F[6..8] <- u of the upper ones
+    T *C = sA + (2 * CB + (act ? c : 0)) * CS;
+    AdvVel<N, T> vx, vy, vz;
+    T wl = 0;
+    AdvCopy<N, T> cp;
+    copy_velocity<N, T, false>(a, cell0, CB, t, 0, cp);
+    if (act) {
+      const auto &tb = atab(a.dt);
+      T u[N], m[N], v[N];
+#pragma unroll
+      for (int k = 0; k < N; ++k) m[k] = a.aux[cell * N3 + k * N2 + l];
+#pragma unroll
+      for (int k = 0; k < N; ++k) u[k] = a.src[cell * N3 + k * N2 + l];
+      for (int it = l; it < 9 * N; it += N2) {
+        const int f = it / N, d = f < 6 ? f / 2 : f - 6;
+        const int below = d == 0 ? nbr[0] : (d == 1 ? nbr[2] : nbr[4]);
+        const int above = d == 0 ? nbr[1] : (d == 1 ? nbr[3] : nbr[5]);
+        const bool up = f >= 6 || f % 2;
+        face_lines<N>(tb.Sf, f < 6 ? a.aux : a.src, F, it, f, d, up ? 0 : N - 1, up ? above : below);
+      }
+      load_velocity<N, 1, T, true>(a, cell, nbr[2], l, vy);
+      wl = a.dt->w[l % N] * a.dt->w[l / N];
+      eo_apply<N, 1>(tb.Sf, m, v);
+      cl_write<N, 2>(B, l, v);
+      eo_apply<N, 1>(tb.Sf, u, v);
+      cl_write<N, 2>(A, l, v);
+    }
+    copy_velocity<N, T, true>(a, cell0, CB, t, 0, cp);
+    __syncthreads();
+    copy_velocity<N, T, false>(a, cell0, CB, t, 1, cp);
+    if (act) {
+      const auto &tb = atab(a.dt);
+      load_velocity<N, 2, T, true>(a, cell, nbr[4], l, vz);
+      sweep_line<N, 0>(tb.Sf, A, l);
+      sweep_line<N, 0>(tb.Sf, B, l);
+      face_sweep<N, 9>(tb.Sf, F, l);
+    }
+    copy_velocity<N, T, true>(a, cell0, CB, t, 1, cp);
+    __syncthreads();
+    T gx[N], gy[N];
+    auto do_dir = [&](auto dirc, const T(&uq)[N], const T(&mq)[N], const AdvVel<N, T> &v, T(&g)[N], T(&r)[N]) {
+      constexpr int DIR = decltype(dirc)::value;
+      const auto &tb = atab(a.dt);
+      T u0, u1, m0, m1;
+      line_traces<N>(tb.tr, uq, u0, u1);
+      line_traces<N>(tb.tr, mq, m0, m1);
+      const T d0 = m0 - F[2 * DIR * N2 + l], d1 = m1 - F[(2 * DIR + 1) * N2 + l], up = F[(6 + DIR) * N2 + l];
+      if constexpr (!adv_flat_copy<N, T>()) store_velocity<N, DIR>(a, cell, l, v);
+      eo_apply<N, -1>(tb.Da[DIR], mq, r);
+#pragma unroll
+      for (int i = 0; i < N; ++i) g[i] = r[i] * (uq[i] * (wl * tb.w[i]));
+      const T sg = v.n1 > T(0) ? T(1) : (v.n1 < T(0) ? T(-1) : T(0));
+      const T uh = T(0.5) * (u1 + up) + T(0.5) * sg * (u1 - up);
+      store_result<adv_nt_grad<N, T>()>(-d1 * uh * (wl * a.jxwf[DIR]),
+                                        a.dst2 + ((long long)DIR * a.ncells + cell) * N2 + l);
+      scale_lift<N>(tb.La[DIR], v.v, (v.n0 > T(0) ? T(2) * v.n0 : T(0)) * d0, (v.n1 > T(0) ? T(2) * v.n1 : T(0)) * d1,
+                    r);
+    };
+    copy_velocity<N, T, false>(a, cell0, CB, t, 2, cp);
+    if (act) {
+      const auto &tb = atab(a.dt);
+      T u[N], uq[N], mq[N], r[N];
+      load_velocity<N, 0, T, true>(a, cell, nbr[0], l, vx);
+      cl_read<N, 1>(A, l, u);
+      eo_apply<N, 1>(tb.Sf, u, uq);
+      cl_write<N, 1>(A, l, uq);
+      cl_read<N, 1>(B, l, u);
+      eo_apply<N, 1>(tb.Sf, u, mq);
+      cl_write<N, 1>(B, l, mq);
+      do_dir(std::integral_constant<int, 1>(), uq, mq, vy, gy, r);
+      cl_write<N, 1>(C, l, r);
+    }
+    copy_velocity<N, T, true>(a, cell0, CB, t, 2, cp);
+    __syncthreads();
+    if (act) {
+      T uq[N], mq[N], gz[N], r[N], b[N];
+      cl_read<N, 2>(A, l, uq);
+      cl_read<N, 2>(B, l, mq);
+      do_dir(std::integral_constant<int, 2>(), uq, mq, vz, gz, r);
+#pragma unroll
+      for (int m = 0; m < N; ++m) store_result<adv_nt_grad<N, T>()>(gz[m], a.dst + (cell * 3 + 2) * N3 + l + m * N2);
+      cl_read<N, 2>(C, l, b);
+#pragma unroll
+      for (int i = 0; i < N; ++i) r[i] += b[i];
+      cl_write<N, 2>(C, l, r);
+    }
+    __syncthreads();
+    if (act) {
+      const auto &tb = atab(a.dt);
+      T uq[N], mq[N], r[N], b[N];
+      cl_read<N, 0>(A, l, uq);
+      cl_read<N, 0>(B, l, mq);
+      do_dir(std::integral_constant<int, 0>(), uq, mq, vx, gx, r);
+      cl_read<N, 0>(C, l, b);
+#pragma unroll
+      for (int i = 0; i < N; ++i) r[i] += b[i];
+      eo_apply<N, 1>(tb.Sw, r, b);
+      cl_write<N, 0>(C, l, b);
+    }
+    __syncthreads();
+    // the x and y gradients leave through A and B as z lines (see kind 3)
+    if (act) {
+      cl_write<N, 0>(A, l, gx);
+      cl_write<N, 1>(B, l, gy);
+      sweep_line<N, 1>(atab(a.dt).Sw, C, l);
+    }
+    __syncthreads();
+    if (act) {
+      T v[N], o[N];
+      cl_read<N, 2>(A, l, v);
+#pragma unroll
+      for (int m = 0; m < N; ++m) store_result<adv_nt_grad<N, T>()>(v[m], a.dst + (cell * 3 + 0) * N3 + l + m * N2);
+      cl_read<N, 2>(B, l, v);
+#pragma unroll
+      for (int m = 0; m < N; ++m) store_result<adv_nt_grad<N, T>()>(v[m], a.dst + (cell * 3 + 1) * N3 + l + m * N2);
+      cl_read<N, 2>(C, l, v);
+      eo_apply<N, 1>(atab(a.dt).Sw, v, o);
+#pragma unroll
+      for (int m = 0; m < N; ++m) __builtin_nontemporal_store(o[m], a.tm + cell * N3 + l + m * N2);
+    }
+    return;
   } else {
     // ------------------------------------------------ L: z values + faces
     // The velocities of a direction are loaded two phases before their use.
     AdvVel<N, T> vx, vy, vz;
+    AdvCopy<N, T> cp;
+    if constexpr (KIND == 5) copy_velocity<N, T, false>(a, cell0, CB, t, 0, cp);
     if (act) {
       const auto &tb = atab(a.dt);
       T u[N], v[N];
@@ -473,14 +663,18 @@ advect_kernel(const AdvArgs<N, T> a)
       eo_apply<N, 1>(tb.Sf, u, v);
       cl_write<N, 2>(A, l, v);
     }
+    if constexpr (KIND == 5) copy_velocity<N, T, true>(a, cell0, CB, t, 0, cp);
     __syncthreads();
+    if constexpr (KIND == 5) copy_velocity<N, T, false>(a, cell0, CB, t, 1, cp);
     if (act) {
       const auto &tb = atab(a.dt);
       load_velocity<N, 2, T, VAR>(a, cell, nbr[4], l, vz);
       sweep_line<N, 0>(tb.Sf, A, l);
-      face_sweep<N>(tb.Sf, F, l);
+      face_sweep<N, 6>(tb.Sf, F, l);
     }
+    if constexpr (KIND == 5) copy_velocity<N, T, true>(a, cell0, CB, t, 1, cp);
     __syncthreads();
+    if constexpr (KIND == 5) copy_velocity<N, T, false>(a, cell0, CB, t, 2, cp);
     if (act) {
       const auto &tb = atab(a.dt);
       T u[N], q[N], r[N];
@@ -488,14 +682,17 @@ advect_kernel(const AdvArgs<N, T> a)
       cl_read<N, 1>(A, l, u);
       eo_apply<N, 1>(tb.Sf, u, q);
       cl_write<N, 1>(A, l, q);
+      if constexpr (KIND == 5 && !adv_flat_copy<N, T>()) store_velocity<N, 1>(a, cell, l, vy);
       adv_dir<N, 1, ADJ>(tb, q, vy, F, l, r);
       cl_write<N, 1>(B, l, r);
     }
+    if constexpr (KIND == 5) copy_velocity<N, T, true>(a, cell0, CB, t, 2, cp);
     __syncthreads();
     if (act) {
       const auto &tb = atab(a.dt);
       T q[N], r[N], b[N];
       cl_read<N, 2>(A, l, q);
+      if constexpr (KIND == 5 && !adv_flat_copy<N, T>()) store_velocity<N, 2>(a, cell, l, vz);
       adv_dir<N, 2, ADJ>(tb, q, vz, F, l, r);
       cl_read<N, 2>(B, l, b);
 #pragma unroll
@@ -508,6 +705,7 @@ advect_kernel(const AdvArgs<N, T> a)
       const auto &tb = atab(a.dt);
       T q[N], r[N], b[N];
       cl_read<N, 0>(A, l, q);
+      if constexpr (KIND == 5 && !adv_flat_copy<N, T>()) store_velocity<N, 0>(a, cell, l, vx);
       adv_dir<N, 0, ADJ>(tb, q, vx, F, l, r);
       cl_read<N, 0>(B, l, b);
 #pragma unroll
@@ -556,9 +754,10 @@ advect_kernel(const AdvArgs<N, T> a)
 }
 
 template <int N, typename T>
-static size_t advect_lds_per_cell_n(bool minv)
+static size_t advect_lds_per_cell_n(int kind)
 {
-  return size_t(minv ? adv_lds_values<N, T, 2>() : adv_lds_values<N, T, 0>()) * sizeof(T);
+  return size_t(kind == 2 ? adv_lds_values<N, T, 2>() : kind == 4 ? adv_lds_values<N, T, 4>() : adv_lds_values<N, T, 0>()) *
+         sizeof(T);
 }
 
 template <int N, typename T>
@@ -576,6 +775,8 @@ static hipError_t launch_advect_n(const AdvectLaunch &L, hipStream_t s)
   a.c_tm = T(L.c_tm);
   a.cell_vel = (const T *)L.cell_vel;
   a.face_vel = (const T *)L.face_vel;
+  a.set_cell = (T *)L.set_cell;
+  a.set_face = (T *)L.set_face;
   const double jxw = 1. / (L.inv_jac[0] * L.inv_jac[1] * L.inv_jac[2]);
   for (int d = 0; d < 3; ++d) {
     a.vel[d] = T(L.vel[d]);
@@ -589,7 +790,7 @@ static hipError_t launch_advect_n(const AdvectLaunch &L, hipStream_t s)
   if (CB * N * N > kAdvMaxThreads) return hipErrorInvalidConfiguration;
   a.cb = CB;
   a.order = L.order;
-  const size_t lds = size_t(CB) * advect_lds_per_cell_n<N, T>(L.kind == 2);
+  const size_t lds = size_t(CB) * advect_lds_per_cell_n<N, T>(L.kind);
   const dim3 grid((unsigned)((L.ncells + CB - 1) / CB)), block(((CB * N * N + 63) / 64) * 64);
   const bool var = L.cell_vel != nullptr;
   decltype(&advect_kernel<N, T, 0, false, false>) kern = nullptr;
@@ -601,6 +802,8 @@ static hipError_t launch_advect_n(const AdvectLaunch &L, hipStream_t s)
   case 1: kern = var ? advect_kernel<N, T, 1, true, false> : advect_kernel<N, T, 1, false, false>; break;
   case 2: kern = advect_kernel<N, T, 2, false, false>; break;
   case 3: kern = advect_kernel<N, T, 3, true, false>; break;
+  case 4: kern = advect_kernel<N, T, 4, true, false>; break;
+  case 5: kern = advect_kernel<N, T, 5, true, false>; break;
   default: return hipErrorInvalidValue;
   }
   const hipError_t e = allow_dynamic_lds((const void *)kern, lds);
@@ -650,7 +853,7 @@ size_t advect_lds_per_cell(int n, bool fp32)
 {
   switch (n) {
 #define SFK_CASE(NN) \
-  case NN: return fp32 ? advect_lds_per_cell_n<NN, float>(false) : advect_lds_per_cell_n<NN, double>(false);
+  case NN: return fp32 ? advect_lds_per_cell_n<NN, float>(0) : advect_lds_per_cell_n<NN, double>(0);
     SFK_CASE(2) SFK_CASE(3) SFK_CASE(4) SFK_CASE(5) SFK_CASE(6) SFK_CASE(7) SFK_CASE(8) SFK_CASE(9) \
     SFK_CASE(10) SFK_CASE(11) SFK_CASE(12) SFK_CASE(13) SFK_CASE(14) SFK_CASE(15) SFK_CASE(16)
 #undef SFK_CASE

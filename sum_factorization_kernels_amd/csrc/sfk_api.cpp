@@ -340,19 +340,26 @@ sfk_status sfk_op_set_velocity(sfk_op *op, const double *cell_host, size_t cell_
 }
 
 // device-to-device copy into handle-owned storage (allocated on first use)
-static sfk_status copy_device(sfk_op *op, void **dev, const void *src, size_t count, size_t expected,
-                              const char *what, hipStream_t s)
+static sfk_status ensure_device_copy(sfk_op *op, void **dev, const void *src, size_t count, size_t expected,
+                                     const char *what)
 {
   SFK_REQUIRE(src != nullptr, SFK_ERR_INVALID_ARG, std::string(what) + ": null device pointer");
   SFK_REQUIRE(count == expected, SFK_ERR_INVALID_ARG,
               std::string(what) + ": expected " + std::to_string(expected) + " values, got " + std::to_string(count));
-  const size_t bytes = count * elem_size(op);
-  if (*dev == nullptr && hipMalloc(dev, bytes) != hipSuccess) {
+  if (*dev == nullptr && hipMalloc(dev, count * elem_size(op)) != hipSuccess) {
     *dev = nullptr;
     set_error(std::string(what) + ": hipMalloc failed");
     return SFK_ERR_ALLOC;
   }
-  SFK_CHECK_HIP(hipMemcpyAsync(*dev, src, bytes, hipMemcpyDeviceToDevice, s));
+  return SFK_OK;
+}
+
+static sfk_status copy_device(sfk_op *op, void **dev, const void *src, size_t count, size_t expected,
+                              const char *what, hipStream_t s)
+{
+  const sfk_status st = ensure_device_copy(op, dev, src, count, expected, what);
+  if (st != SFK_OK) return st;
+  SFK_CHECK_HIP(hipMemcpyAsync(*dev, src, count * elem_size(op), hipMemcpyDeviceToDevice, s));
   return SFK_OK;
 }
 
@@ -710,6 +717,71 @@ sfk_status sfk_grad_velocity(sfk_op *op, const void *u, const void *lambda, void
   L.kind = 3;
   L.src = u;
   L.aux = op->scratch;
+  L.dst = grad_cell;
+  L.dst2 = grad_face;
+  SFK_CHECK_HIP(launch_advect(L, s));
+  return SFK_OK;
+}
+
+// the velocity arrays of a call that takes the operator's velocity from the
+// caller: checked, the operator's own allocated, both entered into the launch
+static sfk_status take_velocity(sfk_op *op, const void *cell, size_t cell_count, const void *face, size_t face_count,
+                                AdvectLaunch &L)
+{
+  SFK_REQUIRE(op->d.kind == SFK_DG_ADVECT && (op->d.flags & SFK_FLAG_VARIABLE_VELOCITY), SFK_ERR_INVALID_ARG,
+              "operator lacks SFK_FLAG_VARIABLE_VELOCITY");
+  // both checked and allocated before anything is written: a refused call leaves the velocity as it was
+  sfk_status st = ensure_device_copy(op, &op->face_vel, face, face_count, (size_t)op->nfq * 3, "face velocity");
+  if (st != SFK_OK) return st;
+  st = ensure_device_copy(op, &op->cell_vel, cell, cell_count, (size_t)op->ncq * 3, "cell velocity");
+  if (st != SFK_OK) return st;
+  SFK_ENSURE_TABLES(op);
+  fill_advect_launch(op, L);
+  L.cell_vel = cell;
+  L.face_vel = face;
+  L.set_cell = op->cell_vel;
+  L.set_face = op->face_vel;
+  return SFK_OK;
+}
+
+sfk_status sfk_advect_forward(sfk_op *op, const void *cell_dev, size_t cell_count, const void *face_dev,
+                              size_t face_count, const void *src, void *dst, void *stream)
+{
+  SFK_REQUIRE(op && src && dst, SFK_ERR_INVALID_ARG, "sfk_advect_forward: null argument");
+  SFK_REQUIRE(src != dst, SFK_ERR_INVALID_ARG, "sfk_advect_forward: src and dst must differ");
+  AdvectLaunch L;
+  const sfk_status st = take_velocity(op, cell_dev, cell_count, face_dev, face_count, L);
+  if (st != SFK_OK) return st;
+  L.kind = 5;
+  L.src = src;
+  L.dst = dst;
+  SFK_CHECK_HIP(launch_advect(L, (hipStream_t)stream));
+  return SFK_OK;
+}
+
+sfk_status sfk_advect_backward(sfk_op *op, const void *cell_dev, size_t cell_count, const void *face_dev,
+                               size_t face_count, const void *u, const void *lambda, void *grad_u, void *grad_cell,
+                               void *grad_face, void *stream)
+{
+  SFK_REQUIRE(op && u && lambda && grad_u && grad_cell && grad_face, SFK_ERR_INVALID_ARG,
+              "sfk_advect_backward: null argument");
+  SFK_REQUIRE(grad_u != u && grad_u != lambda, SFK_ERR_INVALID_ARG,
+              "sfk_advect_backward: grad_u must differ from u and lambda");
+  hipStream_t s = (hipStream_t)stream;
+  sfk_status st = ensure_scratch(op, (size_t)op->nvec * elem_size(op));
+  if (st != SFK_OK) return st;
+  AdvectLaunch L;
+  st = take_velocity(op, cell_dev, cell_count, face_dev, face_count, L);
+  if (st != SFK_OK) return st;
+  // mu = M^{-1} lambda once, then L^T mu and mu^T dL/da u from one pass
+  L.kind = 2;
+  L.src = lambda;
+  L.dst = op->scratch;
+  SFK_CHECK_HIP(launch_advect(L, s));
+  L.kind = 4;
+  L.src = u;
+  L.aux = op->scratch;
+  L.tm = grad_u;
   L.dst = grad_cell;
   L.dst2 = grad_face;
   SFK_CHECK_HIP(launch_advect(L, s));

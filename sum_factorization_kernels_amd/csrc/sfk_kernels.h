@@ -108,12 +108,15 @@ hipError_t launch_sipg_general(const SipgLaunch &L, hipStream_t stream);
 struct AdvectLaunch {
   const Tables1D *tables = nullptr;
   bool fp32 = false;
-  int kind = 0; // 0 forward M^{-1}L u, 1 L^T y (adjoint after M^{-1}), 2 M^{-1} x, 3 velocity gradient
+  // 0 forward M^{-1}L u, 1 L^T y (adjoint after M^{-1}), 2 M^{-1} x, 3 velocity gradient, 4 = 1 and 3 of one mu
+  // (src u, aux mu, dst and dst2 the gradients, tm L^T mu), 5 = 0; 4 and 5 store the velocity into set_cell, set_face
+  int kind = 0;
   bool stage = false;
   const void *src = nullptr, *upd = nullptr, *aux = nullptr;
   void *dst = nullptr, *tm = nullptr, *dst2 = nullptr;
   double c_np = 0., c_tm = 0.;
   const void *cell_vel = nullptr, *face_vel = nullptr;
+  void *set_cell = nullptr, *set_face = nullptr;
   double vel[3] = {0., 0., 0.};
   long long ncells = 0;
   int nc[3] = {1, 1, 1};
