@@ -251,14 +251,14 @@ class Operator:
 
     def apply(self, src, dst=None, stream=None):
         self._check_vec(src)
-        dst = self.new_vector() if dst is None else dst
+        dst = self._empty(self.vector_size * self.n_rhs) if dst is None else dst
         self._check_vec(dst)
         check(lib().sfk_apply(self.handle, _dptr(src), _dptr(dst), _stream(stream)))
         return dst
 
     def apply_transpose(self, src, dst=None, stream=None):
         self._check_vec(src)
-        dst = self.new_vector() if dst is None else dst
+        dst = self._empty(self.vector_size * self.n_rhs) if dst is None else dst
         self._check_vec(dst)
         check(lib().sfk_apply_transpose(self.handle, _dptr(src), _dptr(dst), _stream(stream)))
         return dst
@@ -289,11 +289,9 @@ class Operator:
         return b
 
     def grad_velocity(self, u, lam, stream=None):
-        import torch
         self._check_vec(u)
         self._check_vec(lam)
-        gc = torch.zeros(3 * self.n_cell_q, dtype=self.dtype, device="cuda")
-        gf = torch.zeros(3 * self.n_face_q, dtype=self.dtype, device="cuda")
+        gc, gf = self._empty(3 * self.n_cell_q), self._empty(3 * self.n_face_q)
         check(lib().sfk_grad_velocity(self.handle, _dptr(u), _dptr(lam), _dptr(gc), _dptr(gf), _stream(stream)))
         return gc, gf
 
@@ -369,16 +367,15 @@ class Operator:
         """z = P(rhs): the solver's Chebyshev preconditioner (three-term form on
         the tensor-product kernel); equals cheby_sweep from x = 0"""
         self._check_vec(rhs)
-        z, spare = self.new_vector(), self.new_vector()
+        z, spare = (self._empty(self.vector_size * self.n_rhs) for _ in range(2))
         check(lib().sfk_cheby_precondition(self.handle, _dptr(rhs), _dptr(z), _dptr(spare), int(degree),
                                            float(lambda_min), float(lambda_max), _stream(stream)))
         return z
 
     def grad_coefficient(self, u, lam, stream=None):
-        import torch
         self._check_vec(u)
         self._check_vec(lam)
-        g = torch.zeros(self.n_cell_q, dtype=self.dtype, device="cuda")
+        g = self._empty(self.n_cell_q)
         check(lib().sfk_grad_coefficient(self.handle, _dptr(u), _dptr(lam), _dptr(g), _stream(stream)))
         return g
 

@@ -562,11 +562,9 @@ extern "C" sfk_status sfk_cheby_precondition(sfk_op *op, const void *rhs, void *
   }
   sfk_status st = ensure_device_tables(op);
   if (st != SFK_OK) return st;
-  void *zz = z, *sp = spare;
-  hipError_t e = cheby_tp3(op, rhs, &zz, &sp, degree, lambda_min, lambda_max, (hipStream_t)stream);
-  // odd degree: the result is in the spare vector; copy it to z
-  if (e == hipSuccess && zz != z)
-    e = hipMemcpyAsync(z, zz, size_t(op->nvec) * elem_size(op), hipMemcpyDeviceToDevice, (hipStream_t)stream);
+  // an odd degree ends in the other vector than the one it starts with
+  void *zz = degree % 2 ? spare : z, *sp = degree % 2 ? z : spare;
+  const hipError_t e = cheby_tp3(op, rhs, &zz, &sp, degree, lambda_min, lambda_max, (hipStream_t)stream);
   if (e != hipSuccess) {
     set_error(std::string("sfk_cheby_precondition: ") + hipGetErrorString(e));
     return SFK_ERR_HIP;
