@@ -277,7 +277,7 @@ sfk_status sfk_op_destroy(sfk_op *op)
 {
   if (!op) return SFK_OK;
   for (void *p : {op->cell_metric, op->face_metric, op->coef, op->cell_vel, op->face_vel, op->scratch, op->dtab,
-                  op->tptab})
+                  op->tptab, op->solve_ws})
     if (p) (void)hipFree(p);
   delete op;
   return SFK_OK;

@@ -165,7 +165,9 @@ struct TpArgs {
   // the first iterate s_rhs D^{-1} rhs, formed in the kernel from rhs
   // instead of read (CHEBY 3: src points to rhs)
   T s_rhs;
-  double *dot_part;  // CHEBY 5: per-workgroup partial sums of src . dst
+  double *dot_part;  // CHEBY 5: src . dst summed over the grid (grid_sums) into dot_out
+  unsigned *dot_ticket;
+  double *dot_out;
   int nx, ny, nz;    // cells
   int gx, gy, gz;    // nodes
   int ntx, nty;      // tiles per direction
@@ -552,10 +554,13 @@ cont_tp_kernel(const TpArgs<T> a)
     if (threadIdx.x % 64 == 0) red[wave] = v;
     __syncthreads();
     if (threadIdx.x == 0) {
-      double t = 0.;
-      for (int w = 0; w < nw; ++w) t += red[w];
-      a.dot_part[(long long)blockIdx.y * gridDim.x + blockIdx.x] = t;
+      v = 0.;
+      for (int w = 0; w < nw; ++w) v += red[w];
     }
+    double sum[1] = {v};
+    if (grid_sums<1, C::THREADS>(sum, a.dot_part, a.dot_ticket, blockIdx.y * gridDim.x + blockIdx.x,
+                                 gridDim.x * gridDim.y, red))
+      *a.dot_out = sum[0];
   }
 }
 
@@ -661,6 +666,8 @@ static hipError_t launch_tp_shape(const TpLaunch &L, hipStream_t s)
   if (rsrc && rprev) return hipErrorInvalidValue;
   if (rsrc) a.src = (const T *)L.rhs;
   a.dot_part = L.dot_part;
+  a.dot_ticket = L.dot_ticket;
+  a.dot_out = L.dot_out;
   a.s_rhs = T(L.s_rhs);
   a.c_np = T(L.c_np);
   a.c_tm = T(L.c_tm);
@@ -686,7 +693,7 @@ static hipError_t launch_tp_shape(const TpLaunch &L, hipStream_t s)
   // outer matvec)
   decltype(&cont_tp_kernel<N, T, BX, BY, 0>) kdot = nullptr;
   if constexpr (std::is_same<T, double>::value) kdot = cont_tp_kernel<N, T, BX, BY, 5>;
-  if (L.dot_part && (L.cheby != 0 || L.nrhs != 1 || !kdot)) return hipErrorInvalidValue;
+  if (L.dot_part && (L.cheby != 0 || L.nrhs != 1 || !kdot || !L.dot_ticket || !L.dot_out)) return hipErrorInvalidValue;
   auto kern = rsrc ? cont_tp_kernel<N, T, BX, BY, 3>
               : rprev ? cont_tp_kernel<N, T, BX, BY, 4>
               : L.dot_part ? kdot

@@ -63,9 +63,10 @@ struct TpLaunch {
   // (prev_from_rhs) is s_rhs D^{-1} rhs, formed in the kernel (not read)
   bool src_from_rhs = false, prev_from_rhs = false;
   double s_rhs = 0.;
-  // cheby 0, FP64, one right-hand side: also write the workgroups' partial
-  // sums of src . dst here (tp_launch_blocks of them)
-  double *dot_part = nullptr;
+  // cheby 0, FP64, one right-hand side: also src . dst into dot_out (dot_part:
+  // tp_launch_blocks partial sums, dot_ticket: a zero that is left zero)
+  double *dot_part = nullptr, *dot_out = nullptr;
+  unsigned *dot_ticket = nullptr;
   int nc[3] = {1, 1, 1};
   int nrhs = 1;
   long long vstride = 0;
@@ -188,20 +189,23 @@ hipError_t vec_dot(bool fp32, const void *x, const void *y, long long n, double 
 // allocation, T = float or double
 hipError_t upload_device_tables(const Tables1D &t, bool fp32, void **dev);
 
-// result_dev[0] = x.y, result_dev[1] = x.w (FP64 vectors; partials: 2*n_partials)
-// result_dev[0] = sum of count partial sums (of a fused kernel)
-hipError_t vec_sum_partials(const double *partials, long long count, double *result_dev, hipStream_t s);
-hipError_t vec_dot2(const void *x, const void *y, const void *w, long long n, double *result_dev, double *partials,
-                    int n_partials, hipStream_t s);
-// solver kernels (FP64 vectors): x += alpha p (x null: skipped), r -= alpha
-// q, optionally rs = (float) r, result_dev[0] = r.r (an non-null: alpha =
-// *an / *ad, device scalars); and z = (double) zs with result_dev[0] = z.r,
-// result_dev[1] = z.q (partials: 2*n_partials)
-hipError_t vec_cg_update(long long n, double alpha, const double *an, const double *ad, const void *p,
-                         const void *q, void *x, void *r, void *rs, double *result_dev, double *partials,
-                         int n_partials, hipStream_t s);
-hipError_t vec_widen_dot2(long long n, const void *zs, void *z, const void *r, const void *q, double *result_dev,
-                          double *partials, int n_partials, hipStream_t s);
+// solver kernels (FP64 vectors at 16-byte addresses; partials: 512 doubles;
+// ticket: a device zero that is left zero): r -= alpha q with alpha = *zr / *pq (device scalars),
+// optionally rs = (float) r, *rr = r.r, and host[0..2] = *pq, *rr, *zr in pinned
+// memory; and result_dev[0] = z.r, result_dev[1] = z.q (z FP32 when z_fp32)
+hipError_t vec_cg_update(long long n, const double *zr, const double *pq, const void *q, void *r, void *rs,
+                         double *rr, double *host, double *partials, unsigned *ticket, hipStream_t s);
+hipError_t vec_dot2(bool z_fp32, long long n, const void *z, const void *r, const void *q, double *result_dev,
+                    double *partials, unsigned *ticket, hipStream_t s);
+// Lanczos (FP64 vectors; device scalars): v = w / sqrt(*ww)
+// and t = v isq; w *= isq with *alpha = w . v; w -= *alpha v + sqrt(*bb) v0 (bb
+// null: no second term, v0 not read) with *ww = w . w
+hipError_t vec_lanczos_next(long long n, const void *w, const double *ww, const void *isq, void *v, void *t,
+                            hipStream_t s);
+hipError_t vec_lanczos_dot(long long n, void *w, const void *isq, const void *v, double *alpha, double *partials,
+                           unsigned *ticket, hipStream_t s);
+hipError_t vec_lanczos_update(long long n, void *w, const void *v, const void *v0, const double *alpha,
+                              const double *bb, double *ww, double *partials, unsigned *ticket, hipStream_t s);
 hipError_t vec_axpby(bool fp32, long long n, double a, const void *x, double b, void *y, hipStream_t s);
 // z = c a b (elementwise)
 hipError_t vec_mul_scaled(bool fp32, long long n, double c, const void *a, const void *b, void *z, hipStream_t s);

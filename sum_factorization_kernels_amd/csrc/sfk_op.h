@@ -1,6 +1,8 @@
 // The operator handle behind the opaque sfk_op of include/sfk.h.
 #pragma once
 
+#include <mutex>
+
 #include "sfk.h"
 #include "sfk_internal.h"
 #include "sfk_kernels.h"
@@ -36,6 +38,11 @@ struct sfk_op {
   // precomputed DG Laplacian: neighbour coupling constants not both zero
   // (set with the device tables)
   bool pc_couple = true;
+  // sfk_solve_cg_cheby's work space, kept from call to call up to a bound; a
+  // solve that finds it taken by another thread allocates its own
+  void *solve_ws = nullptr;
+  size_t solve_ws_bytes = 0;
+  std::mutex solve_ws_lock;
 };
 
 namespace sfk {

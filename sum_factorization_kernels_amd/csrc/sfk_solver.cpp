@@ -18,6 +18,7 @@
 #include <chrono>
 #include <cstdio>
 #include <cmath>
+#include <cstring>
 #include <string>
 #include <vector>
 
@@ -30,15 +31,66 @@ namespace sfk {
 namespace {
 
 constexpr int kPartials = 2048;
-constexpr int kSlots = 8; // device result slots after the partial sums
+constexpr int kSlots = 8;   // device result slots after the partial sums
+constexpr int kTickets = 3; // and the tickets of the grid sums, a slot each
 constexpr double kChebyRange = 1000.; // lambda_max / lambda_min of the Chebyshev interval
 
-struct DevBuf {
-  void *p = nullptr;
-  ~DevBuf()
+// Work spaces up to this size stay with the operator between solves (the larger
+// ones are given back, as all were: allocating and freeing 255 MB took 4 of 29
+// ms, Q4 32^3 FP64; both grow with the size like an iteration's time, but large
+// problems also take more iterations)
+constexpr size_t kKeepBytes = size_t(1) << 30;
+
+// one allocation for all work vectors: the operator's, or one of this solve
+struct WorkSpace {
+  sfk_op *op = nullptr;
+  char *own = nullptr, *next = nullptr;
+  bool locked = false;
+  ~WorkSpace()
   {
-    if (p) (void)hipFree(p);
+    if (own) (void)hipFree(own);
+    if (locked) op->solve_ws_lock.unlock();
   }
+  hipError_t get(sfk_op *o, size_t bytes)
+  {
+    op = o;
+    if (bytes <= kKeepBytes) locked = op->solve_ws_lock.try_lock();
+    if (!locked) {
+      const hipError_t e = hipMalloc((void **)&own, bytes);
+      if (e != hipSuccess) own = nullptr;
+      next = own;
+      return e;
+    }
+    if (op->solve_ws_bytes < bytes) {
+      if (op->solve_ws) (void)hipFree(op->solve_ws);
+      op->solve_ws = nullptr;
+      op->solve_ws_bytes = 0;
+      const hipError_t e = hipMalloc(&op->solve_ws, bytes);
+      if (e != hipSuccess) {
+        op->solve_ws = nullptr;
+        return e;
+      }
+      op->solve_ws_bytes = bytes;
+    }
+    next = (char *)op->solve_ws;
+    return hipSuccess;
+  }
+  static size_t padded(size_t bytes) { return (bytes + 255) / 256 * 256; }
+  void *take(size_t bytes)
+  {
+    void *p = next;
+    next += padded(bytes);
+    return p;
+  }
+};
+struct Vec {
+  void *p = nullptr;
+};
+// waits for the stream when the solver returns, before its buffers go (or are
+// handed to the next solve)
+struct StreamGuard {
+  hipStream_t s;
+  ~StreamGuard() { (void)hipStreamSynchronize(s); }
 };
 struct PinnedBuf {
   void *p = nullptr;
@@ -57,12 +109,6 @@ __global__ void inv_diag_kernel(const double *d, double *inv, float *inv32, doub
     if (inv32) inv32[i] = (float)iv;
     isq[i] = v != 0. ? 1. / sqrt(v) : 0.;
   }
-}
-
-__global__ void scale_kernel(const double *a, const double *b, double *c, long long n)
-{
-  for (long long i = blockIdx.x * (long long)blockDim.x + threadIdx.x; i < n; i += (long long)gridDim.x * blockDim.x)
-    c[i] = a[i] * b[i];
 }
 
 // deterministic start vector for Lanczos (interior only: the inverse
@@ -108,13 +154,42 @@ double tridiag_max_eig(const std::vector<double> &al, const std::vector<double> 
   return hi;
 }
 
+// The scalars of an iteration are stored into pinned memory by the kernel that
+// forms them; the host waits until none of them is this NaN any more, or until
+// the stream has nothing left to do (an event after the kernel held up the next
+// one by 6 us).
+double not_yet()
+{
+  const unsigned long long bits = 0x7ff8f00df00df00dull;
+  double v;
+  std::memcpy(&v, &bits, sizeof v);
+  return v;
+}
+hipError_t wait_scalars(const volatile double *h, hipStream_t s)
+{
+  const double mark = not_yet();
+  auto there = [&] {
+    for (int i = 0; i < 3; ++i) {
+      const double v = h[i];
+      if (std::memcmp(&v, &mark, sizeof v) == 0) return false;
+    }
+    return true;
+  };
+  for (unsigned k = 1;; ++k) {
+    if (there()) return hipSuccess;
+    if (k % 1024 == 0) {
+      const hipError_t e = hipStreamQuery(s);
+      if (e != hipErrorNotReady) return e;
+    }
+  }
+}
+
 struct Solver {
   sfk_op *op, *sm;
   hipStream_t s;
   long long n;
   bool fp32;
   double *partials = nullptr, *dres = nullptr;
-  double *hres = nullptr; // pinned host copy of the result slots
   sfk_solve_stats st{};
 
   sfk_status dot(bool f32, const void *x, const void *y, double &out)
@@ -127,57 +202,6 @@ struct Solver {
       return SFK_ERR_HIP;
     }
     if (!std::isfinite(out)) {
-      set_error("solver: non-finite inner product");
-      return SFK_ERR_NONFINITE;
-    }
-    return SFK_OK;
-  }
-
-  // read back `count` sums that a fused kernel left in dres
-  sfk_status results(double *out, int count)
-  {
-    hipError_t e = hipMemcpyAsync(out, dres, count * sizeof(double), hipMemcpyDeviceToHost, s);
-    if (e == hipSuccess) e = hipStreamSynchronize(s);
-    if (e != hipSuccess) {
-      set_error(std::string("solver: ") + hipGetErrorString(e));
-      return SFK_ERR_HIP;
-    }
-    for (int i = 0; i < count; ++i)
-      if (!std::isfinite(out[i])) {
-        set_error("solver: non-finite inner product");
-        return SFK_ERR_NONFINITE;
-      }
-    return SFK_OK;
-  }
-
-  // read back `count` result slots (no finiteness check: the caller checks
-  // the slots it uses)
-  sfk_status read_slots(double *out, int count)
-  {
-    hipError_t e = hipMemcpyAsync(hres, dres, count * sizeof(double), hipMemcpyDeviceToHost, s);
-    if (e == hipSuccess) e = hipStreamSynchronize(s);
-    if (e != hipSuccess) {
-      set_error(std::string("solver: ") + hipGetErrorString(e));
-      return SFK_ERR_HIP;
-    }
-    for (int i = 0; i < count; ++i) out[i] = hres[i];
-    return SFK_OK;
-  }
-
-  // (x . y, x . w) in one pass, FP64 vectors
-  sfk_status dot2(const void *x, const void *y, const void *w, double &xy, double &xw)
-  {
-    hipError_t e = vec_dot2(x, y, w, n, dres, partials, kPartials, s);
-    double h[2] = {0., 0.};
-    if (e == hipSuccess) e = hipMemcpyAsync(h, dres, 2 * sizeof(double), hipMemcpyDeviceToHost, s);
-    if (e == hipSuccess) e = hipStreamSynchronize(s);
-    if (e != hipSuccess) {
-      set_error(std::string("solver: ") + hipGetErrorString(e));
-      return SFK_ERR_HIP;
-    }
-    xy = h[0];
-    xw = h[1];
-    if (!std::isfinite(xy) || !std::isfinite(xw)) {
       set_error("solver: non-finite inner product");
       return SFK_ERR_NONFINITE;
     }
@@ -266,9 +290,9 @@ extern "C" sfk_status sfk_solve_cg_cheby(sfk_op *op, sfk_op *smoother_op, const 
   const long long n = S.n;
   const bool f32 = S.fp32;
   const size_t n8 = (size_t)n * 8, ns = (size_t)n * (f32 ? 4 : 8);
-  // device work space: FP64 vectors, and smoother-precision vectors
-  DevBuf red, d64, inv64, isq, r, w, lv0, lv1, lw, lt, e64;
-  DevBuf rs, zs, qs, tms, inv_s;
+  // FP64 vectors, and smoother-precision vectors
+  Vec d64, inv64, isq, r, w, lv0, lv1, lw, lt, e64;
+  Vec rs, zs, qs, tms, inv_s;
   // the outer matvec on the tensor-product kernel also sums p . q (its
   // workgroups' partial sums, one per workgroup).  It runs on the schedule
   // tuned for the operator's fused Chebyshev launches: like them it holds
@@ -281,24 +305,25 @@ extern "C" sfk_status sfk_solve_cg_cheby(sfk_op *op, sfk_op *smoother_op, const 
     fill_tp_launch(op, T, true);
     if (tp_launch_blocks(T) > n_red) n_red = tp_launch_blocks(T);
   }
-  SOLVER_HIP(hipMalloc(&red.p, sizeof(double) * (n_red + kSlots)));
-  S.partials = (double *)red.p;
+  const int n_lan = 2 * lanczos_steps + 1;
+  const size_t n_scalars = n_red + kSlots + kTickets + n_lan;
+  WorkSpace ws;
+  const size_t ws_bytes = 10 * WorkSpace::padded(n8) + 5 * WorkSpace::padded(ns) + WorkSpace::padded(8 * n_scalars);
+  SOLVER_HIP(ws.get(op, ws_bytes));
+  for (Vec *v : {&d64, &inv64, &isq, &r, &w, &lv0, &lv1, &lw, &lt, &e64}) v->p = ws.take(n8);
+  for (Vec *v : {&rs, &zs, &qs, &tms, &inv_s}) v->p = ws.take(ns);
+  S.partials = (double *)ws.take(8 * n_scalars);
   S.dres = S.partials + n_red; // after the partial sums: the result slots
-  SOLVER_HIP(vec_fill(false, S.dres, kSlots, 0., (hipStream_t)stream));
-  PinnedBuf hres;
-  SOLVER_HIP(hipHostMalloc(&hres.p, sizeof(double) * kSlots));
-  S.hres = (double *)hres.p;
-  for (DevBuf *bb : {&d64, &inv64, &isq, &r, &w, &lv0, &lv1, &lw, &lt, &e64})
-    SOLVER_HIP(hipMalloc(&bb->p, n8));
-  for (DevBuf *bb : {&rs, &zs, &qs, &tms, &inv_s})
-    SOLVER_HIP(hipMalloc(&bb->p, ns));
+  auto ticket = [&](int i) { return reinterpret_cast<unsigned *>(S.dres + kSlots + i); };
+  double *lan = S.dres + kSlots + kTickets; // Lanczos: |w_0|^2, then alpha and |w|^2 of each step
+  PinnedBuf hres;                           // p.q, r.r and z.r of an iteration
+  SOLVER_HIP(hipHostMalloc(&hres.p, sizeof(double) * 3));
+  volatile double *h = (volatile double *)hres.p;
   const hipStream_t s = S.s;
-  // every work vector starts at 0 (a fresh allocation may hold NaN bit
-  // patterns, and 0 * NaN would poison the first Chebyshev step)
-  for (DevBuf *bb : {&d64, &inv64, &isq, &r, &w, &lv0, &lv1, &lw, &lt, &e64})
-    SOLVER_HIP(vec_fill(false, bb->p, n, 0., s));
-  for (DevBuf *bb : {&rs, &zs, &qs, &tms, &inv_s})
-    SOLVER_HIP(vec_fill(f32, bb->p, n, 0., s));
+  const StreamGuard guard{s};
+  // everything starts at 0 (the work space may hold NaN bit patterns, and
+  // 0 * NaN would poison the first Chebyshev step)
+  SOLVER_HIP(vec_fill(false, d64.p, (long long)(ws_bytes / 8), 0., s));
   // point-Jacobi diagonal (FP64), inverse in both precisions
   SOLVER_ST(sfk_compute_diagonal(op, d64.p, stream));
   hipLaunchKernelGGL(inv_diag_kernel, dim3(grid_of(n)), dim3(256), 0, s, (const double *)d64.p, (double *)inv64.p,
@@ -306,33 +331,36 @@ extern "C" sfk_status sfk_solve_cg_cheby(sfk_op *op, sfk_op *smoother_op, const 
   SOLVER_HIP(hipGetLastError());
   const void *inv_sm = f32 ? inv_s.p : inv64.p;
 
-  // ---- Lanczos on D^{-1/2} A D^{-1/2} (FP64)
+  // ---- Lanczos on D^{-1/2} A D^{-1/2} (FP64).  All steps are launched with
+  // their scalars on the device and read back at the end; steps after one with
+  // beta = 0 produce values that are not used.
   hipLaunchKernelGGL(start_vector_kernel, dim3(grid_of(n)), dim3(256), 0, s, (const double *)isq.p,
-                     (double *)lv1.p, n);
-  double nrm2;
-  SOLVER_ST(S.dot(false, lv1.p, lv1.p, nrm2));
-  SOLVER_HIP(vec_axpby(false, n, 0., lv1.p, 1. / std::sqrt(nrm2), lv1.p, s));
-  SOLVER_HIP(vec_fill(false, lv0.p, n, 0., s));
-  std::vector<double> al, be;
-  double beta = 0.;
+                     (double *)lw.p, n);
+  SOLVER_HIP(vec_dot(false, lw.p, lw.p, n, lan, S.partials, kPartials, s));
   for (int k = 0; k < lanczos_steps; ++k) {
-    hipLaunchKernelGGL(scale_kernel, dim3(grid_of(n)), dim3(256), 0, s, (const double *)lv1.p, (const double *)isq.p,
-                       (double *)lt.p, n);
+    // v_k = w / |w| over v_{k-2}, A's argument, w = D^{-1/2} A D^{-1/2} v_k and alpha = w . v_k
+    SOLVER_HIP(vec_lanczos_next(n, lw.p, lan + 2 * k, isq.p, lv1.p, lt.p, s));
     SOLVER_ST(sfk_apply(op, lt.p, lw.p, stream));
-    hipLaunchKernelGGL(scale_kernel, dim3(grid_of(n)), dim3(256), 0, s, (const double *)lw.p, (const double *)isq.p,
-                       (double *)lw.p, n);
+    SOLVER_HIP(vec_lanczos_dot(n, lw.p, isq.p, lv1.p, lan + 2 * k + 1, S.partials, ticket(0), s));
+    // w -= alpha v_k + beta v_{k-1}, |w|^2
+    SOLVER_HIP(vec_lanczos_update(n, lw.p, lv1.p, lv0.p, lan + 2 * k + 1, k > 0 ? lan + 2 * k : nullptr,
+                                  lan + 2 * k + 2, S.partials, ticket(1), s));
+    std::swap(lv0.p, lv1.p);
+  }
+  std::vector<double> al, be, hl(n_lan);
+  SOLVER_HIP(hipMemcpyAsync(hl.data(), lan, 8 * n_lan, hipMemcpyDeviceToHost, s));
+  SOLVER_HIP(hipStreamSynchronize(s));
+  for (int k = 0; k < lanczos_steps; ++k) {
+    const double alpha = hl[2 * k + 1], nrm2 = hl[2 * k + 2];
     ++S.st.matvecs_outer;
-    double alpha;
-    SOLVER_ST(S.dot(false, lw.p, lv1.p, alpha));
-    SOLVER_HIP(vec_axpby(false, n, -alpha, lv1.p, 1., lw.p, s));
-    SOLVER_HIP(vec_axpby(false, n, -beta, lv0.p, 1., lw.p, s));
+    if (!std::isfinite(hl[2 * k]) || !std::isfinite(alpha) || !std::isfinite(nrm2)) {
+      set_error("solver: non-finite inner product");
+      return SFK_ERR_NONFINITE;
+    }
     al.push_back(alpha);
-    SOLVER_ST(S.dot(false, lw.p, lw.p, nrm2));
-    beta = std::sqrt(nrm2);
+    const double beta = std::sqrt(nrm2);
     if (k + 1 == lanczos_steps || beta < 1e-14 * std::fabs(alpha)) break;
     be.push_back(beta);
-    std::swap(lv0.p, lv1.p);
-    SOLVER_HIP(vec_axpby(false, n, 1. / beta, lw.p, 0., lv1.p, s));
   }
   const double lmax = 1.1 * tridiag_max_eig(al, be);
   // the polynomial is a preconditioner inside CG, not a multigrid smoother:
@@ -394,6 +422,7 @@ extern "C" sfk_status sfk_solve_cg_cheby(sfk_op *op, sfk_op *smoother_op, const 
   S.st.initial_residual = std::sqrt(rr);
   double res = S.st.initial_residual;
   int iters = 0;
+  bool confirmed = false;
 
   // preconditioner z = P(r): the Chebyshev polynomial on the smoother
   // operator, in the smoother's precision.  FP32: rs already holds (float) r.
@@ -407,7 +436,7 @@ extern "C" sfk_status sfk_solve_cg_cheby(sfk_op *op, sfk_op *smoother_op, const 
       void *z = zs.p, *spare = qs.p;
       SOLVER_ST(cheby(rs.p, &z, &spare));
       if (zrq_dev) {
-        SOLVER_HIP(vec_widen_dot2(n, z, nullptr, r64, qv, zrq_dev, S.partials, kPartials, s));
+        SOLVER_HIP(vec_dot2(true, n, z, r64, qv, zrq_dev, S.partials, ticket(2), s));
         *z64 = nullptr;
         *z32 = z;
         return SFK_OK;
@@ -418,7 +447,7 @@ extern "C" sfk_status sfk_solve_cg_cheby(sfk_op *op, sfk_op *smoother_op, const 
       void *z = e64.p, *spare = zs.p;
       SOLVER_ST(cheby(r64, &z, &spare));
       *z64 = z;
-      if (zrq_dev) SOLVER_HIP(vec_dot2(z, r64, qv, n, zrq_dev, S.partials, kPartials, s));
+      if (zrq_dev) SOLVER_HIP(vec_dot2(false, n, z, r64, qv, zrq_dev, S.partials, ticket(2), s));
     }
     return SFK_OK;
   };
@@ -462,8 +491,9 @@ extern "C" sfk_status sfk_solve_cg_cheby(sfk_op *op, sfk_op *smoother_op, const 
         T.src = pv;
         T.dst = qv;
         T.dot_part = S.partials;
+        T.dot_ticket = ticket(0);
+        T.dot_out = sl;
         SOLVER_HIP(launch_cont_tp(T, s));
-        SOLVER_HIP(vec_sum_partials(S.partials, tp_launch_blocks(T), sl, s));
       } else {
         SOLVER_ST(sfk_apply(op, pv, qv, stream));
         SOLVER_HIP(vec_dot(false, pv, qv, n, sl, S.partials, kPartials, s));
@@ -474,10 +504,18 @@ extern "C" sfk_status sfk_solve_cg_cheby(sfk_op *op, sfk_op *smoother_op, const 
       // the pass that forms the next search direction (which reads p
       // anyway), or done below when the loop may end
       double *zr = zr_slot(iters);
-      SOLVER_HIP(vec_cg_update(n, 0., zr, sl, nullptr, qv, nullptr, r.p, rs32, sl + 1, S.partials, kPartials, s));
-      double h[2 + 4];
-      SOLVER_ST(S.read_slots(h, 6));
-      const double pq = h[0], rz = h[2 + 2 * (iters & 1)];
+      for (int i = 0; i < 3; ++i) h[i] = not_yet();
+      SOLVER_HIP(vec_cg_update(n, zr, sl, qv, r.p, rs32, sl + 1, (double *)hres.p, S.partials, ticket(1), s));
+      // z = P(r); z.r and z.q -> the slots of the next iteration.  Launched
+      // before the scalars are waited for, so that the GPU has work meanwhile
+      // (25 us an iteration); it touches neither x, r nor p, and the last
+      // iteration's is for nothing
+      const void *z32 = nullptr;
+      double *zrq = zr_slot(iters + 1);
+      const auto inner = S.st.matvecs_inner;
+      SOLVER_ST(precond(r.p, qv, &z64, zrq, &z32));
+      SOLVER_HIP(wait_scalars(h, s));
+      const double pq = h[0], rz = h[2];
       rr = h[1];
       if (!std::isfinite(pq) || !std::isfinite(rr) || !std::isfinite(rz)) {
         set_error("solver: non-finite inner product");
@@ -494,19 +532,17 @@ extern "C" sfk_status sfk_solve_cg_cheby(sfk_op *op, sfk_op *smoother_op, const 
       if (res <= target) {
         // the recursively updated residual drifts from b - A x: confirm
         // with the true residual and restart from it if it is not there yet
+        S.st.matvecs_inner = inner; // of the preconditioner that is not used
         SOLVER_ST(sfk_apply(op, x, r.p, stream));
         ++S.st.matvecs_outer;
         SOLVER_HIP(vec_axpby(false, n, 1., b, -1., r.p, s));
         SOLVER_ST(S.dot(false, r.p, r.p, rr));
         res = std::sqrt(rr);
-        if (res <= target) break;
+        confirmed = res <= target;
+        if (confirmed) break;
         SOLVER_ST(restart(iters));
         continue;
       }
-      // z = P(r); z.r and z.q -> the slots of the next iteration
-      const void *z32 = nullptr;
-      double *zrq = zr_slot(iters);
-      SOLVER_ST(precond(r.p, qv, &z64, zrq, &z32));
       const void *zv = z64 ? (const void *)z64 : z32;
       if (iters == max_iter) {
         // the loop ends: x is up to date; p = z + beta p for completeness
@@ -523,12 +559,13 @@ extern "C" sfk_status sfk_solve_cg_cheby(sfk_op *op, sfk_op *smoother_op, const 
       }
     }
   }
-  // final FP64 residual
-  SOLVER_ST(sfk_apply(op, x, r.p, stream));
-  ++S.st.matvecs_outer;
-  SOLVER_HIP(vec_axpby(false, n, 1., b, -1., r.p, s));
-  SOLVER_ST(S.dot(false, r.p, r.p, rr));
-  SOLVER_HIP(hipStreamSynchronize(s));
+  // final FP64 residual (the loop's last check has just formed it where it confirmed convergence)
+  if (!confirmed) {
+    SOLVER_ST(sfk_apply(op, x, r.p, stream));
+    ++S.st.matvecs_outer;
+    SOLVER_HIP(vec_axpby(false, n, 1., b, -1., r.p, s));
+    SOLVER_ST(S.dot(false, r.p, r.p, rr));
+  }
   S.st.final_residual = std::sqrt(rr);
   S.st.iterations = iters;
   S.st.seconds = std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();

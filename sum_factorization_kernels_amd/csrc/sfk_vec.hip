@@ -64,85 +64,172 @@ __global__ void __launch_bounds__(kThreads) dot_final_kernel(const double *parti
   if (threadIdx.x == 0) *result = red[0];
 }
 
-__global__ void __launch_bounds__(kThreads) dot2_partial_kernel(const double *x, const double *y, const double *w,
-                                                                long long n, double *partials)
+// The passes of a CG iteration over r, q, z are bound by memory; each sums its
+// inner products over the grid itself (grid_sums), so that an iteration has no
+// launch for a final sum and no copy of the scalars to the host (Q4 32^3 FP64:
+// five of those took 23 of 212 us).  The tickets of all workgroups meet at one
+// address, 12 ns each (1049 workgroups of 256: r -= alpha q took 22.8 us), so the
+// grid is one workgroup a CU, and every thread has kSumUnroll pairs of each vector
+// in flight.  With 2.1e6 values: the update 13.3 us (before, with the final sum and
+// the copy, 19.5), z.r and z.q 12.7 us (18.8); 256 x 1024 threads with 4 pairs 13.9
+// and 13.8, 512 x 512 with 4 pairs 15.2 and 14.3.
+constexpr int kSumThreads = 512, kSumUnroll = 8, kSumBlocks = 256;
+
+static unsigned sum_grid(long long n)
 {
-  __shared__ double red[2][kThreads];
-  double s = 0., u = 0.;
-  for (long long i = blockIdx.x * (long long)blockDim.x + threadIdx.x; i < n; i += (long long)gridDim.x * blockDim.x) {
-    const double xv = x[i];
-    s += xv * y[i];
-    u += xv * w[i];
-  }
-  red[0][threadIdx.x] = s;
-  red[1][threadIdx.x] = u;
-  __syncthreads();
-  for (int k = kThreads / 2; k > 0; k >>= 1) {
-    if ((int)threadIdx.x < k) {
-      red[0][threadIdx.x] += red[0][threadIdx.x + k];
-      red[1][threadIdx.x] += red[1][threadIdx.x + k];
-    }
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) {
-    partials[blockIdx.x] = red[0][0];
-    partials[gridDim.x + blockIdx.x] = red[1][0];
-  }
+  const long long b = (n + 2 * kSumThreads - 1) / (2 * kSumThreads);
+  return (unsigned)(b < 1 ? 1 : (b < kSumBlocks ? b : kSumBlocks));
 }
 
-// CG update x += alpha p (skipped when x is null), r -= alpha q (FP64),
-// optionally rs = (float) r, with per-block partial sums of r.r; with an
-// non-null, alpha = *an / *ad (device scalars: no host round trip)
-__global__ void __launch_bounds__(kThreads) cg_update_kernel(long long n, double alpha, const double *an,
-                                                             const double *ad, const double *p, const double *q,
-                                                             double *x, double *r, float *rs, double *partials)
+// sum over the workgroup's threads, in thread 0
+__device__ __forceinline__ double block_sum(double t, double *red)
 {
-  __shared__ double red[kThreads];
-  if (an) alpha = *an / *ad;
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) t += __shfl_xor(t, o);
+  __syncthreads();
+  if (threadIdx.x % 64 == 0) red[threadIdx.x / 64] = t;
+  __syncthreads();
+  t = 0.;
+  if (threadIdx.x == 0)
+    for (int w = 0; w < kSumThreads / 64; ++w) t += red[w];
+  __syncthreads();
+  return t;
+}
+
+template <typename T>
+struct Pair {
+  T x, y;
+};
+
+// r -= alpha q, alpha = *zr / *pq (device scalars: no host round trip),
+// optionally rs = (float) r, *rr = r.r; the three scalars also to the host
+__global__ void __launch_bounds__(kSumThreads) cg_update_kernel(long long n, const double *zr, const double *pq,
+                                                                const double *q, double *r, float *rs, double *rr,
+                                                                double *host, double *partials, unsigned *ticket)
+{
+  __shared__ double red[kSumThreads / 64 + 1];
+  const double alpha = *zr / *pq;
+  const long long t = blockIdx.x * (long long)kSumThreads + threadIdx.x, stride = gridDim.x * (long long)kSumThreads;
+  const long long pairs = n / 2;
+  Pair<double> *r2 = reinterpret_cast<Pair<double> *>(r);
+  const Pair<double> *q2 = reinterpret_cast<const Pair<double> *>(q);
+  Pair<float> *rs2 = reinterpret_cast<Pair<float> *>(rs);
   double acc = 0.;
-  for (long long i = blockIdx.x * (long long)blockDim.x + threadIdx.x; i < n; i += (long long)gridDim.x * blockDim.x) {
-    if (x) x[i] += alpha * p[i];
-    const double ri = r[i] - alpha * q[i];
-    r[i] = ri;
-    if (rs) rs[i] = float(ri);
-    acc += ri * ri;
+  for (long long i0 = t; i0 < pairs; i0 += kSumUnroll * stride) {
+    Pair<double> rv[kSumUnroll], qv[kSumUnroll];
+#pragma unroll
+    for (int u = 0; u < kSumUnroll; ++u)
+      if (i0 + u * stride < pairs) rv[u] = r2[i0 + u * stride], qv[u] = q2[i0 + u * stride];
+#pragma unroll
+    for (int u = 0; u < kSumUnroll; ++u) {
+      const long long i = i0 + u * stride;
+      if (i >= pairs) break;
+      rv[u].x -= alpha * qv[u].x;
+      rv[u].y -= alpha * qv[u].y;
+      r2[i] = rv[u];
+      if (rs) rs2[i] = {float(rv[u].x), float(rv[u].y)};
+      acc += rv[u].x * rv[u].x + rv[u].y * rv[u].y;
+    }
   }
-  red[threadIdx.x] = acc;
-  __syncthreads();
-  for (int w = kThreads / 2; w > 0; w >>= 1) {
-    if ((int)threadIdx.x < w) red[threadIdx.x] += red[threadIdx.x + w];
-    __syncthreads();
+  if (n % 2 == 1 && t == 0) {
+    const double v = r[n - 1] - alpha * q[n - 1];
+    r[n - 1] = v;
+    if (rs) rs[n - 1] = float(v);
+    acc += v * v;
   }
-  if (threadIdx.x == 0) partials[blockIdx.x] = red[0];
+  double sum[1] = {block_sum(acc, red)};
+  if (grid_sums<1, kSumThreads>(sum, partials, ticket, blockIdx.x, gridDim.x, red)) {
+    *rr = sum[0];
+    const double h[3] = {*pq, sum[0], *zr};
+    for (int i = 0; i < 3; ++i) __hip_atomic_store(host + i, h[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+  }
 }
 
-// z = (double) zs (not written when z is null) with per-block partial sums
-// of z.r and z.q
-__global__ void __launch_bounds__(kThreads) widen_dot2_kernel(long long n, const float *zs, double *z,
-                                                              const double *r, const double *q, double *partials)
+// z.r and z.q (z FP32 or FP64)
+template <typename Z>
+__global__ void __launch_bounds__(kSumThreads) dot2_kernel(long long n, const Z *z, const double *r, const double *q,
+                                                           double *result, double *partials, unsigned *ticket)
 {
-  __shared__ double red[2][kThreads];
+  __shared__ double red[kSumThreads / 64 + 1];
+  const long long t = blockIdx.x * (long long)kSumThreads + threadIdx.x, stride = gridDim.x * (long long)kSumThreads;
+  const long long pairs = n / 2;
+  const Pair<Z> *z2 = reinterpret_cast<const Pair<Z> *>(z);
+  const Pair<double> *r2 = reinterpret_cast<const Pair<double> *>(r), *q2 = reinterpret_cast<const Pair<double> *>(q);
   double a = 0., b = 0.;
-  for (long long i = blockIdx.x * (long long)blockDim.x + threadIdx.x; i < n; i += (long long)gridDim.x * blockDim.x) {
-    const double zi = double(zs[i]);
-    if (z) z[i] = zi;
-    a += zi * r[i];
-    b += zi * q[i];
-  }
-  red[0][threadIdx.x] = a;
-  red[1][threadIdx.x] = b;
-  __syncthreads();
-  for (int w = kThreads / 2; w > 0; w >>= 1) {
-    if ((int)threadIdx.x < w) {
-      red[0][threadIdx.x] += red[0][threadIdx.x + w];
-      red[1][threadIdx.x] += red[1][threadIdx.x + w];
+  for (long long i0 = t; i0 < pairs; i0 += kSumUnroll * stride) {
+    Pair<Z> zv[kSumUnroll];
+    Pair<double> rv[kSumUnroll], qv[kSumUnroll];
+#pragma unroll
+    for (int u = 0; u < kSumUnroll; ++u) {
+      const long long i = i0 + u * stride;
+      if (i < pairs) zv[u] = z2[i], rv[u] = r2[i], qv[u] = q2[i];
     }
-    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < kSumUnroll; ++u) {
+      if (i0 + u * stride >= pairs) break;
+      a += double(zv[u].x) * rv[u].x + double(zv[u].y) * rv[u].y;
+      b += double(zv[u].x) * qv[u].x + double(zv[u].y) * qv[u].y;
+    }
   }
-  if (threadIdx.x == 0) {
-    partials[blockIdx.x] = red[0][0];
-    partials[gridDim.x + blockIdx.x] = red[1][0];
+  if (n % 2 == 1 && t == 0) {
+    a += double(z[n - 1]) * r[n - 1];
+    b += double(z[n - 1]) * q[n - 1];
   }
+  a = block_sum(a, red);
+  double sum[2] = {a, block_sum(b, red)};
+  if (grid_sums<2, kSumThreads>(sum, partials, ticket, blockIdx.x, gridDim.x, red)) {
+    result[0] = sum[0];
+    result[1] = sum[1];
+  }
+}
+
+// the Lanczos vector passes of vec_lanczos_*
+__global__ void lanczos_next_kernel(long long n, const double *w, const double *ww, const double *isq, double *v,
+                                    double *t)
+{
+  const double f = 1. / sqrt(*ww);
+  for (long long i = blockIdx.x * (long long)blockDim.x + threadIdx.x; i < n; i += (long long)gridDim.x * blockDim.x) {
+    const double vi = f * w[i];
+    v[i] = vi;
+    t[i] = vi * isq[i];
+  }
+}
+
+__global__ void __launch_bounds__(kSumThreads) lanczos_dot_kernel(long long n, double *w, const double *isq,
+                                                                  const double *v, double *alpha, double *partials,
+                                                                  unsigned *ticket)
+{
+  __shared__ double red[kSumThreads / 64 + 1];
+  double acc = 0.;
+#pragma unroll 4
+  for (long long i = blockIdx.x * (long long)kSumThreads + threadIdx.x; i < n;
+       i += gridDim.x * (long long)kSumThreads) {
+    const double wi = w[i] * isq[i];
+    w[i] = wi;
+    acc += wi * v[i];
+  }
+  double sum[1] = {block_sum(acc, red)};
+  if (grid_sums<1, kSumThreads>(sum, partials, ticket, blockIdx.x, gridDim.x, red)) *alpha = sum[0];
+}
+
+__global__ void __launch_bounds__(kSumThreads) lanczos_update_kernel(long long n, double *w, const double *v,
+                                                                     const double *v0, const double *alpha,
+                                                                     const double *bb, double *ww, double *partials,
+                                                                     unsigned *ticket)
+{
+  __shared__ double red[kSumThreads / 64 + 1];
+  const double a = *alpha, b = bb ? sqrt(*bb) : 0.;
+  double acc = 0.;
+#pragma unroll 4
+  for (long long i = blockIdx.x * (long long)kSumThreads + threadIdx.x; i < n;
+       i += gridDim.x * (long long)kSumThreads) {
+    double wi = w[i] - a * v[i];
+    if (bb) wi -= b * v0[i];
+    w[i] = wi;
+    acc += wi * wi;
+  }
+  double sum[1] = {block_sum(acc, red)};
+  if (grid_sums<1, kSumThreads>(sum, partials, ticket, blockIdx.x, gridDim.x, red)) *ww = sum[0];
 }
 
 template <typename T>
@@ -272,48 +359,47 @@ hipError_t vec_dot(bool fp32, const void *x, const void *y, long long n, double 
   return hipGetLastError();
 }
 
-hipError_t vec_sum_partials(const double *partials, long long count, double *result_dev, hipStream_t s)
+hipError_t vec_cg_update(long long n, const double *zr, const double *pq, const void *q, void *r, void *rs,
+                         double *rr, double *host, double *partials, unsigned *ticket, hipStream_t s)
 {
-  if (count < 0 || count > 0x7fffffffLL) return hipErrorInvalidValue;
-  hipLaunchKernelGGL(dot_final_kernel, dim3(1), dim3(kThreads), 0, s, partials, (int)count, result_dev);
+  hipLaunchKernelGGL(cg_update_kernel, dim3(sum_grid(n)), dim3(kSumThreads), 0, s, n, zr, pq, (const double *)q,
+                     (double *)r, (float *)rs, rr, host, partials, ticket);
   return hipGetLastError();
 }
 
-hipError_t vec_dot2(const void *x, const void *y, const void *w, long long n, double *result_dev, double *partials,
-                    int n_partials, hipStream_t s)
+hipError_t vec_dot2(bool z_fp32, long long n, const void *z, const void *r, const void *q, double *result_dev,
+                    double *partials, unsigned *ticket, hipStream_t s)
 {
-  unsigned g = grid_for(n, 8);
-  if ((int)g > n_partials) g = n_partials;
-  hipLaunchKernelGGL(dot2_partial_kernel, dim3(g), dim3(kThreads), 0, s, (const double *)x, (const double *)y,
-                     (const double *)w, n, partials);
-  hipLaunchKernelGGL(dot_final_kernel, dim3(1), dim3(kThreads), 0, s, (const double *)partials, (int)g, result_dev);
-  hipLaunchKernelGGL(dot_final_kernel, dim3(1), dim3(kThreads), 0, s, (const double *)partials + g, (int)g,
-                     result_dev + 1);
+  if (z_fp32)
+    hipLaunchKernelGGL(dot2_kernel<float>, dim3(sum_grid(n)), dim3(kSumThreads), 0, s, n, (const float *)z,
+                       (const double *)r, (const double *)q, result_dev, partials, ticket);
+  else
+    hipLaunchKernelGGL(dot2_kernel<double>, dim3(sum_grid(n)), dim3(kSumThreads), 0, s, n, (const double *)z,
+                       (const double *)r, (const double *)q, result_dev, partials, ticket);
   return hipGetLastError();
 }
 
-hipError_t vec_cg_update(long long n, double alpha, const double *an, const double *ad, const void *p,
-                         const void *q, void *x, void *r, void *rs, double *result_dev, double *partials,
-                         int n_partials, hipStream_t s)
+hipError_t vec_lanczos_next(long long n, const void *w, const double *ww, const void *isq, void *v, void *t,
+                            hipStream_t s)
 {
-  unsigned g = grid_for(n, 8);
-  if ((int)g > n_partials) g = n_partials;
-  hipLaunchKernelGGL(cg_update_kernel, dim3(g), dim3(kThreads), 0, s, n, alpha, an, ad, (const double *)p,
-                     (const double *)q, (double *)x, (double *)r, (float *)rs, partials);
-  hipLaunchKernelGGL(dot_final_kernel, dim3(1), dim3(kThreads), 0, s, (const double *)partials, (int)g, result_dev);
+  hipLaunchKernelGGL(lanczos_next_kernel, dim3(grid_for(n, 4)), dim3(kThreads), 0, s, n, (const double *)w, ww,
+                     (const double *)isq, (double *)v, (double *)t);
   return hipGetLastError();
 }
 
-hipError_t vec_widen_dot2(long long n, const void *zs, void *z, const void *r, const void *q, double *result_dev,
-                          double *partials, int n_partials, hipStream_t s)
+hipError_t vec_lanczos_dot(long long n, void *w, const void *isq, const void *v, double *alpha, double *partials,
+                           unsigned *ticket, hipStream_t s)
 {
-  unsigned g = grid_for(n, 8);
-  if ((int)g > n_partials) g = n_partials;
-  hipLaunchKernelGGL(widen_dot2_kernel, dim3(g), dim3(kThreads), 0, s, n, (const float *)zs, (double *)z,
-                     (const double *)r, (const double *)q, partials);
-  hipLaunchKernelGGL(dot_final_kernel, dim3(1), dim3(kThreads), 0, s, (const double *)partials, (int)g, result_dev);
-  hipLaunchKernelGGL(dot_final_kernel, dim3(1), dim3(kThreads), 0, s, (const double *)partials + g, (int)g,
-                     result_dev + 1);
+  hipLaunchKernelGGL(lanczos_dot_kernel, dim3(sum_grid(n)), dim3(kSumThreads), 0, s, n, (double *)w,
+                     (const double *)isq, (const double *)v, alpha, partials, ticket);
+  return hipGetLastError();
+}
+
+hipError_t vec_lanczos_update(long long n, void *w, const void *v, const void *v0, const double *alpha,
+                              const double *bb, double *ww, double *partials, unsigned *ticket, hipStream_t s)
+{
+  hipLaunchKernelGGL(lanczos_update_kernel, dim3(sum_grid(n)), dim3(kSumThreads), 0, s, n, (double *)w,
+                     (const double *)v, (const double *)v0, alpha, bb, ww, partials, ticket);
   return hipGetLastError();
 }
 
