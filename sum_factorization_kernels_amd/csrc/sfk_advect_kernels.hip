@@ -39,11 +39,6 @@
 
 namespace sfk {
 
-template <int N>
-constexpr int adv_cells_per_block()
-{
-  return 256 / (N * N) > 0 ? 256 / (N * N) : 1;
-}
 constexpr int kAdvMaxThreads = 256;
 
 // LDS values per cell: two blocks (A, B) and six face layers; kind 2 one block,
@@ -57,7 +52,7 @@ constexpr int adv_lds_values()
 template <int N, typename T, int KIND>
 constexpr int adv_waves()
 {
-  constexpr int cb = adv_cells_per_block<N>();
+  constexpr int cb = full_cells(N);
   return lds_waves_per_simd(cb * adv_lds_values<N, T, KIND>() * (int)sizeof(T), cb * N * N);
 }
 
@@ -786,7 +781,7 @@ static hipError_t launch_advect_n(const AdvectLaunch &L, hipStream_t s)
   a.nx = L.nc[0];
   a.ny = L.nc[1];
   a.nz = L.nc[2];
-  const int CB = L.cb > 0 ? L.cb : adv_cells_per_block<N>();
+  const int CB = L.cb > 0 ? L.cb : full_cells(N);
   if (CB * N * N > kAdvMaxThreads) return hipErrorInvalidConfiguration;
   a.cb = CB;
   a.order = L.order;

@@ -31,20 +31,15 @@ namespace sfk {
 enum class Mode { Local = 0, Cont = 1, DG = 2 };
 
 template <int N>
-constexpr int cells_per_block()
-{
-  return 256 / (N * N) > 0 ? 256 / (N * N) : 1;
-}
-template <int N>
 constexpr int threads_per_block()
 {
-  return ((cells_per_block<N>() * N * N + 63) / 64) * 64;
+  return ((full_cells(N) * N * N + 63) / 64) * 64;
 }
 constexpr int kCellMaxThreads = 256;
 template <int N, typename T, bool FACES>
 constexpr int cell_waves()
 {
-  constexpr int cb = cells_per_block<N>();
+  constexpr int cb = full_cells(N);
   return lds_waves_per_simd(cb * (2 * N * N * N + (FACES ? 12 * N * N : 0)) * (int)sizeof(T), cb * N * N);
 }
 
@@ -525,7 +520,7 @@ cell_kernel(const CellArgs<N, T> a)
 // CU holds, and the tails of the 8 launches (15 %), set the time.
 template <int N, typename T, int NR>
 __global__ void __launch_bounds__(kCellMaxThreads)
-__attribute__((amdgpu_waves_per_eu(1, lds_waves_per_simd(NR * cells_per_block<N>() * 2 * N * N * N * (int)sizeof(T), cells_per_block<N>() * N * N))))
+__attribute__((amdgpu_waves_per_eu(1, lds_waves_per_simd(NR * full_cells(N) * 2 * N * N * N * (int)sizeof(T), full_cells(N) * N * N))))
 cont_coef_kernel(const CellArgs<N, T> a)
 {
   constexpr int N2 = N * N, N3 = N2 * N, p = N - 1;
@@ -691,7 +686,7 @@ struct DiagArgs {
 template <int N, typename T>
 __global__ void __launch_bounds__(threads_per_block<N>()) diag_kernel(const DiagArgs<N, T> a)
 {
-  constexpr int CB = cells_per_block<N>();
+  constexpr int CB = full_cells(N);
   constexpr int N2 = N * N, N3 = N * N * N, p = N - 1;
   __shared__ T sA[CB * N3];
   __shared__ T sR[CB * N3];
@@ -786,7 +781,7 @@ struct CoefGradArgs {
 template <int N, typename T>
 __global__ void __launch_bounds__(threads_per_block<N>()) coef_grad_kernel(const CoefGradArgs<N, T> a)
 {
-  constexpr int CB = cells_per_block<N>();
+  constexpr int CB = full_cells(N);
   constexpr int N2 = N * N, N3 = N * N * N, p = N - 1;
   __shared__ T sU[CB * N3];
   __shared__ T sL[CB * N3];
@@ -907,7 +902,7 @@ static hipError_t launch_coef_grad_n(const CoefGradLaunch &L, hipStream_t s)
   for (int d = 0; d < 3; ++d) a.cdiag[d] = T(L.inv_jac[d] * L.inv_jac[d] * jxw);
   a.nrhs = L.nrhs;
   a.vstride = L.vstride;
-  constexpr int CB = cells_per_block<N>();
+  constexpr int CB = full_cells(N);
   hipLaunchKernelGGL((coef_grad_kernel<N, T>), dim3((unsigned)((L.ncells + CB - 1) / CB)),
                      dim3(threads_per_block<N>()), 0, s, a);
   return hipGetLastError();
@@ -953,7 +948,7 @@ static hipError_t launch_cell_n(const CellLaunch &L, hipStream_t stream)
   }
   a.nrhs = L.nrhs;
   a.vstride = L.vstride;
-  const int CB = L.cb > 0 ? L.cb : cells_per_block<N>();
+  const int CB = L.cb > 0 ? L.cb : full_cells(N);
   if (CB * N * N > kCellMaxThreads) return hipErrorInvalidConfiguration;
   a.cb = CB;
   a.order = L.order;
@@ -1045,7 +1040,7 @@ static hipError_t launch_diag_n(const CellLaunch &L, hipStream_t stream)
   for (int d = 0; d < 3; ++d) a.cdiag[d] = T(L.inv_jac[d] * L.inv_jac[d] * jxw);
   a.jxw = T(jxw);
   a.cont = L.mode == 1;
-  constexpr int CB = cells_per_block<N>();
+  constexpr int CB = full_cells(N);
   const unsigned blocks = (unsigned)((L.ncells + CB - 1) / CB);
   hipLaunchKernelGGL((diag_kernel<N, T>), dim3(blocks), dim3(threads_per_block<N>()), 0, stream, a);
   return hipGetLastError();

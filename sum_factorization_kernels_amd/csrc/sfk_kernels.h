@@ -8,6 +8,31 @@
 
 namespace sfk {
 
+// Default cells per workgroup (n points per direction, n^2 threads per cell).
+// The launch bound's 256 threads unless fewer measured faster: workgroups of few
+// whole waves start and end independently, wait for fewer others at a barrier and
+// use the CU's LDS to the last granule; idle lanes of the last wave cost more
+// than that gains below about 80 % use.
+constexpr int full_cells(int n) { return 256 / (n * n) > 0 ? 256 / (n * n) : 1; }
+// per-q-metric SIPG.  Matvec with 12, 8, 3, 2 cells -> now: FP64 n = 4 37x29x41
+// 74 -> 67 us, n = 5 38x39x37 176 -> 163, n = 7 27x28x26 205 -> 152, n = 8 24x23x25
+// 164 -> 146; FP32 34 -> 32, 95 -> 87, 84 -> 74, 71 -> 67; n = 3 62x60x61 with 28
+// cells FP64 198 -> 189, FP32 127 -> 124 (7 cells 129)
+constexpr int sipg_general_cells(int n, bool fp32)
+{
+  return n == 2 ? (fp32 ? 64 : 16) : n == 3 ? (fp32 ? 5 : 7) : n == 4 ? 4 : n == 5 ? 5 : n == 6 ? 3 : 1;
+}
+// precomputed-matrix DG and Cartesian SIPG.  Matvec with 256 threads -> now, 6e6
+// unknowns: FP64 n = 8 31.2 -> 26.1 us, n = 5 25.1 -> 24.3, FP32 15.1 -> 14.8; FP32
+// n = 2 17.1 -> 16.5, where FP64 with 16 cells took 27.0 instead of 26.2 us.
+// (Advection with 5, 3 and 1 cells for n = 5, 6, 7 lost 3 to 5 % in the reverse
+// pass, the variable coefficient with 12 and 2 for n = 4 and 8 2 to 7 %.)
+constexpr int precomp_cells(int n, bool fp32)
+{
+  return n == 2 && fp32 ? 16 : n == 5 ? 5 : n == 8 && !fp32 ? 1 : full_cells(n);
+}
+
+
 // Workgroup schedule fields of the operator launches: cb = cells per
 // workgroup (0: the degree's default), order = block order (0 linear, 1 one
 // contiguous range of cells per XCD; logical_block in sfk_device.h).

@@ -94,16 +94,10 @@ __device__ __forceinline__ const SFK_CONST_AS PcTab<N, T> &pctab(const PcTab<N, 
   return *(const SFK_CONST_AS PcTab<N, T> *)opaque_ptr(p);
 }
 
-template <int N>
-constexpr int pc_cells_per_block()
-{
-  return kPcMaxThreads / (N * N) > 0 ? kPcMaxThreads / (N * N) : 1;
-}
-
 template <int N, typename T>
 constexpr int pc_waves()
 {
-  constexpr int cb = pc_cells_per_block<N>();
+  constexpr int cb = precomp_cells(N, sizeof(T) == 4);
   return lds_waves_per_simd(3 * cb * PcLds<N>::CS * (int)sizeof(T), cb * N * N);
 }
 
@@ -347,7 +341,7 @@ hipError_t launch_precomp_n(const PrecompLaunch &L, hipStream_t s)
   a.nx = L.nc[0];
   a.ny = L.nc[1];
   a.nz = L.nc[2];
-  const int CB = L.cb > 0 ? L.cb : pc_cells_per_block<N>();
+  const int CB = L.cb > 0 ? L.cb : precomp_cells(N, sizeof(T) == 4);
   if (CB * N * N > kPcMaxThreads) return hipErrorInvalidConfiguration;
   if (L.cheby && L.nrhs != 1) return hipErrorInvalidValue;
   a.cb = CB;

@@ -35,18 +35,11 @@
 
 namespace sfk {
 
-template <int N>
-constexpr int gen_cells_per_block()
-{
-  // default (4 N^3 + 12 N^2 values of LDS per cell); N = 6: 3 cells (108
-  // threads in two waves) measured fastest on MI355X for the 32^3 workload
-  return N <= 3 ? 256 / (N * N) : (N == 4 ? 12 : (N == 5 ? 8 : (N == 6 ? 3 : (N == 7 ? 3 : (N == 8 ? 2 : 1)))));
-}
 constexpr int kGenMaxThreads = 256;
 template <int N, typename T, bool DIAG>
 constexpr int gen_waves()
 {
-  constexpr int cb = gen_cells_per_block<N>();
+  constexpr int cb = sipg_general_cells(N, sizeof(T) == 4);
   return lds_waves_per_simd(cb * (4 * N * N * N + (DIAG ? 0 : 12 * N * N)) * (int)sizeof(T), cb * N * N);
 }
 
@@ -468,7 +461,7 @@ static hipError_t launch_general_n(const SipgLaunch &L, hipStream_t s)
   a.nx = L.nc[0];
   a.ny = L.nc[1];
   a.nz = L.nc[2];
-  a.cb = L.cb > 0 ? L.cb : gen_cells_per_block<N>();
+  a.cb = L.cb > 0 ? L.cb : sipg_general_cells(N, sizeof(T) == 4);
   a.order = L.order;
   if (a.cb * N * N > kGenMaxThreads) return hipErrorInvalidConfiguration;
   const size_t lds = size_t(a.cb) * (4 * N * N * N + (L.diagonal ? 0 : 12 * N * N)) * sizeof(T);

@@ -29,15 +29,18 @@ constexpr int kMaxThreads = 256; // __launch_bounds__ of the operator kernels
     return code;             \
   } while (0)
 
-// the kernel's default cells per workgroup (mirrors the device constants)
+// the kernel's default cells per workgroup
 int default_cb(const sfk_op *op)
 {
   const int n = op->d.degree + 1;
-  if (op->d.kind == SFK_DG_SIPG && op->d.geometry == SFK_GEOM_PER_Q) {
-    static const int tab[10] = {0, 0, 64, 28, 12, 8, 3, 3, 2, 1};
-    return n < 10 ? tab[n] : 1;
+  const bool fp32 = op->d.precision == SFK_FP32;
+  switch (op->d.kind) {
+  case SFK_DG_SIPG:
+    if (op->d.geometry == SFK_GEOM_PER_Q) return sipg_general_cells(n, fp32);
+    return sipg_kron(op) ? precomp_cells(n, fp32) : full_cells(n);
+  case SFK_DG_PRECOMP: return precomp_cells(n, fp32);
+  default: return full_cells(n);
   }
-  return kMaxThreads / (n * n) > 0 ? kMaxThreads / (n * n) : 1;
 }
 
 // LDS bytes per cell of the operator kernel behind sfk_apply
