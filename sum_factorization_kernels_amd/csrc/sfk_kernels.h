@@ -23,13 +23,13 @@ constexpr int sipg_general_cells(int n, bool fp32)
   return n == 2 ? (fp32 ? 64 : 16) : n == 3 ? (fp32 ? 5 : 7) : n == 4 ? 4 : n == 5 ? 5 : n == 6 ? 3 : 1;
 }
 // precomputed-matrix DG and Cartesian SIPG.  Matvec with 256 threads -> now, 6e6
-// unknowns: FP64 n = 8 31.2 -> 26.1 us, n = 5 25.1 -> 24.3, FP32 15.1 -> 14.8; FP32
-// n = 2 17.1 -> 16.5, where FP64 with 16 cells took 27.0 instead of 26.2 us.
+// unknowns: FP64 n = 8 31.2 -> 26.1 us; FP32 n = 5 15.1 -> 14.8, n = 2 17.1 -> 16.5,
+// where FP64 with 16 cells took 27.0 instead of 26.2 us.
 // (Advection with 5, 3 and 1 cells for n = 5, 6, 7 lost 3 to 5 % in the reverse
 // pass, the variable coefficient with 12 and 2 for n = 4 and 8 2 to 7 %.)
 constexpr int precomp_cells(int n, bool fp32)
 {
-  return n == 2 && fp32 ? 16 : n == 5 ? 5 : n == 8 && !fp32 ? 1 : full_cells(n);
+  return n == 2 && fp32 ? 16 : n == 5 && fp32 ? 5 : n == 8 && !fp32 ? 1 : full_cells(n);
 }
 
 

@@ -156,6 +156,19 @@ __device__ __forceinline__ void pc_load_layers(const T *src, const int (&nbr)[6]
   }
 }
 
+// Matvec results that leave as the block's consecutive values instead of z lines:
+// where a z line's lanes cover parts of cache lines (72 B for n = 3, 200 B for n =
+// 5 in FP64), non-temporal stores of them cost HBM a read where the vectors exceed
+// the Infinity Cache.  z lines -> consecutive: n = 3 FP64 3e6 unknowns 16.6 -> 13.8
+// us, 1.9e7 123 -> 101, FP32 1.9e7 50.5 -> 47.9; n = 5 FP64 1.9e7 107 -> 93, but
+// 3e6 13.8 -> 14.7; n = 5 FP32, n = 7 and 9: 3 to 7 % slower.  (Plain stores of
+// either form: 5 to 30 % slower at most sizes.)
+template <int N, typename T>
+constexpr bool pc_flat_store()
+{
+  return N == 3 || (N == 5 && sizeof(T) == 8);
+}
+
 template <int N, typename T, bool COUPLE, bool CHEBY>
 __global__ void __launch_bounds__(kPcMaxThreads) __attribute__((amdgpu_waves_per_eu(1, pc_waves<N, T>())))
 precomp_kernel(PcArgs<N, T> a)
@@ -167,6 +180,7 @@ precomp_kernel(PcArgs<N, T> a)
   // such pieces cost more than coalesced copies through LDS on both ends (p = 2
   // FP32 Chebyshev step 30 us flat, 36 us on z lines)
   constexpr bool FLAT = CHEBY && N <= 3;
+  constexpr bool FLAT_ST = FLAT || (!CHEBY && pc_flat_store<N, T>());
   const long long c0 = (long long)logical_block(blockIdx.x, gridDim.x, a.order) * cb;
   const long long voff = (long long)blockIdx.y * a.nvec;
   const T *src = a.src + voff;
@@ -174,12 +188,12 @@ precomp_kernel(PcArgs<N, T> a)
   const bool act = c < cb && c0 + c < a.ncells;
   // (the divisions of the cell's coordinates on the scalar unit)
   int nbr[6] = {0, 0, 0, 0, 0, 0};
-  const long long cell = act ? locate_cell((unsigned)c0, (unsigned)c, a.nx, a.ny, a.nz, FLAT ? 0 : a.order, nbr) : 0;
+  const long long cell = act ? locate_cell((unsigned)c0, (unsigned)c, a.nx, a.ny, a.nz, FLAT_ST ? 0 : a.order, nbr) : 0;
   T *U = dyn_lds<T>() + (act ? c : 0) * CS;
   T *P = U + cb * CS, *Q = P + cb * CS;
   const long long g0 = cell * N3 + l; // this thread's z line: g0 + k N2
   // FLAT: the block's nval consecutive values lie in LDS as in memory
-  static_assert(!FLAT || CS == N3, "unpadded");
+  static_assert(!FLAT_ST || CS == N3, "unpadded");
   const long long rem = a.ncells - c0;
   const int nval = (rem < cb ? (int)rem : cb) * N3;
 
@@ -271,13 +285,13 @@ precomp_kernel(PcArgs<N, T> a)
     pc_read<N, 2>(Q, l, v);
     eo_apply<N, 1>(pt.M, v, o);
     pc_read<N, 2>(P, l, v);
-    if constexpr (FLAT) {
+    if constexpr (FLAT_ST) {
 #pragma unroll
       for (int k = 0; k < N; ++k) o[k] += v[k];
       pc_write<N, 2>(U, l, o);
     }
 #pragma unroll
-    for (int k = 0; k < (FLAT ? 0 : N); ++k) {
+    for (int k = 0; k < (FLAT_ST ? 0 : N); ++k) {
       const long long g = g0 + k * N2;
       const T au = o[k] + v[k];
       if constexpr (CHEBY) {
@@ -292,13 +306,16 @@ precomp_kernel(PcArgs<N, T> a)
       }
     }
   }
-  if constexpr (FLAT) {
+  if constexpr (FLAT_ST) {
     __syncthreads();
 #pragma unroll
     for (int k = 0; k < N; ++k) {
       const int i = t + k * (int)blockDim.x;
-      if (i < nval) {
-        const long long g = c0 * N3 + i;
+      if (i >= nval) break;
+      const long long g = c0 * N3 + i;
+      if constexpr (!CHEBY) {
+        __builtin_nontemporal_store(dyn_lds<T>()[i], a.dst + voff + g);
+      } else {
         const T res = dyn_lds<T>()[i] - a.rhs[g];
         T tmv = a.c_np * a.diag[g] * res;
         if (a.c_tm != T(0)) tmv = a.c_tm * a.tm[g] + tmv;
