@@ -259,7 +259,10 @@ sfk_status sfk_tune(sfk_op *op, int repeats, sfk_schedule *best, double *best_se
  * upper/1000: a preconditioner acting on most of the spectrum).  The preconditioner runs on `smoother_op` (FP32 or FP64 operator
  * on the same mesh); the residual, inner products, Lanczos and the final
  * residual stay FP64 on `op` (which must be FP64).  x: initial guess in,
- * solution out; b: right-hand side (FP64, Dirichlet rows 0). */
+ * solution out; b: right-hand side (FP64, Dirichlet rows 0).  Its work space
+ * (10 FP64 and 5 smoother-precision vectors) stays with `op` from call to call
+ * up to 1 GiB and goes with sfk_op_destroy; a larger one, or that of a solve
+ * that runs while another thread solves with `op`, is freed on return. */
 typedef struct sfk_solve_stats {
   int iterations;
   double initial_residual, final_residual; /* ||b - A x||_2 (FP64) */
