@@ -253,13 +253,10 @@ cont_tp_kernel(const TpArgs<T> a)
   T *dst = a.dst + (long long)blockIdx.y * a.vstride;
   const int it = threadIdx.x;
 
-  // ---- phase Y: this thread's y line is column X, plane ez p + 1 + ys, rows
-  // (ey-1) p .. (ey+1) p.  Offsets are relative to row -p of the layer's
-  // first plane, so they are never negative.  Row 0 of the line is a node
-  // with a value if ey >= 2, rows 1..p if ey >= 1, the last row if the cell
-  // is not the last in y; the grid's last plane (ys = p-1 of the last layer)
-  // has none.
-  unsigned o_first, o_low, o_mid, o_last, top_plane;
+  // ---- phase Y: this thread's y line (tp_line); the grid's last plane (ys =
+  // p-1 of the last layer) is Dirichlet
+  TpLine o;
+  unsigned top_plane;
   int ys;
   T *ya, *yu = nullptr;
   T dxz = T(0), exz = T(0), dxz0 = T(0), exz0 = T(0);
@@ -268,12 +265,7 @@ cont_tp_kernel(const TpArgs<T> a)
     const int xh = i % HX, rest = i / HX, eyl = rest % BY;
     ys = rest / BY;
     const int ey = ey0 + eyl, X = x0 - p + xh;
-    const bool ok = ey < a.ny && X > 0 && X < gx - 1;
-    const unsigned o = (unsigned)(((1 + ys) * plane + ey * p * gx + X) * ES);
-    o_first = ok && ey >= 2 ? o : kOob;
-    o_low = ok && ey >= 1 ? o : kOob;
-    o_mid = ok ? o : kOob;
-    o_last = ok && ey + 1 < a.ny ? o : kOob;
+    o = tp_line(p, ES, gx, a.ny, plane, ys, ey, X);
     top_plane = ys == p - 1 ? kOob : 0u;
     ya = sA + ys * PSA + eyl * p * RPA + xh;
     if constexpr (FUSED) {
@@ -294,8 +286,8 @@ cont_tp_kernel(const TpArgs<T> a)
     }
   }
   T u[2 * N - 1];
-  auto load_lines = [&](const T *layer, unsigned bytes, unsigned v0, unsigned v1, unsigned vm, unsigned vl) {
-    const Rsrc r = make_rsrc(layer - (long long)p * gx, bytes);
+  auto load_lines = [&](const T *base, unsigned bytes, unsigned v0, unsigned v1, unsigned vm, unsigned vl) {
+    const Rsrc r = make_rsrc(base, bytes);
     const unsigned rb = opaque_s(row_bytes);
 #pragma unroll
     for (int j = 0; j < 2 * N - 1; ++j)
@@ -304,7 +296,8 @@ cont_tp_kernel(const TpArgs<T> a)
   // (live false: nothing is read, the loads only keep the loop uniform)
   auto load_y = [&](int ez, bool live) {
     const unsigned m = ez == a.nz - 1 ? top_plane : 0u;
-    load_lines(src + (long long)ez * layer_size, live ? kAll : 0u, o_first | m, o_low | m, o_mid | m, o_last | m);
+    load_lines(src + ((long long)ez * layer_size + tp_line_base(p, gx, plane)), live ? kAll : 0u, o.first | m, o.low | m,
+               o.mid | m, o.last | m);
   };
   auto phase_y = [&](bool plane0) {
     T un[FUSED ? p : 1]; // the input (RSRC: the right-hand side) at the line's own nodes
@@ -519,8 +512,9 @@ cont_tp_kernel(const TpArgs<T> a)
     // without stores
     const int e0 = ez_begin - 1;
     const bool on = ys == 0 && e0 > 0;
-    auto below = [&](unsigned o) { return on && o != kOob ? o - plane_bytes : kOob; };
-    load_lines(src + (long long)e0 * layer_size, kAll, below(o_first), below(o_low), below(o_mid), below(o_last));
+    auto below = [&](unsigned v) { return on ? v : kOob; };
+    load_lines(src + ((long long)e0 * layer_size + tp_line_base(p, gx, 0)), kAll, below(o.first), below(o.low),
+               below(o.mid), below(o.last));
     phase_y(true);
     if (PF) load_y(e0, true);
     phase_x();
@@ -682,9 +676,7 @@ static hipError_t launch_tp_shape(const TpLaunch &L, hipStream_t s)
   a.zc = L.zc > 0 ? (L.zc < a.nz ? L.zc : a.nz) : a.nz;
   a.order = L.order;
   a.vstride = L.vstride;
-  // 32-bit byte offsets: a plane, and the p+1 planes of a layer, hold less
-  // than 2^31 bytes
-  if ((long long)N * a.gx * a.gy * (long long)sizeof(T) >= (1LL << 31)) return hipErrorInvalidValue;
+  if (!tp_offsets_fit(N, a.gx, a.gy, (int)sizeof(T))) return hipErrorInvalidValue;
   const long long nchunks = (a.nz + a.zc - 1) / a.zc;
   const long long blocks = (long long)a.ntx * a.nty * nchunks;
   if (blocks <= 0 || blocks > 0x7fffffffLL) return hipErrorInvalidConfiguration;

@@ -9,6 +9,7 @@
 #include <vector>
 
 #include "sfk_internal.h"
+#include "sfk_tp_offsets.h"
 
 namespace sfk {
 
@@ -430,9 +431,7 @@ __device__ __forceinline__ T load_stream(const T *p)
 }
 
 // Buffer accesses: a uniform base, a 32-bit offset per lane and a uniform
-// offset.  A lane offset of kOob lies beyond every buffer described here
-// (fewer than 2^31 bytes): such lanes read 0 and store nothing.
-constexpr unsigned kOob = 0x80000000u, kAll = 0x7fffffffu;
+// offset.  Lanes whose offset is out of range (kOob) read 0 and store nothing.
 typedef unsigned sfk_u2 __attribute__((ext_vector_type(2)));
 using Rsrc = __amdgpu_buffer_rsrc_t;
 template <typename T>
