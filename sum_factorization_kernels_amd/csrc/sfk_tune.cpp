@@ -104,10 +104,26 @@ int max_cb(const sfk_op *op)
 
 // ---- tuning cache: the file named by SFK_TUNE_CACHE holds one line per
 // tuned operator, "<key> <cb> <order> <scatter> <shape> <zc> <cheby shape>
-// <cheby zc> <cheby order> <seconds>", the key naming the device and every
-// descriptor field the kernels and their timing depend on.  Lines are
-// appended; the last line of a key wins.
+// <cheby zc> <cheby order> <seconds>", the key naming the device, every
+// descriptor field the kernels and their timing depend on, and the library's
+// schedules (a line of a library with other kernels or tiles holds a time and a
+// choice that mean nothing here).  Lines are appended; the last line of a key
+// wins.
 std::mutex g_cache_mutex;
+
+// Raised by one with every change of a kernel, of its default schedule or of
+// the rule that picks it, for any operator; the tile table counts by itself.
+constexpr int kScheduleGeneration = 2;
+unsigned tile_table_hash(int n)
+{
+  unsigned h = 2166136261u; // FNV-1a over the tiles' cells
+  for (int sh = 1; sh < tp_shape_count(n); ++sh) {
+    int b[2];
+    tp_shape(n, sh, &b[0], &b[1]);
+    for (int v : b) h = (h ^ (unsigned)v) * 16777619u;
+  }
+  return h;
+}
 
 std::string cache_key(const sfk_op *op)
 {
@@ -123,7 +139,9 @@ std::string cache_key(const sfk_op *op)
   const sfk_op_desc &d = op->d;
   std::ostringstream k;
   k << dev << "/k" << d.kind << "/p" << d.degree << "/f" << d.precision << "/b" << d.basis << "/g" << d.geometry
-    << "/fl" << d.flags << "/n" << d.n_cells[0] << "x" << d.n_cells[1] << "x" << d.n_cells[2] << "/r" << d.n_rhs;
+    << "/fl" << d.flags << "/n" << d.n_cells[0] << "x" << d.n_cells[1] << "x" << d.n_cells[2] << "/r" << d.n_rhs
+    << "/s" << kScheduleGeneration;
+  if (tp_ok(op)) k << "t" << std::hex << tile_table_hash(d.degree + 1);
   return k.str();
 }
 
@@ -264,6 +282,8 @@ sfk_status sfk_tune(sfk_op *op, int repeats, sfk_schedule *best, double *best_se
         const bool cheby_ok =
             dg_cheby ? e.cheby[1] <= max_cb(op) && e.cheby[2] >= 0 && e.cheby[2] <= 2
                      : e.cheby[0] < 0 || (tp_ok(op) && e.cheby[0] < tp_shape_count(op->d.degree + 1) &&
+                                          tp_shape_fits(op->d.degree + 1, e.cheby[0],
+                                                        op->d.precision == SFK_FP32, lds_limit()) &&
                                           e.cheby[1] >= 0 && (e.cheby[2] == 0 || e.cheby[2] == 1));
         if (cheby_ok) {
           op->cheby_shape = dg_cheby ? -1 : e.cheby[0];
