@@ -21,9 +21,10 @@
  * lane-interleaved layout: sfk_layout_*.
  *
  * All device pointers are caller-owned device memory (hipMalloc, torch).
- * A handle is not thread-safe; use one handle per host thread.  Every
- * entry point returns an sfk_status; sfk_last_error() returns a
- * thread-local description of the last failure.
+ * A handle is not thread-safe; use one handle per host thread (concurrent
+ * solves excepted: sfk_solve_cg_cheby).  Every entry point returns an
+ * sfk_status; sfk_last_error() returns a thread-local description of the last
+ * failure.
  */
 #ifndef SFK_H
 #define SFK_H
@@ -263,7 +264,9 @@ sfk_status sfk_tune(sfk_op *op, int repeats, sfk_schedule *best, double *best_se
  * solution out; b: right-hand side (FP64, Dirichlet rows 0).  Its work space
  * (10 FP64 and 5 smoother-precision vectors) stays with `op` from call to call
  * up to 1 GiB and goes with sfk_op_destroy; a larger one, or that of a solve
- * that runs while another thread solves with `op`, is freed on return. */
+ * that runs while another thread solves with `op`, is freed on return.
+ * Several threads may solve with the same operators at once, each on a stream
+ * of its own, while nobody changes the operators' data or schedules. */
 typedef struct sfk_solve_stats {
   int iterations;
   double initial_residual, final_residual; /* ||b - A x||_2 (FP64) */

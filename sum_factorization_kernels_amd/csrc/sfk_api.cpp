@@ -102,7 +102,6 @@ bool sipg_kron(const sfk_op *op)
          !(op->d.flags & SFK_FLAG_REF_X_SWEEP) && op->d.degree <= kMaxDegreeTp;
 }
 
-// the operator's 1D tables in device memory, uploaded on the first launch
 // the precomputed DG Laplacian's kernels read their own table type
 static hipError_t upload_precomp(sfk_op *op, void **dev)
 {
@@ -129,25 +128,36 @@ static bool has_tp(const sfk_op *op)
 
 sfk_status ensure_device_tables(sfk_op *op)
 {
-  if (op->dtab && (op->tptab || !has_tp(op))) return SFK_OK;
-  hipError_t e = hipSuccess;
-  if (!op->dtab)
-    e = op->d.kind == SFK_DG_PRECOMP || sipg_kron(op)
-            ? upload_precomp(op, &op->dtab)
-        : op->d.kind == SFK_DG_ADVECT
-            ? upload_advect_tables(op->tab, op->d.inv_jac, op->d.precision == SFK_FP32, &op->dtab)
-            : upload_device_tables(op->tab, op->d.precision == SFK_FP32, &op->dtab);
-  if (e == hipSuccess && has_tp(op) && !op->tptab)
-    e = upload_tp_tables(op->tab, op->d.inv_jac, op->d.precision == SFK_FP32, &op->tptab);
+  if (op->tables_ready.load(std::memory_order_acquire)) return SFK_OK;
+  std::lock_guard<std::mutex> lock(op->lazy_lock);
+  // entered into the handle only when complete
+  auto upload_to = [](void **dev, auto up) {
+    if (*dev) return hipSuccess;
+    void *p = nullptr;
+    const hipError_t e = up(&p);
+    if (e == hipSuccess) *dev = p;
+    else if (p) (void)hipFree(p);
+    return e;
+  };
+  const bool fp32 = op->d.precision == SFK_FP32;
+  hipError_t e = upload_to(&op->dtab, [&](void **p) {
+    if (op->d.kind == SFK_DG_PRECOMP || sipg_kron(op)) return upload_precomp(op, p);
+    if (op->d.kind == SFK_DG_ADVECT) return upload_advect_tables(op->tab, op->d.inv_jac, fp32, p);
+    return upload_device_tables(op->tab, fp32, p);
+  });
+  if (e == hipSuccess && has_tp(op))
+    e = upload_to(&op->tptab, [&](void **p) { return upload_tp_tables(op->tab, op->d.inv_jac, fp32, p); });
   if (e != hipSuccess) {
     set_error(std::string("device tables: ") + hipGetErrorString(e));
     return SFK_ERR_HIP;
   }
+  op->tables_ready.store(true, std::memory_order_release);
   return SFK_OK;
 }
 
 sfk_status ensure_scratch(sfk_op *op, size_t bytes)
 {
+  std::lock_guard<std::mutex> lock(op->lazy_lock);
   if (op->scratch_bytes >= bytes) return SFK_OK;
   if (op->scratch) (void)hipFree(op->scratch);
   op->scratch = nullptr;

@@ -1,6 +1,7 @@
 // The operator handle behind the opaque sfk_op of include/sfk.h.
 #pragma once
 
+#include <atomic>
 #include <mutex>
 
 #include "sfk.h"
@@ -43,6 +44,10 @@ struct sfk_op {
   void *solve_ws = nullptr;
   size_t solve_ws_bytes = 0;
   std::mutex solve_ws_lock;
+  // device tables uploaded (the flag is set last); the lock covers their upload
+  // and the allocation of the scratch space, not the scratch space's use
+  std::atomic<bool> tables_ready{false};
+  std::mutex lazy_lock;
 };
 
 namespace sfk {

@@ -396,7 +396,10 @@ extern "C" sfk_status sfk_solve_cg_cheby(sfk_op *op, sfk_op *smoother_op, const 
     double rho_old = 1. / sigma1;
     for (int j = 1; j < cheby_degree; ++j) {
       const double rho = 1. / (2. * sigma1 - rho_old);
-      SOLVER_ST(sfk_cheby_step(S.sm, rr, z, inv_sm, *spare, tms.p, 2. * rho / delta, rho * rho_old, stream));
+      // sfk_cheby_step with A z in this solve's work space (a Lanczos vector):
+      // the operator's scratch space would be shared with solves in other threads
+      SOLVER_ST(sfk_apply(S.sm, z, lw.p, stream));
+      SOLVER_HIP(vec_cheby_update(f32, n, lw.p, rr, z, inv_sm, *spare, tms.p, 2. * rho / delta, rho * rho_old, s));
       std::swap(z, *spare);
       rho_old = rho;
       ++S.st.matvecs_inner;
