@@ -178,6 +178,25 @@ bool uses_tp(const sfk_op *op)
   return has_tp(op) && (op->cont_scatter == 2 || op->cont_scatter == -1);
 }
 
+static sfk_op::TpRun resolve_tp(const sfk_op *op, int shape, int zc)
+{
+  if (has_tp(op) && shape >= 0) tp_plan(op->d.degree + 1, op->d.precision == SFK_FP32, op->d.n_cells, &shape, &zc);
+  return {shape, zc};
+}
+void set_tp_schedule(sfk_op *op, int shape, int zc)
+{
+  op->tp_shape = shape;
+  op->tp_zc = zc;
+  op->tp_run = resolve_tp(op, shape, zc);
+}
+void set_cheby_schedule(sfk_op *op, int shape, int zc, int order)
+{
+  op->cheby_shape = shape;
+  op->cheby_zc = zc;
+  op->cheby_order = order;
+  op->cheby_run = resolve_tp(op, shape, zc);
+}
+
 void fill_tp_launch(const sfk_op *op, TpLaunch &L, bool cheby)
 {
   L.n = op->d.degree + 1;
@@ -187,9 +206,9 @@ void fill_tp_launch(const sfk_op *op, TpLaunch &L, bool cheby)
   L.nrhs = op->d.n_rhs;
   L.vstride = op->nvec;
   const bool own = cheby && op->cheby_shape >= 0;
-  L.shape = own ? op->cheby_shape : op->tp_shape;
-  L.zc = own ? op->cheby_zc : op->tp_zc;
-  tp_plan(L.n, L.fp32, L.nc, &L.shape, &L.zc);
+  const sfk_op::TpRun &run = own ? op->cheby_run : op->tp_run;
+  L.shape = run.shape;
+  L.zc = run.zc;
   L.order = own ? op->cheby_order : op->sched_order;
 }
 
@@ -291,6 +310,7 @@ sfk_status sfk_op_create(const sfk_op_desc *desc, sfk_op **out)
   }
   op->ncq = op->ncells * n * n * n;
   op->nfq = op->ncells * n * n;
+  set_tp_schedule(op, 0, 0);
   // tables to the device now when a device is present (a first launch
   // inside a graph capture must not allocate); without one the upload
   // waits for the first launch

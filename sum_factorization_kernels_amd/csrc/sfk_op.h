@@ -32,6 +32,11 @@ struct sfk_op {
   // solver's smoother): tile shape, cells in z and block order chosen by
   // sfk_tune for those launches (cheby_shape -1: the matvec's)
   int cheby_shape = -1, cheby_zc = 0, cheby_order = 1;
+  // both with the automatic parts resolved for the mesh (set_tp_schedule,
+  // set_cheby_schedule: the only writers of these and of the four above)
+  struct TpRun {
+    int shape = 1, zc = 0;
+  } tp_run, cheby_run;
   // the per-q-metric SIPG kernel's fused Chebyshev step: cells per block
   // chosen by sfk_tune for it, with cheby_order (0: the matvec's schedule)
   int cheby_cb = 0;
@@ -108,6 +113,11 @@ sfk_status ensure_device_tables(sfk_op *op);
 bool sipg_kron(const sfk_op *op);
 // the continuous Laplacian's launches use the tensor-product kernel
 bool uses_tp(const sfk_op *op);
+// schedules of the tensor-product kernel's launches (0: automatic, resolved
+// here, once: the cost model of tp_plan takes 1 to 2.5 us, which every launch of
+// an untuned operator paid when it was asked there)
+void set_tp_schedule(sfk_op *op, int shape, int zc);
+void set_cheby_schedule(sfk_op *op, int shape, int zc, int order);
 // (cheby: the schedule of the fused Chebyshev launches)
 void fill_tp_launch(const sfk_op *op, TpLaunch &L, bool cheby = false);
 

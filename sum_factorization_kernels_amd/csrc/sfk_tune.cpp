@@ -258,9 +258,8 @@ sfk_status sfk_op_set_schedule(sfk_op *op, const sfk_schedule *s)
   op->sched_cb = s->cells_per_block;
   op->sched_order = s->block_order;
   op->cont_scatter = s->cont_scatter;
-  op->tp_shape = s->tile_shape;
-  op->tp_zc = s->z_cells;
-  op->cheby_shape = -1; // the Chebyshev launches follow the new schedule
+  set_tp_schedule(op, s->tile_shape, s->z_cells);
+  set_cheby_schedule(op, -1, 0, op->cheby_order); // the Chebyshev launches follow the new schedule
   op->cheby_cb = 0;
   return SFK_OK;
 }
@@ -286,10 +285,8 @@ sfk_status sfk_tune(sfk_op *op, int repeats, sfk_schedule *best, double *best_se
                                                         op->d.precision == SFK_FP32, lds_limit()) &&
                                           e.cheby[1] >= 0 && (e.cheby[2] == 0 || e.cheby[2] == 1));
         if (cheby_ok) {
-          op->cheby_shape = dg_cheby ? -1 : e.cheby[0];
-          op->cheby_zc = dg_cheby ? 0 : e.cheby[1];
+          set_cheby_schedule(op, dg_cheby ? -1 : e.cheby[0], dg_cheby ? 0 : e.cheby[1], e.cheby[2]);
           op->cheby_cb = dg_cheby ? e.cheby[1] : 0;
-          op->cheby_order = e.cheby[2];
           if (best) *best = e.s;
           if (best_seconds) *best_seconds = e.seconds;
           return SFK_OK;
@@ -365,8 +362,7 @@ sfk_status sfk_tune(sfk_op *op, int repeats, sfk_schedule *best, double *best_se
             if (tp_cost(n, op->d.n_cells, sh, zc) > kTpTry * tp_best) continue;
             op->sched_order = order;
             op->cont_scatter = 2;
-            op->tp_shape = sh;
-            op->tp_zc = zc;
+            set_tp_schedule(op, sh, zc);
             trial(sfk_schedule{win_cb, order, 2, sh, zc});
           }
       }
@@ -393,9 +389,7 @@ sfk_status sfk_tune(sfk_op *op, int repeats, sfk_schedule *best, double *best_se
         for (int zc : tp_zc_candidates(nz)) {
           if (status != SFK_OK) break;
           if (tp_cost(n, op->d.n_cells, sh, zc) > kTpTry * tp_best) continue;
-          op->cheby_shape = sh;
-          op->cheby_order = order;
-          op->cheby_zc = zc;
+          set_cheby_schedule(op, sh, zc, order);
           TpLaunch T;
           fill_tp_launch(op, T, true);
           T.cheby = 2;
@@ -475,17 +469,12 @@ sfk_status sfk_tune(sfk_op *op, int repeats, sfk_schedule *best, double *best_se
     op->sched_cb = saved_cb;
     op->sched_order = saved_order;
     op->cont_scatter = saved_scatter;
-    op->tp_shape = saved_shape;
-    op->tp_zc = saved_zc;
-    op->cheby_shape = saved_cshape;
-    op->cheby_zc = saved_czc;
-    op->cheby_order = saved_corder;
+    set_tp_schedule(op, saved_shape, saved_zc);
+    set_cheby_schedule(op, saved_cshape, saved_czc, saved_corder);
     op->cheby_cb = saved_ccb;
     return status != SFK_OK ? status : SFK_ERR_HIP;
   }
-  op->cheby_shape = cwin[0];
-  op->cheby_zc = cwin[1];
-  op->cheby_order = cwin[2];
+  set_cheby_schedule(op, cwin[0], cwin[1], cwin[2]);
   op->cheby_cb = 0;
   if (dwin[0] > 0) {
     op->cheby_cb = dwin[0];
@@ -499,8 +488,7 @@ sfk_status sfk_tune(sfk_op *op, int repeats, sfk_schedule *best, double *best_se
   op->sched_cb = win.cells_per_block;
   op->sched_order = win.block_order;
   op->cont_scatter = win.cont_scatter;
-  op->tp_shape = win.tile_shape;
-  op->tp_zc = win.z_cells;
+  set_tp_schedule(op, win.tile_shape, win.z_cells);
   if (best) *best = win;
   if (best_seconds) *best_seconds = win_t;
   return SFK_OK;
