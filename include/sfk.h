@@ -229,7 +229,7 @@ sfk_status sfk_op_set_schedule(sfk_op *op, const sfk_schedule *s);
 sfk_status sfk_op_max_cells_per_block(const sfk_op *op, int *max_cells);
 /* Number of tile shapes of the continuous tensor-product kernel and the
  * shape's cells in x and y (bx, by may be NULL; shape 0: those of the shape
- * chosen for this operator's mesh). */
+ * that the matvec runs on with tile_shape 0 and the operator's z_cells). */
 sfk_status sfk_op_tile_shape(const sfk_op *op, int shape, int *count, int *bx, int *by);
 /* Times sfk_apply for every candidate schedule (`repeats` applies each,
  * after a warm-up apply, on internal scratch vectors; stream-ordered on

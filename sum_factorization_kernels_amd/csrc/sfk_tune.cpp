@@ -222,7 +222,7 @@ sfk_status sfk_op_tile_shape(const sfk_op *op, int shape, int *count, int *bx, i
   const int n = op->d.degree + 1, c = tp_shape_count(n);
   if (count) *count = c;
   if (shape < 0 || shape >= c) TUNE_FAIL(SFK_ERR_INVALID_ARG, "tile shape must be in 0.." + std::to_string(c - 1));
-  int x = 0, y = 0, zc = 1;
+  int x = 0, y = 0, zc = op->tp_zc;
   if (shape == 0) tp_plan(n, op->d.precision == SFK_FP32, op->d.n_cells, &shape, &zc);
   tp_shape(n, shape, &x, &y);
   if (bx) *bx = x;

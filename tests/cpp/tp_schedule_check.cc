@@ -1,6 +1,8 @@
 // The tensor-product launches of an operator with an automatic schedule: what
 // they run on is the cost model's choice, and filling a launch does not ask the
-// model again (it allocates; nothing may be allocated here).  Without a device.
+// model again (it allocates; nothing may be allocated here); and the tile that
+// sfk_op_tile_shape names for tile_shape 0 is the one they run on.  Without a
+// device.
 #include <cstdio>
 #include <cstdlib>
 #include <new>
@@ -34,6 +36,18 @@ static int check(sfk_op *op, bool cheby, int shape, int zc)
   return 1;
 }
 
+static int check_tile(sfk_op *op)
+{
+  TpLaunch L;
+  fill_tp_launch(op, L);
+  int bx = 0, by = 0, lx = 0, ly = 0;
+  tp_shape(op->d.degree + 1, L.shape, &lx, &ly);
+  if (sfk_op_tile_shape(op, 0, nullptr, &bx, &by) == SFK_OK && bx == lx && by == ly) return 0;
+  std::printf("degree %d, %d cells in z, z_cells %d: tile 0 is %d x %d, the launch's %d x %d\n", op->d.degree,
+              op->d.n_cells[2], op->tp_zc, bx, by, lx, ly);
+  return 1;
+}
+
 int main()
 {
   int bad = 0;
@@ -52,11 +66,13 @@ int main()
         sfk_op *op = nullptr;
         if (sfk_op_create(&d, &op) != SFK_OK) return std::printf("create: %s\n", sfk_last_error()), EXIT_FAILURE;
         for (bool cheby : {false, true}) bad += check(op, cheby, 0, 0);
+        bad += check_tile(op);
         for (int asked : {0, 1, 2})
           for (int zc : {0, 2}) {
             const sfk_schedule s{0, 1, 2, asked, zc};
             if (sfk_op_set_schedule(op, &s) != SFK_OK) return std::printf("set: %s\n", sfk_last_error()), EXIT_FAILURE;
             for (bool cheby : {false, true}) bad += check(op, cheby, asked, zc);
+            if (asked == 0) bad += check_tile(op);
           }
         sfk_op_destroy(op);
       }

@@ -1,5 +1,6 @@
 """Automatic schedules of the tensor-product kernel are resolved once, not at
-every launch (CPU: the launch descriptors an operator makes)."""
+every launch, and sfk_op_tile_shape names their tile (CPU: the launch
+descriptors an operator makes)."""
 import os
 import subprocess
 
@@ -24,5 +25,5 @@ def run_check(name, tmp_path):
     assert r.returncode == 0, r.stdout + r.stderr
 
 
-def test_launches_do_not_plan(tmp_path):
+def test_automatic_schedules(tmp_path):
     run_check("tp_schedule_check", tmp_path)
