@@ -178,9 +178,20 @@ bool uses_tp(const sfk_op *op)
   return has_tp(op) && (op->cont_scatter == 2 || op->cont_scatter == -1);
 }
 
+Chip current_chip()
+{
+  Chip c;
+  int dev = 0, v = 0;
+  if (hipGetDevice(&dev) != hipSuccess) return c;
+  if (hipDeviceGetAttribute(&v, hipDeviceAttributeMaxSharedMemoryPerBlock, dev) == hipSuccess && v > 0) c.lds = v;
+  if (hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && v > 0) c.cus = v;
+  return c;
+}
+
 static sfk_op::TpRun resolve_tp(const sfk_op *op, int shape, int zc)
 {
-  if (has_tp(op) && shape >= 0) tp_plan(op->d.degree + 1, op->d.precision == SFK_FP32, op->d.n_cells, &shape, &zc);
+  if (has_tp(op) && (shape == 0 || (shape > 0 && zc == 0)))
+    tp_plan(op->d.degree + 1, op->d.precision == SFK_FP32, op->d.n_cells, current_chip(), &shape, &zc);
   return {shape, zc};
 }
 void set_tp_schedule(sfk_op *op, int shape, int zc)

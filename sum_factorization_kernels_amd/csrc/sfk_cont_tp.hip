@@ -733,10 +733,8 @@ void tp_shape(int n, int shape, int *bx, int *by)
 #undef SFK_X
 }
 
-// a CU (lds_max bytes) holds two workgroups of the matvec: below that the
-// kernel's phases have nothing to overlap with (Q6 52x50x52 FP64 on 24 x 1
-// cells, one workgroup of 94 KB per CU: 196 us instead of 129 us)
-bool tp_shape_fits(int n, int shape, bool fp32, size_t lds_max)
+// LDS of a workgroup of the matvec
+static size_t tp_lds_bytes(int n, int shape, bool fp32)
 {
   size_t v = 0;
 #define SFK_X(NN, SH, BXX, BYY) \
@@ -744,7 +742,15 @@ bool tp_shape_fits(int n, int shape, bool fp32, size_t lds_max)
     v = fp32 ? TpCfg<NN, float, BXX, BYY>::lds_values(false) * 4 : TpCfg<NN, double, BXX, BYY>::lds_values(false) * 8;
   SFK_TP_SHAPES(SFK_X)
 #undef SFK_X
-  return 2 * v <= lds_max;
+  return v;
+}
+
+// a CU (lds_max bytes) holds two workgroups of the matvec: below that the
+// kernel's phases have nothing to overlap with (Q6 52x50x52 FP64 on 24 x 1
+// cells, one workgroup of 94 KB per CU: 196 us instead of 129 us)
+bool tp_shape_fits(int n, int shape, bool fp32, size_t lds_max)
+{
+  return 2 * tp_lds_bytes(n, shape, fp32) <= lds_max;
 }
 
 // Modelled cost of a schedule, in work items x layers per CU.  A workgroup
@@ -754,14 +760,14 @@ bool tp_shape_fits(int n, int shape, bool fp32, size_t lds_max)
 // its range of cells in z costs 1.2 layers more when it starts above the
 // bottom and 0.6 for its start; and a CU with few workgroups still needs the
 // latency of a layer, about what 500 items cost, per set of resident ones.
-double tp_cost(int n, const int nc[3], int shape, int zc)
+double tp_cost(int n, const int nc[3], int shape, int zc, const Chip &chip)
 {
   int bx = 0, by = 0;
   tp_shape(n, shape, &bx, &by);
   if (bx <= 0 || zc <= 0) return 1e300;
   const int p = n - 1, items = p * by * (bx * p + p + 1), waves = (items + 63) / 64;
   const long long tiles = (long long)((nc[0] + bx - 1) / bx) * ((nc[1] + by - 1) / by);
-  const long long chunks = (nc[2] + zc - 1) / zc, per_cu = (tiles * chunks + 255) / 256;
+  const long long chunks = (nc[2] + zc - 1) / zc, per_cu = (tiles * chunks + chip.cus - 1) / chip.cus;
   const long long slots = 16 / waves > 0 ? 16 / waves : 1;
   const long long resident = (per_cu < slots ? per_cu : slots) * waves;
   double work = double(per_cu) * (0.5 * items + 0.5 * 256 * ((waves + 3) / 4));
@@ -783,17 +789,20 @@ std::vector<int> tp_zc_candidates(int nz)
 // the schedule of shape 0 and / or zc 0 (automatic): the cheapest by tp_cost.
 // Untuned Q6 64^3 FP64 380 -> 266 us (the tuner finds 264), Q4 16^3: see the
 // launch-bound meshes' 500-item latency above.
-void tp_plan(int n, bool fp32, const int nc[3], int *shape, int *zc)
+void tp_plan(int n, bool fp32, const int nc[3], const Chip &chip, int *shape, int *zc)
 {
   if (*shape > 0 && *zc > 0) return;
   const std::vector<int> zcs = *zc > 0 ? std::vector<int>{*zc < nc[2] ? *zc : nc[2]} : tp_zc_candidates(nc[2]);
   const int s0 = *shape > 0 ? *shape : 1, s1 = *shape > 0 ? *shape : tp_shape_count(n) - 1;
   double best = -1.;
   int bs = s0, bz = zcs[0];
+  // (where no tile leaves room for two workgroups: the smallest one)
+  for (int sh = s0 + 1; sh <= s1; ++sh)
+    if (tp_lds_bytes(n, sh, fp32) < tp_lds_bytes(n, bs, fp32)) bs = sh;
   for (int sh = s0; sh <= s1; ++sh) {
-    if (*shape == 0 && !tp_shape_fits(n, sh, fp32, 163840)) continue;
+    if (*shape == 0 && !tp_shape_fits(n, sh, fp32, chip.lds)) continue;
     for (int z : zcs) {
-      const double c = tp_cost(n, nc, sh, z);
+      const double c = tp_cost(n, nc, sh, z, chip);
       if (best < 0. || c < best) {
         best = c;
         bs = sh;

@@ -105,10 +105,15 @@ hipError_t upload_tp_tables(const Tables1D &t, const double inv_jac[3], bool fp3
 int tp_shape_count(int n);
 void tp_shape(int n, int shape, int *bx, int *by);
 bool tp_shape_fits(int n, int shape, bool fp32, size_t lds_max);
-double tp_cost(int n, const int nc[3], int shape, int zc);
+// what the schedules count with (current_chip() in sfk_op.h asks the device)
+struct Chip {
+  size_t lds = 163840; // bytes of LDS per workgroup
+  int cus = 256;
+};
+double tp_cost(int n, const int nc[3], int shape, int zc, const Chip &chip);
 std::vector<int> tp_zc_candidates(int nz);
 // resolves an automatic tile shape (0) and / or cells in z (0) for a mesh
-void tp_plan(int n, bool fp32, const int nc[3], int *shape, int *zc);
+void tp_plan(int n, bool fp32, const int nc[3], const Chip &chip, int *shape, int *zc);
 hipError_t launch_cell_diagonal(const CellLaunch &L, hipStream_t stream);
 
 // DG-SIPG with per-quadrature-point metric (deformed mesh)

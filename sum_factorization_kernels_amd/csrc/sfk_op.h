@@ -107,6 +107,8 @@ inline void fill_precomp_launch(const sfk_op *op, PrecompLaunch &L)
 }
 
 size_t elem_size(const sfk_op *op);
+// the current device's limits (an MI355X's when no device can be queried)
+Chip current_chip();
 // device tables of the operator (uploaded on first use)
 sfk_status ensure_device_tables(sfk_op *op);
 // the Cartesian DG-SIPG operator runs on the precomputed operator's kernel

@@ -57,19 +57,6 @@ size_t lds_per_cell(const sfk_op *op)
   }
 }
 
-// LDS per workgroup of the current device (gfx950: 160 KiB when no device
-// can be queried)
-int lds_limit()
-{
-  int dev = 0, lds_max = 163840;
-  if (hipGetDevice(&dev) == hipSuccess) {
-    int v = 0;
-    if (hipDeviceGetAttribute(&v, hipDeviceAttributeMaxSharedMemoryPerBlock, dev) == hipSuccess && v > 0)
-      lds_max = v;
-  }
-  return lds_max;
-}
-
 bool sipg_per_q(const sfk_op *op)
 {
   return op->d.kind == SFK_DG_SIPG && op->d.geometry == SFK_GEOM_PER_Q;
@@ -85,19 +72,18 @@ bool tp_ok(const sfk_op *op)
 // sweep over tiles and z ranges was modelled within 1.45 of the cheapest for
 // every degree, in both precisions, matvec and Chebyshev step)
 constexpr double kTpTry = 1.6;
-double tp_best_cost(const sfk_op *op)
+double tp_best_cost(const sfk_op *op, const Chip &chip)
 {
   int shape = 0, zc = 0;
-  tp_plan(op->d.degree + 1, op->d.precision == SFK_FP32, op->d.n_cells, &shape, &zc);
-  return tp_cost(op->d.degree + 1, op->d.n_cells, shape, zc);
+  tp_plan(op->d.degree + 1, op->d.precision == SFK_FP32, op->d.n_cells, chip, &shape, &zc);
+  return tp_cost(op->d.degree + 1, op->d.n_cells, shape, zc, chip);
 }
 
 int max_cb(const sfk_op *op)
 {
   const int n = op->d.degree + 1;
-  const int lds_max = lds_limit();
   int m = kMaxThreads / (n * n);
-  const int by_lds = (int)(size_t(lds_max) / lds_per_cell(op));
+  const int by_lds = (int)(current_chip().lds / lds_per_cell(op));
   if (by_lds < m) m = by_lds;
   return m > 0 ? m : 1;
 }
@@ -223,7 +209,7 @@ sfk_status sfk_op_tile_shape(const sfk_op *op, int shape, int *count, int *bx, i
   if (count) *count = c;
   if (shape < 0 || shape >= c) TUNE_FAIL(SFK_ERR_INVALID_ARG, "tile shape must be in 0.." + std::to_string(c - 1));
   int x = 0, y = 0, zc = op->tp_zc;
-  if (shape == 0) tp_plan(n, op->d.precision == SFK_FP32, op->d.n_cells, &shape, &zc);
+  if (shape == 0) tp_plan(n, op->d.precision == SFK_FP32, op->d.n_cells, current_chip(), &shape, &zc);
   tp_shape(n, shape, &x, &y);
   if (bx) *bx = x;
   if (by) *by = y;
@@ -252,7 +238,7 @@ sfk_status sfk_op_set_schedule(sfk_op *op, const sfk_schedule *s)
     TUNE_FAIL(SFK_ERR_INVALID_ARG, "tile_shape out of range");
   if (s->z_cells < 0) TUNE_FAIL(SFK_ERR_INVALID_ARG, "z_cells must be >= 0");
   if (s->cont_scatter == 2 || s->cont_scatter == -1) {
-    if (tp_ok(op) && !tp_shape_fits(op->d.degree + 1, s->tile_shape, op->d.precision == SFK_FP32, lds_limit()))
+    if (tp_ok(op) && !tp_shape_fits(op->d.degree + 1, s->tile_shape, op->d.precision == SFK_FP32, current_chip().lds))
       TUNE_FAIL(SFK_ERR_UNSUPPORTED, "tile shape needs more LDS than leaves room for two workgroups per CU");
   }
   op->sched_cb = s->cells_per_block;
@@ -268,6 +254,7 @@ sfk_status sfk_tune(sfk_op *op, int repeats, sfk_schedule *best, double *best_se
 {
   if (!op) TUNE_FAIL(SFK_ERR_INVALID_ARG, "sfk_tune: null handle");
   if (repeats < 1 || repeats > 10000) TUNE_FAIL(SFK_ERR_INVALID_ARG, "sfk_tune: repeats must be in 1..10000");
+  const Chip chip = current_chip();
   const char *cache = std::getenv("SFK_TUNE_CACHE");
   const std::string key = cache && *cache ? cache_key(op) : std::string();
   if (!key.empty()) {
@@ -282,7 +269,7 @@ sfk_status sfk_tune(sfk_op *op, int repeats, sfk_schedule *best, double *best_se
             dg_cheby ? e.cheby[1] <= max_cb(op) && e.cheby[2] >= 0 && e.cheby[2] <= 2
                      : e.cheby[0] < 0 || (tp_ok(op) && e.cheby[0] < tp_shape_count(op->d.degree + 1) &&
                                           tp_shape_fits(op->d.degree + 1, e.cheby[0],
-                                                        op->d.precision == SFK_FP32, lds_limit()) &&
+                                                        op->d.precision == SFK_FP32, current_chip().lds) &&
                                           e.cheby[1] >= 0 && (e.cheby[2] == 0 || e.cheby[2] == 1));
         if (cheby_ok) {
           set_cheby_schedule(op, dg_cheby ? -1 : e.cheby[0], dg_cheby ? 0 : e.cheby[1], e.cheby[2]);
@@ -352,14 +339,14 @@ sfk_status sfk_tune(sfk_op *op, int repeats, sfk_schedule *best, double *best_se
     if (tp_ok(op)) {
       // tensor-product kernel: tile shapes x cells in z per workgroup
       const int n = op->d.degree + 1, nz = op->d.n_cells[2];
-      const double tp_best = tp_best_cost(op);
+      const double tp_best = tp_best_cost(op, chip);
       const int win_cb = saved_cb > 0 ? saved_cb : default_cb(op); // (unused by this kernel)
       for (int sh = 1; sh < tp_shape_count(n) && status == SFK_OK; ++sh) {
-        if (!tp_shape_fits(n, sh, op->d.precision == SFK_FP32, lds_limit())) continue;
+        if (!tp_shape_fits(n, sh, op->d.precision == SFK_FP32, chip.lds)) continue;
         for (int order = 0; order <= 1 && status == SFK_OK; ++order)
           for (int zc : tp_zc_candidates(nz)) {
             if (status != SFK_OK) break;
-            if (tp_cost(n, op->d.n_cells, sh, zc) > kTpTry * tp_best) continue;
+            if (tp_cost(n, op->d.n_cells, sh, zc, chip) > kTpTry * tp_best) continue;
             op->sched_order = order;
             op->cont_scatter = 2;
             set_tp_schedule(op, sh, zc);
@@ -382,13 +369,13 @@ sfk_status sfk_tune(sfk_op *op, int repeats, sfk_schedule *best, double *best_se
     if (status == SFK_OK) status = sfk_vec_fill(op->d.precision, pv, op->nvec * op->d.n_rhs, 0.0, stream);
     if (status == SFK_OK) status = ensure_device_tables(op);
     const int n = op->d.degree + 1, nz = op->d.n_cells[2];
-    const double tp_best = tp_best_cost(op);
+    const double tp_best = tp_best_cost(op, chip);
     for (int sh = 1; sh < tp_shape_count(n) && status == SFK_OK; ++sh) {
-      if (!tp_shape_fits(n, sh, op->d.precision == SFK_FP32, lds_limit())) continue;
+      if (!tp_shape_fits(n, sh, op->d.precision == SFK_FP32, chip.lds)) continue;
       for (int order = 0; order <= 1 && status == SFK_OK; ++order)
         for (int zc : tp_zc_candidates(nz)) {
           if (status != SFK_OK) break;
-          if (tp_cost(n, op->d.n_cells, sh, zc) > kTpTry * tp_best) continue;
+          if (tp_cost(n, op->d.n_cells, sh, zc, chip) > kTpTry * tp_best) continue;
           set_cheby_schedule(op, sh, zc, order);
           TpLaunch T;
           fill_tp_launch(op, T, true);

@@ -29,7 +29,7 @@ static int check(sfk_op *op, bool cheby, int shape, int zc)
   for (int i = 0; i < 100; ++i) fill_tp_launch(op, L, cheby);
   const long allocated = g_allocations - before;
   const int n = op->d.degree + 1;
-  tp_plan(n, op->d.precision == SFK_FP32, op->d.n_cells, &shape, &zc);
+  tp_plan(n, op->d.precision == SFK_FP32, op->d.n_cells, current_chip(), &shape, &zc);
   if (allocated == 0 && L.shape == shape && L.zc == zc) return 0;
   std::printf("degree %d, %d cells in z, %s: tile %d, %d cells (planned %d, %d), %ld allocations in 100 launches\n",
               n - 1, op->d.n_cells[2], cheby ? "Chebyshev" : "matvec", L.shape, L.zc, shape, zc, allocated);

@@ -27,3 +27,7 @@ def run_check(name, tmp_path):
 
 def test_automatic_schedules(tmp_path):
     run_check("tp_schedule_check", tmp_path)
+
+
+def test_planned_tile_is_accepted(tmp_path):
+    run_check("tp_plan_check", tmp_path)
