@@ -672,7 +672,6 @@ template <int N, typename T>
 struct DiagArgs {
   Eo<N, T> S2b, G2b; // backward contractions with S^2 and G1^2
   Eo<N, T> S1b;      // load vector: backward contraction with S
-  int load;          // 1: b_i = sum_q f JxW_q phi_i(x_q) instead of the diagonal
   T fval, jxw;
   T w[N];
   const T *coef;
@@ -683,7 +682,10 @@ struct DiagArgs {
   int cont;
 };
 
-template <int N, typename T>
+// LOAD: b_i = sum_q f JxW_q phi_i(x_q) instead of the diagonal; COEF: with a
+// coefficient.  Kernels of their own: as run-time choices, their loads and
+// registers cost the plain diagonal 25 % (Q6 FP64 1.2e7 nodes: 328 us)
+template <int N, typename T, bool LOAD, bool COEF>
 __global__ void __launch_bounds__(threads_per_block<N>()) diag_kernel(const DiagArgs<N, T> a)
 {
   constexpr int CB = full_cells(N);
@@ -695,17 +697,17 @@ __global__ void __launch_bounds__(threads_per_block<N>()) diag_kernel(const Diag
   const bool act = c < CB && cell < a.ncells;
   T *A = sA + (act ? c : 0) * N3;
   T *R = sR + (act ? c : 0) * N3;
-  for (int d = 0; d < (a.load ? 1 : 3); ++d) {
+  for (int d = 0; d < (LOAD ? 1 : 3); ++d) {
     if (act) {
-      // weights c_d w_q k_q on x-line l
+      // weights c_d w_q k_q on x-line l (the coefficient holds the quadrature weight)
       T u[N], v[N];
+      const T f = LOAD ? a.fval * a.jxw : a.cdiag[d];
 #pragma unroll
       for (int i = 0; i < N; ++i) {
-        // (the coefficient holds the quadrature weight)
-        const T w = a.coef && !a.load ? a.coef[cell * N3 + l * N + i] : line_weight<N, 0>(a.w, l, i);
-        u[i] = (a.load ? a.fval * a.jxw : a.cdiag[d]) * w;
+        if constexpr (COEF) u[i] = f * a.coef[cell * N3 + l * N + i];
+        else u[i] = f * line_weight<N, 0>(a.w, l, i);
       }
-      if (a.load) eo_apply<N, 1>(a.S1b, u, v);
+      if constexpr (LOAD) eo_apply<N, 1>(a.S1b, u, v);
       else if (d == 0) eo_apply<N, 1>(a.G2b, u, v);
       else eo_apply<N, 1>(a.S2b, u, v);
       lds_write_line<N, N, 0>(A, l, v);
@@ -714,7 +716,7 @@ __global__ void __launch_bounds__(threads_per_block<N>()) diag_kernel(const Diag
     if (act) {
       T u[N], v[N];
       lds_read_line<N, N, 1>(A, l, u);
-      if (a.load) eo_apply<N, 1>(a.S1b, u, v);
+      if constexpr (LOAD) eo_apply<N, 1>(a.S1b, u, v);
       else if (d == 1) eo_apply<N, 1>(a.G2b, u, v);
       else eo_apply<N, 1>(a.S2b, u, v);
       lds_write_line<N, N, 1>(A, l, v);
@@ -723,7 +725,7 @@ __global__ void __launch_bounds__(threads_per_block<N>()) diag_kernel(const Diag
     if (act) {
       T u[N], v[N], r[N];
       lds_read_line<N, N, 2>(A, l, u);
-      if (a.load) eo_apply<N, 1>(a.S1b, u, v);
+      if constexpr (LOAD) eo_apply<N, 1>(a.S1b, u, v);
       else if (d == 2) eo_apply<N, 1>(a.G2b, u, v);
       else eo_apply<N, 1>(a.S2b, u, v);
       if (d > 0) lds_read_line<N, N, 2>(R, l, r);
@@ -1024,7 +1026,6 @@ static hipError_t launch_diag_n(const CellLaunch &L, hipStream_t stream)
   a.S2b = make_eo<N, T>(S2, false);
   a.G2b = make_eo<N, T>(G2, false);
   a.S1b = make_eo<N, T>(t.S, false);
-  a.load = L.load ? 1 : 0;
   a.fval = T(L.load_value);
   for (int i = 0; i < N; ++i) a.w[i] = T(t.weights[i]);
   a.coef = (const T *)L.coef;
@@ -1042,7 +1043,9 @@ static hipError_t launch_diag_n(const CellLaunch &L, hipStream_t stream)
   a.cont = L.mode == 1;
   constexpr int CB = full_cells(N);
   const unsigned blocks = (unsigned)((L.ncells + CB - 1) / CB);
-  hipLaunchKernelGGL((diag_kernel<N, T>), dim3(blocks), dim3(threads_per_block<N>()), 0, stream, a);
+  auto kern = L.load ? diag_kernel<N, T, true, false>
+                     : (L.coef ? diag_kernel<N, T, false, true> : diag_kernel<N, T, false, false>);
+  hipLaunchKernelGGL(kern, dim3(blocks), dim3(threads_per_block<N>()), 0, stream, a);
   return hipGetLastError();
 }
 
