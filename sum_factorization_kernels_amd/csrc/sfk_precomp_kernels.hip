@@ -37,6 +37,8 @@
 // -> 15.8 us; Chebyshev step p = 5 FP64 80 -> 70 us, p = 8 20x21x22 78 -> 62 us.
 // Tried and not kept: workgroups that loop over several blocks and load the
 // next one early (no faster at 4 to 64 workgroups per CU).
+#include <type_traits>
+
 #include "sfk_device.h"
 #include "sfk_kernels.h"
 
@@ -156,31 +158,42 @@ __device__ __forceinline__ void pc_load_layers(const T *src, const int (&nbr)[6]
   }
 }
 
-// Matvec results that leave as the block's consecutive values instead of z lines:
-// where a z line's lanes cover parts of cache lines (72 B for n = 3, 200 B for n =
-// 5 in FP64), non-temporal stores of them cost HBM a read where the vectors exceed
-// the Infinity Cache.  z lines -> consecutive: n = 3 FP64 3e6 unknowns 16.6 -> 13.8
-// us, 1.9e7 123 -> 101, FP32 1.9e7 50.5 -> 47.9; n = 5 FP64 1.9e7 107 -> 93, but
-// 3e6 13.8 -> 14.7; n = 5 FP32, n = 7 and 9: 3 to 7 % slower.  (Plain stores of
-// either form: 5 to 30 % slower at most sizes.)
+// How the vectors are read and written: kLines as z lines; kFlatStore: the matvec's
+// results leave through LDS as the block's consecutive values; kFlat: that at both
+// ends.  Where a z line's lanes cover parts of cache lines (n^2 values: 32 to 200
+// B), the pieces cost HBM more than LDS saves once the vectors exceed the Infinity
+// Cache, the non-temporal stores of the matvec most.  Matvec, lines / flat stores /
+// flat: n = 2 FP64 3e6 unknowns 15.1 / 14.5 / 15.5 us, 3e7 175 / 162 / 164; n = 3
+// FP64 6e6 32 / 26 / 27.5, 2e7 132 / 107 / 105, FP32 1e7 28.5 / 27.1 / 27.9, 3e7
+// 103 / 94 / 90; n = 5 FP64 2e7 107 / 101 / 98, FP32 2e7 45.7 / 47.5 / 50, 3e7 97 /
+// 86 / 84; n = 6 FP32 2e7 43.8 / 45.9 / 47.9, 3e7 83.5 / 78.3 / 78.4; n = 7 and
+// above, and n = 6 FP64: lines 3 to 13 % faster.  Chebyshev step (six streams),
+// lines / flat: n = 5 FP32 6e6 24.8 / 28.2, 1.5e7 94 / 83, 3e7 182 / 167; n = 3 FP32
+// 36 / 30; n = 5 FP64 and n >= 6: lines 1 to 30 % faster.  (Plain instead of
+// non-temporal stores: 5 to 30 % slower at most sizes.)  "Large" is the size of one
+// vector, pc_large_bytes: two of the matvec's, six of the step's fill most of the
+// 256 MB Infinity Cache.
+enum PcForm { kLines = 0, kFlatStore = 1, kFlat = 2 };
 template <int N, typename T>
-constexpr bool pc_flat_store()
+constexpr PcForm pc_form(bool cheby, bool large)
 {
-  return N == 3 || (N == 5 && sizeof(T) == 8);
+  const bool fp32 = sizeof(T) == 4;
+  if (cheby) return N <= 3 || (N == 5 && fp32 && large) ? kFlat : kLines;
+  if (N == 2) return fp32 ? kLines : kFlatStore;
+  if (N == 3) return large ? kFlat : kFlatStore;
+  if (N == 5 && !fp32) return kFlatStore;
+  return (N == 5 || N == 6) && fp32 && large ? kFlat : kLines;
 }
+constexpr long long pc_large_bytes(bool cheby) { return cheby ? 36LL << 20 : 104LL << 20; }
 
-template <int N, typename T, bool COUPLE, bool CHEBY>
+template <int N, typename T, bool COUPLE, bool CHEBY, PcForm FORM>
 __global__ void __launch_bounds__(kPcMaxThreads) __attribute__((amdgpu_waves_per_eu(1, pc_waves<N, T>())))
 precomp_kernel(PcArgs<N, T> a)
 {
   constexpr int N2 = N * N, N3 = N2 * N;
   const int cb = a.cb;
   constexpr int CS = PcLds<N>::CS;
-  // n <= 3: a z line's lanes cover less than a cache line, and six streams of
-  // such pieces cost more than coalesced copies through LDS on both ends (p = 2
-  // FP32 Chebyshev step 30 us flat, 36 us on z lines)
-  constexpr bool FLAT = CHEBY && N <= 3;
-  constexpr bool FLAT_ST = FLAT || (!CHEBY && pc_flat_store<N, T>());
+  constexpr bool FLAT = FORM == kFlat, FLAT_ST = FORM != kLines;
   const long long c0 = (long long)logical_block(blockIdx.x, gridDim.x, a.order) * cb;
   const long long voff = (long long)blockIdx.y * a.nvec;
   const T *src = a.src + voff;
@@ -198,7 +211,15 @@ precomp_kernel(PcArgs<N, T> a)
   const int nval = (rem < cb ? (int)rem : cb) * N3;
 
   T u[N], nb[3][4], keep[FLAT ? N : 1];
+  auto load_layers = [&]() {
+    if constexpr (COUPLE) {
+      pc_load_layers<N, 2>(src, nbr, l, nb[2]);
+      pc_load_layers<N, 1>(src, nbr, l, nb[1]);
+      pc_load_layers<N, 0>(src, nbr, l, nb[0]);
+    }
+  };
   if constexpr (FLAT) {
+    if (act) load_layers(); // in flight together with the block's own values
     // blockDim.x >= cb n^2: n rounds cover the block
 #pragma unroll
     for (int k = 0; k < N; ++k) {
@@ -217,12 +238,10 @@ precomp_kernel(PcArgs<N, T> a)
     else
 #pragma unroll
       for (int k = 0; k < N; ++k) u[k] = src[g0 + k * N2];
-    if constexpr (COUPLE) {
-      pc_load_layers<N, 2>(src, nbr, l, nb[2]);
-      pc_load_layers<N, 1>(src, nbr, l, nb[1]);
-      pc_load_layers<N, 0>(src, nbr, l, nb[0]);
+    if constexpr (!FLAT) {
+      load_layers();
+      pc_write<N, 2>(U, l, u);
     }
-    if constexpr (!FLAT) pc_write<N, 2>(U, l, u);
     const auto &pt = pctab(a.pt);
     T o[N];
     eo_apply<N, 1>(pt.L[2], u, o);
@@ -255,17 +274,20 @@ precomp_kernel(PcArgs<N, T> a)
     pc_write<N, 0>(U, l, r);
   }
   __syncthreads();
-  // fused update: its streams are loaded one phase ahead (n <= 3: see below)
+  // fused update: its streams are loaded one phase ahead
   T s_rhs[CHEBY ? N : 1], s_diag[CHEBY ? N : 1], s_tm[CHEBY ? N : 1];
-  if (act) {
-    if constexpr (CHEBY && !FLAT) {
+  if constexpr (CHEBY) {
+    if (FLAT || act)
 #pragma unroll
       for (int k = 0; k < N; ++k) {
-        s_rhs[k] = a.rhs[g0 + k * N2];
-        s_diag[k] = a.diag[g0 + k * N2];
-        s_tm[k] = a.c_tm != T(0) ? a.tm[g0 + k * N2] : T(0); // c_tm == 0: tm not read
+        const int i = t + k * (int)blockDim.x;
+        const long long g = FLAT ? c0 * N3 + (i < nval ? i : nval - 1) : g0 + k * N2;
+        s_rhs[k] = a.rhs[g];
+        s_diag[k] = a.diag[g];
+        s_tm[k] = a.c_tm != T(0) ? a.tm[g] : T(0); // c_tm == 0: tm not read
       }
-    }
+  }
+  if (act) {
     const auto &pt = pctab(a.pt);
     T v[N], o[N];
     pc_read<N, 1>(P, l, v);
@@ -316,9 +338,9 @@ precomp_kernel(PcArgs<N, T> a)
       if constexpr (!CHEBY) {
         __builtin_nontemporal_store(dyn_lds<T>()[i], a.dst + voff + g);
       } else {
-        const T res = dyn_lds<T>()[i] - a.rhs[g];
-        T tmv = a.c_np * a.diag[g] * res;
-        if (a.c_tm != T(0)) tmv = a.c_tm * a.tm[g] + tmv;
+        const T res = dyn_lds<T>()[i] - s_rhs[k];
+        T tmv = a.c_np * s_diag[k] * res;
+        if (a.c_tm != T(0)) tmv = a.c_tm * s_tm[k] + tmv;
         a.tm[g] = tmv;
         a.dst[g] = keep[k] - tmv;
       }
@@ -365,9 +387,17 @@ hipError_t launch_precomp_n(const PrecompLaunch &L, hipStream_t s)
   a.order = L.order;
   const size_t lds = size_t(3) * CB * PcLds<N>::CS * sizeof(T);
   const dim3 grid((unsigned)((L.ncells + CB - 1) / CB), (unsigned)L.nrhs), block(((CB * N * N + 63) / 64) * 64);
-  decltype(&precomp_kernel<N, T, true, false>) kern;
-  if (L.couple) kern = L.cheby ? precomp_kernel<N, T, true, true> : precomp_kernel<N, T, true, false>;
-  else kern = L.cheby ? precomp_kernel<N, T, false, true> : precomp_kernel<N, T, false, false>;
+  decltype(&precomp_kernel<N, T, true, false, kLines>) kern;
+  const bool large = a.nvec * (long long)sizeof(T) >= pc_large_bytes(L.cheby);
+  auto pick = [&](auto cheby, auto big) {
+    constexpr bool C = decltype(cheby)::value;
+    constexpr PcForm F = pc_form<N, T>(C, decltype(big)::value);
+    kern = L.couple ? precomp_kernel<N, T, true, C, F> : precomp_kernel<N, T, false, C, F>;
+  };
+  using no = std::false_type;
+  using yes = std::true_type;
+  if (L.cheby) large ? pick(yes(), yes()) : pick(yes(), no());
+  else large ? pick(no(), yes()) : pick(no(), no());
   const hipError_t e = allow_dynamic_lds((const void *)kern, lds);
   if (e != hipSuccess) return e;
   hipLaunchKernelGGL(kern, grid, block, lds, s, a);
