@@ -518,7 +518,9 @@ cell_kernel(const CellArgs<N, T> a)
 // 40x37x42, 3, FP64 181 -> 163 us; p = 5 24x26x28, 5, FP32 132 -> 114 us; p = 8
 // 24^3, 1, FP64 143 -> 134 us, but 8, FP32 467 -> 465 us: there the workgroups a
 // CU holds, and the tails of the 8 launches (15 %), set the time.
-template <int N, typename T, int NR>
+// PART: the last workgroup's right-hand sides may be fewer than NR; the others' work
+// is left out (tested at run time, which cost full pairs up to 4 %)
+template <int N, typename T, int NR, bool PART>
 __global__ void __launch_bounds__(kCellMaxThreads)
 __attribute__((amdgpu_waves_per_eu(1, lds_waves_per_simd(NR * full_cells(N) * 2 * N * N * N * (int)sizeof(T), full_cells(N) * N * N))))
 cont_coef_kernel(const CellArgs<N, T> a)
@@ -549,6 +551,7 @@ cont_coef_kernel(const CellArgs<N, T> a)
       }
 #pragma unroll
     for (int r = 0; r < NR; ++r) {
+      if (PART && r >= nr) break;
       eo_apply<N, 1>(ctab(a.dt).Sf, u[r], v);
       lds_write_line<N, N, 2>(A + r * rs, l, v);
     }
@@ -557,6 +560,7 @@ cont_coef_kernel(const CellArgs<N, T> a)
   if (act) {
 #pragma unroll
     for (int r = 0; r < NR; ++r) {
+      if (PART && r >= nr) break;
       T u[N], v[N];
       lds_read_line<N, N, 0>(A + r * rs, l, u);
       eo_apply<N, 1>(ctab(a.dt).Sf, u, v);
@@ -587,6 +591,7 @@ cont_coef_kernel(const CellArgs<N, T> a)
   if (act) {
 #pragma unroll
     for (int r = 0; r < NR; ++r) {
+      if (PART && r >= nr) break;
       T u[N], v[N], w[N];
       lds_read_line<N, N, 1>(A + r * rs, l, u);
       eo_apply<N, 1>(ctab(a.dt).Sf, u, v);
@@ -600,6 +605,7 @@ cont_coef_kernel(const CellArgs<N, T> a)
   if (act) {
 #pragma unroll
     for (int r = 0; r < NR; ++r) {
+      if (PART && r >= nr) break;
       T v[N], w[N], b[N];
       lds_read_line<N, N, 0>(A + r * rs, l, v);
       grad(0, k, v, w);
@@ -614,6 +620,7 @@ cont_coef_kernel(const CellArgs<N, T> a)
   if (act) {
 #pragma unroll
     for (int r = 0; r < NR; ++r) {
+      if (PART && r >= nr) break;
       T v[N], w[N], b[N];
       lds_read_line<N, N, 2>(A + r * rs, l, v);
       grad(2, k, v, w);
@@ -628,6 +635,7 @@ cont_coef_kernel(const CellArgs<N, T> a)
   if (act) {
 #pragma unroll
     for (int r = 0; r < NR; ++r) {
+      if (PART && r >= nr) break;
       T u[N], v[N];
       lds_read_line<N, N, 1>(A + r * rs, l, u);
       eo_apply<N, 1>(ctab(a.dt).Sb, u, v);
@@ -636,9 +644,13 @@ cont_coef_kernel(const CellArgs<N, T> a)
   }
   __syncthreads();
   T o[NR][N];
+  if constexpr (PART)
+#pragma unroll
+    for (int i = 0; i < N; ++i) o[NR - 1][i] = T(0);
   if (act) {
 #pragma unroll
     for (int r = 0; r < NR; ++r) {
+      if (PART && r >= nr) break;
       T u[N];
       lds_read_line<N, N, 0>(A + r * rs, l, u);
       eo_apply<N, 1>(ctab(a.dt).Sb, u, o[r]);
@@ -972,20 +984,28 @@ static hipError_t launch_cell_n(const CellLaunch &L, hipStream_t stream)
     // index arithmetic and coefficient outweigh the halved number of resident
     // workgroups (8 right-hand sides, p = 2 80x70x75 FP32: 370 -> 297 us, p = 4
     // 40x37x42 156 -> 150 us, p = 8 24^3 462 -> 493 us; FP64 p = 1 227 -> 184 us,
-    // p = 3 50x52x55 263 -> 290 us)
+    // p = 3 50x52x55 263 -> 290 us), and only where each colour's launch still
+    // fills the chip (2 right-hand sides FP32 p = 4 35x30x30, 450 pairs a colour:
+    // 72 us one by one, 82 us in pairs; 55x47x48, 1728: 174 and 153 us; p = 3
+    // 46x40x40 with 4, 1200: 99.5 and 103 us; p = 1 73x64x64 with 2, 1024: 53 and 49
+    // us).  The atomic scatter gains nothing from pairs (p = 3 24x21x22 with 8: 117
+    // and 120 us).
     constexpr int NR2 = N <= (std::is_same<T, float>::value ? 5 : 2) ? 2 : 1;
-    const bool two = L.coef && L.nrhs > 1 && NR2 == 2;
-    auto kern = L.coef ? (two ? cont_coef_kernel<N, T, NR2> : cont_coef_kernel<N, T, 1>)
-                       : cell_kernel<N, T, Mode::Cont, false, false, false>;
+    a.nseg = (a.nx + CB - 1) / CB;
+    const bool colored = cont_colored(L, CB);
+    const long long pairs = (long long)((a.nseg + 1) / 2) * ((a.ny + 1) / 2) * ((a.nz + 1) / 2) * ((L.nrhs + 1) / 2);
+    const bool two = L.coef && L.nrhs > 1 && NR2 == 2 && colored && pairs >= (N == 2 ? 1000 : 1300);
+    auto kern = cell_kernel<N, T, Mode::Cont, false, false, false>;
+    if (two) kern = L.nrhs % 2 ? cont_coef_kernel<N, T, NR2, NR2 == 2> : cont_coef_kernel<N, T, NR2, false>;
+    else if (L.coef) kern = cont_coef_kernel<N, T, 1, false>;
     const size_t klds = two ? 2 * lds : lds;
     const unsigned ny = two ? (L.nrhs + 1) / 2 : L.nrhs;
-    if (!cont_colored(L, CB)) {
+    if (!colored) {
       a.color = -1;
       const hipError_t e = vec_fill(std::is_same<T, float>::value, L.dst, L.vstride * L.nrhs, 0., stream);
       if (e != hipSuccess) return e;
       return launch(kern, dim3(blocks, ny), klds);
     }
-    a.nseg = (a.nx + CB - 1) / CB;
     // colours in ascending order: the first unit to touch a node stores it
     for (int color = 0; color < 8; ++color) {
       const int ps = color >> 2 & 1, py = color & 1, pz = color >> 1 & 1;
