@@ -477,24 +477,27 @@ hipError_t layout_convert(int degree, const int nc[3], int lanes, const double *
 // position in the cell of a workgroup's first value is uniform and the threads'
 // follow by 32-bit arithmetic.  Takes the place of a device copy when a
 // coefficient is set and saves every later apply one multiplication per q-point
-// (Q8 24^3: FP32 15.8 us, the copy 12.2 us; FP64 24.6 us, the copy 23.1 us).
+// (Q8, 8e6 nodes: FP32 15.1 us, the copy 13.4; FP64 28.5 us, the copy 31.9; with
+// the weights loaded before the values 16.8 and 30.5.  Set and one apply together
+// take no longer than a copy and the apply that multiplied).
 constexpr int kWeightRounds = 8;
 template <int N, typename T>
 __global__ void __launch_bounds__(kThreads) weight_kernel(const DevTab<N, T> *dt, const T *x, T *y, long long n)
 {
   constexpr unsigned N3 = N * N * N;
-  const auto &w = ctab(dt).w;
-  __shared__ T sw[N];
-  if (threadIdx.x < N) sw[threadIdx.x] = w[threadIdx.x];
-  __syncthreads();
   const long long i0 = blockIdx.x * (long long)(kThreads * kWeightRounds);
   const unsigned q0 = (unsigned)(i0 % N3);
   T v[kWeightRounds];
 #pragma unroll
   for (int r = 0; r < kWeightRounds; ++r) {
     const long long i = i0 + r * kThreads + threadIdx.x;
-    if (i < n) v[r] = x[i];
+    v[r] = x[i < n ? i : n - 1];
   }
+  // the weights while the values are on their way
+  const auto &w = ctab(dt).w;
+  __shared__ T sw[N];
+  if (threadIdx.x < N) sw[threadIdx.x] = w[threadIdx.x];
+  __syncthreads();
 #pragma unroll
   for (int r = 0; r < kWeightRounds; ++r) {
     const long long i = i0 + r * kThreads + threadIdx.x;
