@@ -272,7 +272,10 @@ typedef struct sfk_solve_stats {
   double initial_residual, final_residual; /* ||b - A x||_2 (FP64) */
   double lambda_max, lambda_min;           /* Chebyshev bounds used */
   double seconds;                          /* wall time of the solve */
-  int matvecs_outer, matvecs_inner;
+  int matvecs_outer, matvecs_inner; /* inner: the smoother's, of the
+                                       preconditioners that were used (the last
+                                       one is launched before the iteration
+                                       is known to have converged) */
 } sfk_solve_stats;
 
 sfk_status sfk_solve_cg_cheby(sfk_op *op, sfk_op *smoother_op, const double *b, double *x,
