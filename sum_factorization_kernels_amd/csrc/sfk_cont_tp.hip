@@ -231,6 +231,10 @@ cont_tp_kernel(const TpArgs<T> a)
   // s_rhs D^{-1} rhs (the first iterate, never stored)
   constexpr bool TT = CHEBY >= 2 && CHEBY <= 4, RSRC = CHEBY == 3, RPREV = CHEBY == 4, DOT = CHEBY == 5;
   constexpr bool FUSED = CHEBY != 0; // phase Z needs the input at its nodes
+  // the Dirichlet nodes beyond a tile's end: the update's loads of a layer's
+  // planes in flight together, from where there are planes enough (Q1 FP32 with it
+  // 8 % slower; the matvec has nothing to load, and the code cost it up to 8 %)
+  constexpr bool TOGETHER = CHEBY == 1 ? N > 2 : TT && N > 3;
   constexpr bool PF = tp_prefetch<N, T, CHEBY>(), EARLY = tp_streams_early<N, T, CHEBY>();
   T *sA = dyn_lds<T>(); // a, then c; b, then d follow at C::LA
   T *sU = sA + 2 * C::LA;
@@ -532,19 +536,25 @@ cont_tp_kernel(const TpArgs<T> a)
         if constexpr (DOT) dot_acc += double(us[k]) * double(v);
       }
     }
-    // the grid's last column, row and corner: the layer's planes together, so
-    // that the update's loads are in flight together.  One plane after another,
+    // the grid's last column, row and corner.  With an update, the layer's planes
+    // together, so that its loads are in flight together.  One plane after another,
     // each waited for its own, every layer of a tile at the grid's end took p
     // more round trips to memory: six-stream Chebyshev step Q6 15x13x12 FP32 15.6
     // -> 10.9 us, Q3 84x72x73 FP32 156 -> 96, Q7 36x31x31 FP64 333 -> 247
-    if (xtra)
+    if (xtra) {
+      if constexpr (TOGETHER) {
 #pragma unroll 1
-      for (int e = 0; e < 3; ++e) {
-        const unsigned off = e == 0   ? (xtra_x ? coff + ES : kOob)
-                             : e == 1 ? (xtra_y ? coff + row_bytes : kOob)
-                                      : (xtra_x && xtra_y ? coff + row_bytes + ES : kOob);
-        put_zeros(ez, off);
+        for (int e = 0; e < 3; ++e) {
+          const unsigned off = e == 0   ? (xtra_x ? coff + ES : kOob)
+                               : e == 1 ? (xtra_y ? coff + row_bytes : kOob)
+                                        : (xtra_x && xtra_y ? coff + row_bytes + ES : kOob);
+          put_zeros(ez, off);
+        }
+      } else {
+#pragma unroll 1
+        for (int k = 0; k < p; ++k) put_xtra(ez * p + k);
       }
+    }
   };
 
   // one layer; next: the layer to prefetch (ez itself: none)
