@@ -241,7 +241,8 @@ sfk_status sfk_op_tile_shape(const sfk_op *op, int shape, int *count, int *bx, i
  * that its cost model puts within 1.6 of the cheapest; for that kernel the
  * fused Chebyshev launch (three-term form, four
  * vector streams) is timed over the same tile shapes, z_cells and orders and
- * its fastest kept separately (sfk_op_get_smoother_schedule), and for the
+ * its fastest kept separately (sfk_op_get_smoother_schedule; where several are
+ * within 3 %, by all launches of a solver iteration), and for the
  * per-q-metric SIPG kernel the fused Chebyshev step over cells_per_block and
  * the three orders, kept the same way.  Requires the
  * operator's data (metric, coefficient, velocity) to be set.

@@ -759,9 +759,13 @@ static hipError_t launch_tp_shape(const TpLaunch &L, hipStream_t s)
 
 // Tile shapes (BX, BY) per points per direction N, from 1 (shape 0: tp_plan
 // chooses).  Wide in x (the x halo of p+1 columns costs (p+1)/(BX p)), with
-// BY p BX as large as fits and a phase Y that fills a multiple of four waves:
-// 4 or 8 of them spread evenly over the SIMDs (Q6 52x50x52 FP64: 13 x 1 cells
-// in 8 full waves 129 us, 7 x 1 in 5 waves 177 us, 16 x 1 in 10 waves 195 us).
+// BY p BX as large as fits, and first the tiles whose phase Y fills 4 or 8 waves,
+// which spread evenly over the SIMDs (Q6 52x50x52 FP64: 13 x 1 cells in 8 waves 129
+// us, 7 x 1 in 5 waves 177 us, 16 x 1 in 10 waves 195 us).  From N = 6 on few
+// widths do: the tiles of 5, 6 and 7 waves are there for meshes whose cells in x
+// they divide better (Q6 42x36x37 FP32 six-stream step: 11 x 1 in 7 waves 86 us, 5 x
+// 1 in 4 waves 88 us, 13 x 1 in 8 waves more), and Q6's 24 x 1 in 15 waves, which leaves room for two
+// workgroups a CU in FP32 only, for rows that it covers with one tile less.
 #define SFK_TP_SHAPES(X)                                                        \
   X(2, 1, 30, 8) X(2, 2, 126, 4) X(2, 3, 62, 4) X(2, 4, 30, 16)                  \
   X(3, 1, 30, 2) X(3, 2, 62, 2) X(3, 3, 30, 4) X(3, 4, 14, 4)                    \
@@ -847,8 +851,9 @@ std::vector<int> tp_zc_candidates(int nz)
 }
 
 // the schedule of shape 0 and / or zc 0 (automatic): the cheapest by tp_cost.
-// Untuned Q6 64^3 FP64 380 -> 266 us (the tuner finds 264), Q4 16^3: see the
-// launch-bound meshes' 500-item latency above.
+// Untuned Q6 64^3 FP64 380 -> 266 us (the tuner finds 264).  Its weak side are
+// meshes with fewer workgroups than CUs: Q4 16^3 it takes 14 x 1 tiles and 2 cells
+// in z (8.1 us), the tuner 6 x 2 and 1 (7.7 us).
 void tp_plan(int n, bool fp32, const int nc[3], const Chip &chip, int *shape, int *zc)
 {
   if (*shape > 0 && *zc > 0) return;
