@@ -62,8 +62,8 @@
 //   phase Z instead of reading them again: with 10 MB of streams per layer in
 //   flight on an XCD the second read missed its 4 MB L2 (29 % more HBM reads).
 // Measured before -> after: matvec FP64 282 -> 264 us (3.5 TB/s; 3.9 TB/s with
-// the halo), FP32 172 -> 127 us; three-term Chebyshev step FP64 675 -> 457 us
-// (4.0 TB/s), FP32 358 -> 247 us; Q3 101x107x100 FP32 96 -> 58 us.
+// the halo), FP32 172 -> 127 us; three-term Chebyshev step FP64 675 -> 443 us
+// (4.1 TB/s), FP32 358 -> 244 us; Q3 101x107x100 FP32 96 -> 58 us.
 #include <cmath>
 #include <type_traits>
 

@@ -31,8 +31,8 @@
 // z lines, whose lanes touch consecutive dofs, both the block load and the
 // store go straight between registers and memory: 17 LDS accesses per point
 // and 4 barriers, where a coalesced copy through LDS on both ends took 20 and
-// 5.  Measured, before -> after,
-// matvec: p = 3 56x50x55 FP64 44 -> 38 us (4.1 TB/s), FP32 24 -> 19.6 us; p = 5
+// 5.  Measured, before -> after, on vectors in turn,
+// matvec: p = 3 56x50x55 FP64 41.0 -> 36.3 us (4.3 TB/s), FP32 24 -> 19.6 us; p = 5
 // 31x37x29 FP64 33.3 -> 29.3 us, FP32 18.4 -> 16 us; p = 7 22x25x24 FP32 21.4
 // -> 15.8 us; Chebyshev step p = 5 FP64 80 -> 70 us, p = 8 20x21x22 78 -> 62 us.
 // Tried and not kept: workgroups that loop over several blocks and load the
