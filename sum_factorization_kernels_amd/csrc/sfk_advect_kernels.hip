@@ -30,9 +30,9 @@
 // end so that the first and the last run on the z lines that are loaded and
 // stored (consecutive dofs across lanes), and the y derivative starts from the
 // registers of the y value sweep: 7 phases instead of 10.  Measured, before ->
-// after: apply FP64 p = 3 48^3 62.7 -> 55.7 us (5.7 TB/s, as a large copy), p = 7
-// 24x25x26 74 -> 62, FP32 p = 3 47x51x45 29.3 -> 27.5; transpose FP64 p = 3 90 ->
-// 83; LSRK stage FP64 p = 3 95 -> 79, p = 8 22x21x20 104 -> 81; velocity gradient
+// after: apply FP64 p = 3 48^3 62.7 -> 55.7 us (5.8 TB/s, as a large elementwise
+// kernel), p = 7 24x25x26 74 -> 62, FP32 p = 3 47x51x45 29.3 -> 27.5; transpose
+// FP64 p = 3 90 -> 83; LSRK stage FP64 p = 3 95 -> 79, p = 8 22x21x20 104 -> 81; velocity gradient
 // FP64 p = 3 108 -> 74, FP32 51 -> 39.
 #include "sfk_device.h"
 #include "sfk_kernels.h"
